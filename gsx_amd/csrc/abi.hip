@@ -892,12 +892,11 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     GSX_HIP_TRY(hipGetLastError(), "tile_ranges_kernel");
     GSX_TRY(record(ctx, 5, stream));
     const int tiles_padded = ((tiles + 7) / 8) * 8;
-    hipLaunchKernelGGL(blend_forward_kernel, dim3((unsigned)tiles_padded), dim3(256), 0, stream,
-                       ctx->ranges.as<uint2>(), ctx->sorted_vals, ctx->inst_gauss.as<uint32_t>(),
+    hipLaunchKernelGGL(train ? blend_forward_kernel<true> : blend_forward_kernel<false>, dim3((unsigned)tiles_padded),
+                       dim3(256), 0, stream, ctx->ranges.as<uint2>(), ctx->sorted_vals, ctx->inst_gauss.as<uint32_t>(),
                        ctx->rec.as<float4>(), ctx->rec.as<float4>() + 2 * n,
                        reinterpret_cast<const uint2*>(ctx->rec.as<float4>() + 3 * n),
-                       train ? ctx->sorted_g.as<uint32_t>() : nullptr, cam, out_rgb,
-                       ctx->final_t.as<float>(),
+                       train ? ctx->sorted_g.as<uint32_t>() : nullptr, cam, out_rgb, ctx->final_t.as<float>(),
                        ctx->last.as<uint32_t>(), train ? ctx->ckpt.as<float>() : nullptr);
     GSX_HIP_TRY(hipGetLastError(), "blend_forward_kernel");
     GSX_TRY(record(ctx, 6, stream));

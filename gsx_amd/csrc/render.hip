@@ -685,21 +685,68 @@ __device__ inline size_t checkpoint_slot(uint32_t range_start, int tile, uint32_
     return (size_t)(range_start / kBucket) + (size_t)tile + (size_t)((position - range_start) / kBucket);
 }
 
+// An entry of a tile's list as the blend kernels stage it in LDS, 48 bytes. The conic is stored as
+// (-a / 2, -b, -c / 2): the power -(a dx^2 + 2 b dx dy + c dy^2) / 2 then needs no final
+// multiplication, and every product rounds as the CPU's (a scaling by powers of two is exact).
+struct BlendEntry {
+    float4 a;  // mean2d x, y, -inv_a / 2, -inv_b
+    float4 b;  // -inv_c / 2, opacity, colour r, g
+    float4 c;  // colour b, contribution box low corner and extent (packed halves), next list position
+};
+
+__device__ inline BlendEntry blend_entry(float4 geo0, float4 geo1, float4 col, uint2 box, uint32_t next) {
+    BlendEntry e;
+    e.a = make_float4(geo0.x, geo0.y, -0.5f * geo0.z, -0.5f * geo0.w);
+    e.b = make_float4(-0.5f * geo1.x, geo1.y, col.x, col.y);
+    e.c = make_float4(col.z, __uint_as_float(box.x), __uint_as_float(box.y), __uint_as_float(next));
+    return e;
+}
+
+// Whether a packed contribution box meets the 8 x 8 quadrant whose first pixel is (qx, qy). Lane l
+// of a wave asks for entry l of 64, so one ballot tells the wave which of them it has to look at:
+// an entry that misses the quadrant costs 1/64 of this test instead of a box test by every pixel,
+// and the branches of the walk are scalar.
+__device__ inline bool box_meets_quadrant(uint32_t lo, uint32_t ext, uint32_t qx, uint32_t qy) {
+    const uint32_t x0 = lo & 0xffffu, y0 = lo >> 16;
+    return (x0 <= qx + 7u) & (x0 + (ext & 0xffffu) >= qx) & (y0 <= qy + 7u) & (y0 + (ext >> 16) >= qy);
+}
+
+// render.c:1045-1070 for one entry and pixel, without the transmittance: alpha, and whether the
+// pixel takes the entry if it is still open. A power above 0 counts as 0 and one below the cut is not
+// taken, so the exponential's argument is the power clamped to [cut, 0]; a NaN power is not taken.
+__device__ inline bool blend_alpha(const BlendEntry& e, float fpx, float fpy, uint32_t pxy, const uint64_t* s_exp2,
+                                   float& gval, float& alpha) {
+    const float dx = fpx - e.a.x;
+    const float dy = fpy - e.a.y;
+    const float power = e.a.z * dx * dx + e.a.w * dx * dy + e.b.x * dy * dy;
+    const bool near = in_box_packed(pxy, __float_as_uint(e.c.y), __float_as_uint(e.c.z)) & (power >= kPowerThreshold);
+    gval = gsx_expf_blend(__builtin_amdgcn_fmed3f(power, kPowerThreshold, 0.0f), s_exp2);
+    alpha = fminf(kMaxFragmentAlpha, e.b.y * gval);
+    return near & (alpha >= kMinAlpha);
+}
+
 // ---------------------------------------------------------------------------------------------
 // Blend forward: render.c:1018-1088, per pixel in per-tile (depth, index) order. Records of the
 // tile's Gaussians are staged through LDS in batches of 256; a tile stops early once every pixel
 // has T < 1e-4. Writes out_rgb (CHW, background composed: C + T*bg), final T, the exclusive end
 // of the last contributing position, and (TRAIN) the bucket checkpoints.
+// Each wave walks, 64 entries at a time, only the entries whose box meets its quadrant, in groups
+// of kGroup whose alphas (independent of the transmittance, some 30 dependent operations and two
+// LDS reads each) are evaluated side by side before they are composited in order: a tile's list is a
+// serial chain, which sets the time where few waves share a SIMD (4000 Gaussians on 48 tiles: 106 us
+// testing every entry one by one, 49 so), and the vector ALUs set it otherwise (1M Gaussians on a plane
+// at 1024^2: 506 -> 398 us; full-HD clusters 65 -> 55 us). Groups of 4 need 92 registers with the
+// checkpoints (5 waves per SIMD; 2 need 62): the TRAIN forward takes 2 (398 against 426 us).
 // ---------------------------------------------------------------------------------------------
+template <bool kTrain>
 __global__ __launch_bounds__(kBlendThreads) void blend_forward_kernel(
     const uint2* __restrict__ ranges, const uint32_t* __restrict__ values,
     const uint32_t* __restrict__ instance_gaussian, const float4* __restrict__ rec, const float4* __restrict__ col,
     const uint2* __restrict__ cbox, uint32_t* __restrict__ sorted_g,
     CameraParams cam, float* __restrict__ out_rgb,
     float* __restrict__ out_t, uint32_t* __restrict__ out_last, float* __restrict__ ckpt) {
-    __shared__ float4 s_r0[kBlendThreads];
-    __shared__ float4 s_r1[kBlendThreads];
-    __shared__ float4 s_r2[kBlendThreads];
+    constexpr int kGroup = kTrain ? 2 : 4;
+    __shared__ BlendEntry s_entry[kBlendThreads];
     __shared__ uint64_t s_exp2[GSX_EXPF_BLEND_TABLE_SIZE];
     const int tiles = cam.tiles_x * cam.tiles_y;
     const int tile = xcd_tile_index(blockIdx.x, tiles);
@@ -714,70 +761,92 @@ __global__ __launch_bounds__(kBlendThreads) void blend_forward_kernel(
     const float fpx = (float)px + 0.5f;
     const float fpy = (float)py + 0.5f;
     const uint32_t pxy = (uint32_t)px | ((uint32_t)py << 16);  // for in_box_packed
+    const uint32_t lane = __lane_id();
+    const uint32_t qx = (uint32_t)px & ~7u, qy = (uint32_t)py & ~7u;
     // t only falls, and a pixel is done once an accepted contribution takes it below the
     // threshold, so "done" is t < threshold; pixels outside the image start done (t = 0, never
     // written out)
     float t = inside ? 1.0f : 0.0f, c0 = 0.0f, c1 = 0.0f, c2 = 0.0f;
     uint32_t last = range.x;
-    for (uint32_t base = range.x; base < range.y; base += kBlendThreads) {
-        if (__syncthreads_count(t < kTransmittanceThreshold ? 1 : 0) == kBlendThreads) break;
-        const uint32_t j = base + threadIdx.x;
-        if (j < range.y) {
-            const uint32_t g = instance_gaussian[values[j]];
-            if (sorted_g != nullptr) sorted_g[j] = g;  // TRAIN: the backward reads it
-            const float4 geo1 = rec[2 * (size_t)g + 1], c = col[g];
-            const uint2 box = cbox[g];
-            s_r0[threadIdx.x] = rec[2 * (size_t)g + 0];
-            s_r1[threadIdx.x] = make_float4(geo1.x, geo1.y, c.x, c.y);
-            s_r2[threadIdx.x] = make_float4(c.z, __uint_as_float(box.x), __uint_as_float(box.y), c.w);
-        } else {
-            // past the list: a box no pixel lies in, so the last bucket can run whole
-            s_r2[threadIdx.x] = make_float4(0.0f, __uint_as_float(kEmptyBoxLo), 0.0f, 0.0f);
+    // The first batch is kFirstBatch entries, staged by four threads each: where near Gaussians
+    // saturate a tile its list ends there (metric scene: about 50 of some 650 entries per tile), and
+    // 256 would mostly be loaded in vain. Later batches are 256, one entry per thread, whose Gaussians
+    // are looked up a batch ahead.
+    constexpr uint32_t kFirstBatch = kWave;
+    uint32_t g_next = 0;
+    uint32_t batch = kFirstBatch;
+    for (uint32_t base = range.x; base < range.y; base += batch, batch = kBlendThreads) {
+        const bool first = base == range.x;
+        if (!first && __syncthreads_count(t < kTransmittanceThreshold ? 1 : 0) == kBlendThreads) break;
+        const uint32_t slot = first ? threadIdx.x / 4 : threadIdx.x;
+        const uint32_t j = base + slot;
+        // past the list: the last entry's records, with a box no pixel lies in
+        const uint32_t jc = min(j, range.y - 1u);
+        const uint32_t g = base <= range.x + kFirstBatch ? instance_gaussian[values[jc]] : g_next;
+        if (kTrain && j < range.y && (!first || (threadIdx.x & 3u) == 3u)) sorted_g[j] = g;  // for the backward
+        const BlendEntry mine = blend_entry(rec[2 * (size_t)g], rec[2 * (size_t)g + 1], col[g],
+                                            j < range.y ? cbox[g] : make_uint2(kEmptyBoxLo, 0u), j + 1u);
+        if (!first) {
+            s_entry[slot] = mine;
+            if (range.y - base > (uint32_t)kBlendThreads)
+                g_next = instance_gaussian[values[min(j + (uint32_t)kBlendThreads, range.y - 1u)]];
+        } else if ((threadIdx.x & 3u) == 0u) {
+            s_entry[slot] = mine;
         }
         __syncthreads();
-        // wave-uniform bound, held in a scalar register, rounded up to whole buckets
-        const int count = __builtin_amdgcn_readfirstlane((int)min((uint32_t)kBlendThreads, range.y - base));
-        const int padded = (count + kBucket - 1) & ~(kBucket - 1);
-        // the lanes not done (t only changes where an entry is evaluated, so the mask is
-        // re-formed there, not per entry)
-        uint64_t open_mask = wave_ballot(t >= kTransmittanceThreshold);
-        // buckets of kBucket entries, each unrolled: the checkpoint at the bucket's start and
-        // the loop control cost no instructions per entry
-        for (int k0 = 0; k0 < padded; k0 += kBucket) {
-            if (mask_none(open_mask)) break;  // uniform: every pixel of this wave is saturated
-            if (ckpt != nullptr && t >= kTransmittanceThreshold)
-                ckpt[checkpoint_slot(range.x, tile, base + (uint32_t)k0) * kBlendThreads + threadIdx.x] = t;
+        // wave-uniform bound, held in a scalar register
+        const int count = __builtin_amdgcn_readfirstlane((int)min(batch, range.y - base));
+        uint64_t open = wave_ballot(t >= kTransmittanceThreshold);
+        // one entry's place in the order: its (independent) alpha composited where the pixel is open
+        int bucket = -1;
+        auto composite = [&](int k, bool ok, float alpha, const BlendEntry& e) {
+            if (kTrain && k / kBucket != bucket) {  // uniform: the first entry of a bucket in this quadrant
+                bucket = k / kBucket;
+                if (t >= kTransmittanceThreshold)
+                    ckpt[checkpoint_slot(range.x, tile, base + (uint32_t)k) * kBlendThreads + threadIdx.x] = t;
+            }
+            // a lane that does not take the entry uses alpha = 0: it adds (0 * colour) = +-0, which
+            // leaves its sums exactly as they are (they start at +0 and stay finite), and multiplies t
+            // by 1, so one select serves the colour sums and t
+            const bool take = ok & (t >= kTransmittanceThreshold);
+            const float a_used = take ? alpha : 0.0f;
+            const float w = a_used * t;
+            c0 = c0 + w * e.b.z;
+            c1 = c1 + w * e.b.w;
+            c2 = c2 + w * e.c.x;
+            t = t * (1.0f - a_used);
+            last = take ? __float_as_uint(e.c.w) : last;
+        };
+        for (int k0 = 0; k0 < count && !mask_none(open); k0 += kWave) {
+            const BlendEntry& mine = s_entry[k0 + lane];
+            uint64_t todo = wave_ballot(
+                box_meets_quadrant(__float_as_uint(mine.c.y), __float_as_uint(mine.c.z), qx, qy));
+            while (todo != 0ull) {
+                if (__builtin_popcountll(todo) >= kGroup) {
+                    int k[kGroup];
+                    bool ok[kGroup];
+                    float alpha[kGroup], gval;
+                    BlendEntry e[kGroup];
 #pragma unroll
-            for (int i = 0; i < kBucket; ++i) {
-                const int k = k0 + i;
-                const float4 r2 = s_r2[k];
-                const bool ib = in_box_packed(pxy, __float_as_uint(r2.y), __float_as_uint(r2.z));
-                const uint64_t live_mask = open_mask & wave_ballot(ib);
-                if (mask_none(live_mask)) continue;  // uniform
-                const bool live = __builtin_amdgcn_inverse_ballot_w64(live_mask);
-                // branch-free evaluation for the wave; lanes outside the box or done keep their state
-                const float4 r0 = s_r0[k];
-                const float4 r1 = s_r1[k];
-                const float dx = fpx - r0.x;
-                const float dy = fpy - r0.y;
-                float power = -0.5f * (r0.z * dx * dx + r0.w * dx * dy + r1.x * dy * dy);
-                power = power > 0.0f ? 0.0f : power;
-                bool ok = live & (power >= kPowerThreshold);
-                const float gval = gsx_expf_blend(fmaxf(power, kPowerThreshold), s_exp2);
-                const float alpha = fminf(kMaxFragmentAlpha, r1.y * gval);
-                ok = ok & (alpha >= kMinAlpha);
-                // a lane that does not take the entry uses alpha = 0: it adds (0 * colour) = +-0,
-                // which leaves its sums exactly as they are (they start at +0 and stay finite), and
-                // multiplies t by 1, so one select serves the colour sums and t
-                const float a_used = ok ? alpha : 0.0f;
-                const float w = a_used * t;
-                c0 = c0 + w * r1.z;
-                c1 = c1 + w * r1.w;
-                c2 = c2 + w * r2.x;
-                t = t * (1.0f - a_used);
-                last = ok ? base + (uint32_t)k + 1u : last;
-                open_mask = wave_ballot(t >= kTransmittanceThreshold);
-                if (mask_none(open_mask)) break;  // uniform
+                    for (int i = 0; i < kGroup; ++i) {
+                        k[i] = k0 + __builtin_ctzll(todo);
+                        todo &= todo - 1ull;
+                        e[i] = s_entry[k[i]];
+                    }
+#pragma unroll
+                    for (int i = 0; i < kGroup; ++i) ok[i] = blend_alpha(e[i], fpx, fpy, pxy, s_exp2, gval, alpha[i]);
+#pragma unroll
+                    for (int i = 0; i < kGroup; ++i) composite(k[i], ok[i], alpha[i], e[i]);
+                } else {
+                    const int k = k0 + __builtin_ctzll(todo);
+                    todo &= todo - 1ull;
+                    const BlendEntry e = s_entry[k];
+                    float alpha, gval;
+                    const bool ok = blend_alpha(e, fpx, fpy, pxy, s_exp2, gval, alpha);
+                    composite(k, ok, alpha, e);
+                }
+                open = wave_ballot(t >= kTransmittanceThreshold);
+                if (mask_none(open)) break;  // uniform: every pixel of this wave is saturated
             }
         }
         __syncthreads();
