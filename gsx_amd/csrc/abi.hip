@@ -262,7 +262,7 @@ int bits_for(uint32_t v) {
 }  // namespace
 
 struct gsx_hip_render_context {
-    DeviceBuffer rec, cov_coef, ckpt, inst_gauss, inst_tile, tiles_alt, tiles_sorted, vals_alt, vals, tile_cut, touched,
+    DeviceBuffer rec, cov_coef, ckpt, inst_gauss, inst_tile, tiles_alt, tiles_sorted, vals_alt, vals, tile_cut, tile_exact, touched,
         inst_grad, tile_count, big_list, offsets, scan_temp, sort_temp, ranges, sorted_g, final_t, last, grad2d,
         depth_keys, depth_keys_alt, rank_g, rank_count, g_rank, long_list, multi_list, counters,
         depth_sort_temp;
@@ -588,7 +588,7 @@ gsx_hip_status gsx_hip_render_context_destroy(gsx_hip_render_context* ctx) {
     if (ctx == nullptr) return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "context must be non-null");
     DeviceBuffer* all[] = {&ctx->rec,       &ctx->cov_coef, &ctx->ckpt,      &ctx->inst_gauss, &ctx->inst_tile,
                            &ctx->tiles_alt, &ctx->tiles_sorted, &ctx->vals_alt, &ctx->vals,
-                           &ctx->tile_cut,  &ctx->touched,  &ctx->inst_grad,
+                           &ctx->tile_cut,  &ctx->tile_exact, &ctx->touched,  &ctx->inst_grad,
                            &ctx->tile_count, &ctx->big_list, &ctx->offsets,   &ctx->scan_temp,
                            &ctx->sort_temp,  &ctx->ranges,
                            &ctx->sorted_g,   &ctx->final_t,  &ctx->last,      &ctx->grad2d,     &ctx->depth_keys,
@@ -716,6 +716,7 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     GSX_TRY(ctx->rec.reserve(n1 * (3 * sizeof(float4) + sizeof(uint2)), "rec", ctx->call_stream));
     if (train) GSX_TRY(ctx->cov_coef.reserve(n1 * 2 * sizeof(float4), "cov_coef", ctx->call_stream));
     if (train) GSX_TRY(ctx->touched.reserve(n1, "touched", ctx->call_stream));
+    if (train) GSX_TRY(ctx->tile_exact.reserve((size_t)tiles * sizeof(uint32_t), "tile_exact", ctx->call_stream));
     GSX_TRY(ctx->tile_count.reserve(n1 * sizeof(uint32_t), "tile_count", ctx->call_stream));
     GSX_TRY(ctx->counters.reserve(8 * sizeof(uint32_t), "counters", ctx->call_stream));
     GSX_TRY(ctx->big_list.reserve(n1 * sizeof(uint32_t), "big_list", ctx->call_stream));
@@ -897,7 +898,8 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
                        ctx->rec.as<float4>(), ctx->rec.as<float4>() + 2 * n,
                        reinterpret_cast<const uint2*>(ctx->rec.as<float4>() + 3 * n),
                        train ? ctx->sorted_g.as<uint32_t>() : nullptr, cam, out_rgb, ctx->final_t.as<float>(),
-                       ctx->last.as<uint32_t>(), train ? ctx->ckpt.as<float>() : nullptr);
+                       ctx->last.as<uint32_t>(), train ? ctx->ckpt.as<float>() : nullptr,
+                       train ? ctx->tile_exact.as<uint32_t>() : nullptr);
     GSX_HIP_TRY(hipGetLastError(), "blend_forward_kernel");
     GSX_TRY(record(ctx, 6, stream));
     if (ctx->timing && ctx->cur >= 0) ctx->has_fwd[ctx->cur] = 1;
@@ -949,7 +951,7 @@ gsx_hip_status enqueue_backward(gsx_hip_render_context* ctx, const float* grad_r
     hipLaunchKernelGGL(blend_backward_kernel, dim3((unsigned)tiles_padded), dim3(256), 0, stream,
                        ctx->ranges.as<uint2>(), svals, ctx->sorted_g.as<uint32_t>(), ctx->rec.as<float4>(),
                        ctx->rec.as<float4>() + 2 * n, reinterpret_cast<const uint2*>(ctx->rec.as<float4>() + 3 * n),
-                       ctx->cov_coef.as<float4>(), ctx->ckpt.as<float>(), cam, grad_rgb, ctx->final_t.as<float>(),
+                       ctx->cov_coef.as<float4>(), ctx->ckpt.as<float>(), ctx->tile_exact.as<uint32_t>(), cam, grad_rgb, ctx->final_t.as<float>(),
                        ctx->last.as<uint32_t>(), ctx->inst_grad.as<float>(), inst_grad_op,
                        ctx->tile_cut.as<uint32_t>(), ctx->touched.as<uint8_t>(), sinks);
     GSX_HIP_TRY(hipGetLastError(), "blend_backward_kernel");

@@ -413,6 +413,12 @@ __device__ inline uint32_t wave_min_u32(uint32_t v) {
     return v;
 }
 
+__device__ inline uint32_t wave_max_u32(uint32_t v) {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, off, kWave));
+    return v;
+}
+
 // Orders the LDS accesses of one wave around this point (the lanes of a wave exchange data
 // through LDS without a workgroup barrier).
 __device__ inline void wave_lds_sync() {
@@ -461,50 +467,6 @@ __device__ inline uint32_t wave_reduce_sum_u32(uint32_t v) {
     v += dpp_move_u32<0x142, 0xa>(v);
     v += dpp_move_u32<0x143, 0xc>(v);
     return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-}
-
-// Row totals (over the 16 lanes of each DPP row) of v[0..8], scattered over the row: the returned
-// value of lane l (l = lane index within its row) is the row total of v[(l >> 1) & 7], and
-// total8 receives the row total of v[8] in every lane. Each step pairs every lane with a partner
-// whose lane-group bit differs and halves the values a lane carries: the lane keeps one half and
-// sends its partner the other (two lane-constant selects), and adds what the partner sent (one
-// fused DPP add). Partners: row rotate by 8 (l ^ 8, group bit 3), row half mirror (l ^ 7 within
-// each 8-lane half, group bit 2), quad permute l ^ 2 (bit 1), then l ^ 1 adds the last value:
-// 22 lane operations for the 8 values instead of 32, plus 4 for v[8], and 8 lanes of a row hold
-// the 8 totals, so one store writes them all.
-__device__ inline float row_reduce_scatter9(const float (&v)[9], float& total8) {
-    // lane-constant predicates from constant lane masks (scalar moves; (l & 8) != 0 etc. would be
-    // recomputed with vector instructions wherever scalar registers run short)
-    const bool b3 = __builtin_amdgcn_inverse_ballot_w64(0xff00ff00ff00ff00ull);  // lane bit 3
-    const bool b2 = __builtin_amdgcn_inverse_ballot_w64(0xf0f0f0f0f0f0f0f0ull);  // lane bit 2
-    const bool b1 = __builtin_amdgcn_inverse_ballot_w64(0xccccccccccccccccull);  // lane bit 1
-    float b[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        // lanes 0-7 of the row keep v[i], lanes 8-15 keep v[4 + i]
-        const float keep = b3 ? v[4 + i] : v[i];
-        const float send = b3 ? v[i] : v[4 + i];
-        b[i] = keep + dpp_move<0x128, 0xf>(send);  // row_ror:8
-    }
-    float c[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        // lanes with bit 2 clear keep b[i], the others b[2 + i]
-        const float keep = b2 ? b[2 + i] : b[i];
-        const float send = b2 ? b[i] : b[2 + i];
-        c[i] = keep + dpp_move<0x141, 0xf>(send);  // row_half_mirror
-    }
-    const float keep = b1 ? c[1] : c[0];
-    const float send = b1 ? c[0] : c[1];
-    float d = keep + dpp_move<0x4e, 0xf>(send);  // quad_perm [2,3,0,1]
-    d += dpp_move<0xb1, 0xf>(d);                 // quad_perm [1,0,3,2]
-    float t = v[8];
-    t += dpp_move<0xb1, 0xf>(t);
-    t += dpp_move<0x4e, 0xf>(t);
-    t += dpp_move<0x141, 0xf>(t);  // row_half_mirror
-    t += dpp_move<0x140, 0xf>(t);  // row_mirror
-    total8 = t;
-    return d;
 }
 
 // n / d rounded to nearest for normal, finite operands whose quotient is normal (no scaling

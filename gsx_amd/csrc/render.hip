@@ -711,15 +711,38 @@ __device__ inline bool box_meets_quadrant(uint32_t lo, uint32_t ext, uint32_t qx
     return (x0 <= qx + 7u) & (x0 + (ext & 0xffffu) >= qx) & (y0 <= qy + 7u) & (y0 + (ext >> 16) >= qy);
 }
 
+// A regular entry: its 2D covariance has an eigenvalue ratio of at most kRegularRatio and eigenvalues
+// of at most kRegularExtent (a standard deviation of 1024 pixels). With trace t and determinant d of
+// the conic, ratio <= r iff t^2 <= d (r + 2 + 1 / r), and the covariance's larger eigenvalue is at most
+// t / d; from the staged conic (halved: t / 2 and d / 4). A NaN is not regular.
+//  * A pixel outside a regular entry's 3-sigma box fails the power cut by itself: it lies at least half
+//    a pixel beyond 3 sigma, where the power is below -4.5 (1 + 1 / (3 sigma)) <= -4.5 (1 + 3e-4), and
+//    the float evaluation is off by less than 6e-5 of it (the form's terms are at most 2 r = 128 times
+//    their sum, each rounded a few times). So its pixels need no box test: 3 instructions of some 40,
+//    left out where a whole tile is regular (blend_backward_kernel's moments: 934 -> 906 us at 1M
+//    Gaussians on a plane; a branch per group in the forward cost more than it saved, 394 -> 417 us).
+//  * The map from moments to covariance gradients loses no more digits than the ratio says
+//    (blend_backward_kernel).
+constexpr float kRegularRatio = 64.0f;
+constexpr float kRegularExtent = 1048576.0f;
+__device__ inline bool entry_is_regular(const BlendEntry& e) {
+    const float half_trace = -(e.a.z + e.b.x);
+    const float quarter_det = e.a.z * e.b.x - 0.25f * e.a.w * e.a.w;
+    return (half_trace * half_trace <= quarter_det * (kRegularRatio + 2.0f + 1.0f / kRegularRatio)) &
+           (half_trace <= quarter_det * (2.0f * kRegularExtent));
+}
+
 // render.c:1045-1070 for one entry and pixel, without the transmittance: alpha, and whether the
 // pixel takes the entry if it is still open. A power above 0 counts as 0 and one below the cut is not
 // taken, so the exponential's argument is the power clamped to [cut, 0]; a NaN power is not taken.
+template <bool kBoxTest>
 __device__ inline bool blend_alpha(const BlendEntry& e, float fpx, float fpy, uint32_t pxy, const uint64_t* s_exp2,
                                    float& gval, float& alpha) {
     const float dx = fpx - e.a.x;
     const float dy = fpy - e.a.y;
     const float power = e.a.z * dx * dx + e.a.w * dx * dy + e.b.x * dy * dy;
-    const bool near = in_box_packed(pxy, __float_as_uint(e.c.y), __float_as_uint(e.c.z)) & (power >= kPowerThreshold);
+    bool near = power >= kPowerThreshold;
+    if (kBoxTest) near = near & in_box_packed(pxy, __float_as_uint(e.c.y), __float_as_uint(e.c.z));
     gval = gsx_expf_blend(__builtin_amdgcn_fmed3f(power, kPowerThreshold, 0.0f), s_exp2);
     alpha = fminf(kMaxFragmentAlpha, e.b.y * gval);
     return near & (alpha >= kMinAlpha);
@@ -744,14 +767,17 @@ __global__ __launch_bounds__(kBlendThreads) void blend_forward_kernel(
     const uint32_t* __restrict__ instance_gaussian, const float4* __restrict__ rec, const float4* __restrict__ col,
     const uint2* __restrict__ cbox, uint32_t* __restrict__ sorted_g,
     CameraParams cam, float* __restrict__ out_rgb,
-    float* __restrict__ out_t, uint32_t* __restrict__ out_last, float* __restrict__ ckpt) {
+    float* __restrict__ out_t, uint32_t* __restrict__ out_last, float* __restrict__ ckpt,
+    uint32_t* __restrict__ tile_exact) {
     constexpr int kGroup = kTrain ? 2 : 4;
     __shared__ BlendEntry s_entry[kBlendThreads];
     __shared__ uint64_t s_exp2[GSX_EXPF_BLEND_TABLE_SIZE];
+    __shared__ uint32_t s_exact;  // TRAIN: an entry that a wave looked at is not regular
     const int tiles = cam.tiles_x * cam.tiles_y;
     const int tile = xcd_tile_index(blockIdx.x, tiles);
     if (tile >= tiles) return;
     if (threadIdx.x < GSX_EXPF_BLEND_TABLE_SIZE) s_exp2[threadIdx.x] = gsx_expf_blend_entry(threadIdx.x);
+    if (kTrain && threadIdx.x == 0) s_exact = 0u;
     const int tx = tile % cam.tiles_x, ty = tile / cam.tiles_x;
     const int2 tp = tile_pixel_of_thread((int)threadIdx.x);
     const int px = tx * kTile + tp.x;
@@ -821,6 +847,7 @@ __global__ __launch_bounds__(kBlendThreads) void blend_forward_kernel(
             const BlendEntry& mine = s_entry[k0 + lane];
             uint64_t todo = wave_ballot(
                 box_meets_quadrant(__float_as_uint(mine.c.y), __float_as_uint(mine.c.z), qx, qy));
+            if (kTrain && !mask_none(wave_ballot(!entry_is_regular(mine)) & todo) && lane == 0u) s_exact = 1u;
             while (todo != 0ull) {
                 if (__builtin_popcountll(todo) >= kGroup) {
                     int k[kGroup];
@@ -834,7 +861,8 @@ __global__ __launch_bounds__(kBlendThreads) void blend_forward_kernel(
                         e[i] = s_entry[k[i]];
                     }
 #pragma unroll
-                    for (int i = 0; i < kGroup; ++i) ok[i] = blend_alpha(e[i], fpx, fpy, pxy, s_exp2, gval, alpha[i]);
+                    for (int i = 0; i < kGroup; ++i)
+                        ok[i] = blend_alpha<true>(e[i], fpx, fpy, pxy, s_exp2, gval, alpha[i]);
 #pragma unroll
                     for (int i = 0; i < kGroup; ++i) composite(k[i], ok[i], alpha[i], e[i]);
                 } else {
@@ -842,7 +870,7 @@ __global__ __launch_bounds__(kBlendThreads) void blend_forward_kernel(
                     todo &= todo - 1ull;
                     const BlendEntry e = s_entry[k];
                     float alpha, gval;
-                    const bool ok = blend_alpha(e, fpx, fpy, pxy, s_exp2, gval, alpha);
+                    const bool ok = blend_alpha<true>(e, fpx, fpy, pxy, s_exp2, gval, alpha);
                     composite(k, ok, alpha, e);
                 }
                 open = wave_ballot(t >= kTransmittanceThreshold);
@@ -851,6 +879,8 @@ __global__ __launch_bounds__(kBlendThreads) void blend_forward_kernel(
         }
         __syncthreads();
     }
+    // (an empty list never reaches the barriers that order s_exact; its backward walks nothing)
+    if (kTrain && threadIdx.x == 0) tile_exact[tile] = range.x < range.y ? s_exact : 0u;
     if (inside) {
         const size_t pix = (size_t)py * (size_t)cam.width + (size_t)px;
         const size_t plane = (size_t)cam.width * (size_t)cam.height;
@@ -871,81 +901,446 @@ constexpr int kGradRecord = 8;  // per-instance partials: channels 0-7 in one 32
 // Blend backward: render.c:1559-1666 restated per pixel, back to front, with the CPU's exact
 // T_before: for each 8-entry bucket (last first) the pixel reloads the bucket's checkpointed T,
 // replays the bucket forward (same operations as the forward, so T_before, G and the contribution
-// set are bit-identical to the CPU's) and then walks it backwards accumulating the suffix colour
-// exactly as the CPU does. Per contribution the gradient terms are the CPU's, including the
-// d(conic)/d(cov2d) map applied per contribution.
-// Reduction without atomics: each 16-pixel row sums its lanes' 9 partials per entry with DPP
-// moves (row_reduce_scatter9), the 16 row totals are combined through LDS, and the tile writes
-// one 9-float partial per reached instance at its emission position (channels 0-7 as one 32-byte
-// record of instance_grad, channel 8, the opacity term, in instance_grad_op) and its cut
-// position (tile_cut: the instances past it were not reached and have no partial);
-// reduce_instance_grads_kernel then sums each Gaussian's contiguous run of positions. The result
-// is deterministic and immune to the contention of full-screen Gaussians (present in every tile),
-// and the instances behind saturated pixels cost the backward nothing.
+// set are bit-identical to the CPU's) and then walks it backwards accumulating the suffix colour.
+// Each wave looks only at the entries that meet its quadrant, as the forward does.
+//
+// A tile takes one of two forms of the gradient terms (tile_exact, from the forward):
+//  * Moments. Every term of an entry's nine partials is one of two per-pixel scalars, h = dL/dopacity
+//    of the pixel and w = alpha T, times something fixed over the list: with dpow = opacity h,
+//      dmean2d, d(conic)  are sums of dpow times 1, dx, dy, dx^2, dx dy, dy^2,
+//      dcolor             are sums of w times the pixel's image gradient.
+//    So the sum over a quadrant's 64 pixels is a product of matrices: 16 rows (h and w of 8 entries)
+//    by 64 pixels, times 64 pixels by 9 columns (the monomials of the pixel's offset u, v from the
+//    quadrant's centre, |u|, |v| <= 3.5, and the three image gradients): 16 f32 16x16x4 matrix
+//    instructions per 8 entries. (On gfx950 an f32 matrix instruction takes the vector ALUs' time,
+//    about 7 vector instructions' worth; that is 15 per entry, where the products and their reduction
+//    over lanes took some 60.) Once per entry and tile the moments are moved from the quadrants'
+//    centres to the entry's mean, added over the quadrants, and mapped through the conic and the
+//    d(conic)/d(cov2d) coefficients. The suffix is one scalar, its product with the image gradient.
+//  * Per contribution. That map amplifies rounding by the eigenvalue ratio of the 2D covariance:
+//    near-plane Gaussians reach ratios of 1e6 and more, where the CPU's gradient is mostly the
+//    rounding of its per-contribution map. A tile with an entry that is not regular forms every term per contribution with the CPU's operations, the suffix colour and its division
+//    included, and sums the nine values over the wave with lane swaps and DPP moves.
+//
+// Reduction without atomics: every wave leaves one row of nine sums per entry in LDS, four threads
+// per entry combine the four waves' rows, and the tile writes one 9-float partial per reached
+// instance at its emission position (channels 0-7 as one 32-byte record of instance_grad, channel 8,
+// the opacity term, in instance_grad_op) and its cut position (tile_cut: the instances past it were
+// not reached and have no partial); reduce_instance_grads_kernel then sums each Gaussian's
+// contiguous run of positions. The result is deterministic and immune to the contention of
+// full-screen Gaussians (present in every tile), and the instances behind saturated pixels cost the
+// backward nothing.
 // ---------------------------------------------------------------------------------------------
 constexpr int kWavesPerTile = kBlendThreads / kWave;
-constexpr int kRowsPerTile = kTile;  // 16 DPP rows of 16 lanes per workgroup
 
-// The backward stages 64 entries per batch (8 buckets of 8): the kernel fits 71 VGPRs and 19 KB
-// of LDS, i.e. 7 waves per SIMD (16-entry buckets need 87 VGPRs and 28 KB: 5 waves; the
-// checkpoints of the smaller buckets cost the forward less than the occupancy gains here).
+// Entries per batch: staged together, four threads each, and combined together.
 constexpr int kBackBatch = 64;
-constexpr int kBatchBuckets = kBackBatch / kBucket;
+constexpr int kMomentEntries = 8;  // entries of one matrix product
 
-__global__ __launch_bounds__(kBlendThreads) void blend_backward_kernel(
+typedef float gsx_f32x4 __attribute__((ext_vector_type(4)));
+
+// Sum over the four lanes of a quad, in every lane.
+__device__ inline float quad_sum(float v) {
+    v += dpp_move<0xb1, 0xf>(v);        // quad_perm [1,0,3,2]
+    return v + dpp_move<0x4e, 0xf>(v);  // quad_perm [2,3,0,1]
+}
+
+// a's and b's sums over the lane pairs (l, l + 32): a's in lanes 0-31, b's in lanes 32-63.
+__device__ inline float merge_halves(float a, float b) {
+    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+// The same over neighbouring rows of 16 lanes: a's in rows 0 and 2, b's in rows 1 and 3.
+__device__ inline float merge_rows(float a, float b) {
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+
+// Sums of v[0..8] over the wave: the returned value of lane l is the sum of v[wave_sum9_index(l)],
+// total8 that of v[8] in lane 63. Each merge halves the registers and the lanes a value spreads
+// over: 24 lane operations for all nine.
+__device__ inline int wave_sum9_index(uint32_t lane) {
+    return (int)(((lane >> 1) & 4u) | ((lane >> 3) & 2u) | (lane >> 5));
+}
+__device__ inline float wave_sum9(const float (&v)[9], float& total8) {
+    const float a = merge_rows(merge_halves(v[0], v[1]), merge_halves(v[2], v[3]));  // rows: 0, 2, 1, 3
+    const float b = merge_rows(merge_halves(v[4], v[5]), merge_halves(v[6], v[7]));  // rows: 4, 6, 5, 7
+    const bool b3 = __builtin_amdgcn_inverse_ballot_w64(0xff00ff00ff00ff00ull);      // lane bit 3
+    const float keep = b3 ? b : a;
+    const float send = b3 ? a : b;
+    float d = keep + dpp_move<0x128, 0xf>(send);  // row_ror:8
+    d += dpp_move<0x141, 0xf>(d);                 // row_half_mirror
+    d = quad_sum(d);
+    float t = quad_sum(v[8]);
+    t += dpp_move<0x141, 0xf>(t);  // row_half_mirror
+    t += dpp_move<0x140, 0xf>(t);  // row_mirror
+    t += dpp_move<0x142, 0xa>(t);  // row_bcast:15 into rows 1 and 3
+    t += dpp_move<0x143, 0xc>(t);  // row_bcast:31 into rows 2 and 3
+    total8 = t;
+    return d;
+}
+
+// LDS of a backward workgroup. s_sum: per wave a row of nine sums for each entry that it took, the
+// highest entry first (s_used: which); a product writes kMomentEntries rows whatever its fill.
+struct BackwardShared {
+    BlendEntry entry[kBackBatch];  // c.w: the entry's emission position
+    uint64_t exp2[GSX_EXPF_BLEND_TABLE_SIZE];
+    uint64_t used[kWavesPerTile];
+    uint32_t max_last;
+    float sum[kWavesPerTile][(kBackBatch + kMomentEntries) * kGrad2d];
+    union {
+        // rows 2 i (h) and 2 i + 1 (w) of the i-th entry of a product, 64 pixels each; the 4-float
+        // blocks of row r are stored at block index ^ r, so that 16 lanes that read one block of 16
+        // rows meet all banks
+        alignas(256) float x[kWavesPerTile][2 * kMomentEntries * kWave];
+        float4 k[2][kBackBatch];  // d(conic)/d(cov2d) coefficients (per contribution)
+    };
+};
+
+// What a thread knows of its pixel.
+struct BackwardPixel {
+    float fpx, fpy;
+    uint32_t pxy;
+    uint32_t last;      // exclusive end of its contributions (the list's start: none, or outside)
+    float t_final;
+    float d0, d1, d2;   // image gradient
+};
+
+// The tile's list walked back to front: batches, within them the buckets that hold an entry for the
+// wave. Workgroup-uniform arguments except pix.
+template <bool kMoments>
+__device__ inline void blend_backward_walk(BackwardShared& sm, const BackwardPixel& pix, uint2 range, int tile, int tx,
+                                           int ty, uint32_t wave_last, uint32_t end_all, uint32_t part_end,
+                                           const uint32_t* __restrict__ values, const uint32_t* __restrict__ sorted_g,
+                                           const float4* __restrict__ rec, const float4* __restrict__ col,
+                                           const uint2* __restrict__ cbox, const float4* __restrict__ cov_coef,
+                                           const float* __restrict__ ckpt, const CameraParams& cam,
+                                           float* __restrict__ instance_grad, float* __restrict__ instance_grad_op,
+                                           uint8_t* __restrict__ touched) {
+    const uint32_t lane = __lane_id();
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const float d0 = pix.d0, d1 = pix.d1, d2 = pix.d2;
+    // render.c:1552-1557: the suffix starts as T_final * background (moments: times the gradient)
+    float s0 = pix.t_final * cam.bg[0], s1 = pix.t_final * cam.bg[1], s2 = pix.t_final * cam.bg[2];
+    if (kMoments) s0 = s0 * d0 + s1 * d1 + s2 * d2;
+
+    // Moments: this lane's column of the products' second factor, one value per step: step s takes the
+    // pixels 16 (lane / 16) + s of the quadrant. Columns 0-5: 1, u, v, u^2, u v, v^2; 6-8: the image
+    // gradient.
+    float* const x = sm.x[wave];
+    const uint32_t column = lane & 15u;
+    float factor[kMoments ? 16 : 1];
+    if constexpr (kMoments) {
+        x[lane] = d0;
+        x[kWave + lane] = d1;
+        x[2 * kWave + lane] = d2;
+        wave_lds_sync();
+        const float* dcol = x + kWave * (min(max((int)column, 6), 8) - 6) + 16 * (lane >> 4);
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const float u = (float)(s & 7) - 3.5f, v = (float)(2 * (int)(lane >> 4) + (s >> 3)) - 3.5f;
+            float f = dcol[s];
+            if (column == 0) f = 1.0f;
+            if (column == 1) f = u;
+            if (column == 2) f = v;
+            if (column == 3) f = u * u;
+            if (column == 4) f = u * v;
+            if (column == 5) f = v * v;
+            factor[s] = column < 9u ? f : 0.0f;
+        }
+        wave_lds_sync();
+    }
+    // where this lane reads its row of the first factor: row lane % 16, block 4 (lane / 16) of it (and,
+    // for t = 1..3, that byte offset ^ 16 t)
+    const uint32_t read_at = column * (kWave * 4u) + ((4u * (lane >> 4)) ^ column) * 16u;
+
+    const uint32_t first_batch = range.x + ((end_all - 1u - range.x) / kBackBatch) * kBackBatch;
+    // part p of entry e of a batch is staged by thread 4 e + p, its Gaussian and position looked up a batch
+    // ahead. sorted_g was written by the TRAIN forward for every batch that it staged, and every entry below
+    // part_end lies in one; threads past the batch repeat its first entry, with an empty box.
+    const uint32_t e = threadIdx.x >> 2, p = threadIdx.x & 3u;
+    uint32_t j = first_batch + e < part_end ? first_batch + e : first_batch;
+    uint32_t g = sorted_g[j], position = values[j];
+    for (int64_t bstart = first_batch; bstart >= (int64_t)range.x; bstart -= kBackBatch) {
+        const int count = (int)min((uint32_t)kBackBatch, part_end - (uint32_t)bstart);
+        {
+            const bool in = (int)e < count;
+            const float4* const first = p < 2 ? rec + 2 * (size_t)g + p : (p == 2 ? col + g : cov_coef + 2 * (size_t)g);
+            const float4* const second = p == 3 ? cov_coef + 2 * (size_t)g + 1 : col + g;
+            const float4 x0 = *first, x1 = *second;
+            const uint2 box = cbox[g];
+            if (p == 3) {
+                if (!kMoments) {
+                    sm.k[0][e] = x0;
+                    sm.k[1][e] = x1;
+                }
+                if (in && j < end_all) touched[g] = 1;
+            } else {
+                float4 y = make_float4(x0.x, x0.y, -0.5f * x0.z, -0.5f * x0.w);
+                if (p == 1) y = make_float4(-0.5f * x0.x, x0.y, x1.x, x1.y);
+                if (p == 2)
+                    y = make_float4(x0.z, __uint_as_float(in ? box.x : kEmptyBoxLo), __uint_as_float(in ? box.y : 0u),
+                                    __uint_as_float(position));
+                reinterpret_cast<float4*>(&sm.entry[e])[p] = y;
+            }
+        }
+        const uint32_t g_combine = g;
+        if (bstart > (int64_t)range.x) {
+            j = (uint32_t)bstart - kBackBatch + e;
+            g = sorted_g[j];
+            position = values[j];
+        }
+        __syncthreads();
+        // the entries of the batch that meet this quadrant before its pixels' last contribution
+        uint64_t todo;
+        {
+            const BlendEntry& mine = sm.entry[lane];
+            todo = wave_ballot((uint32_t)bstart + lane < wave_last &&
+                               box_meets_quadrant(__float_as_uint(mine.c.y), __float_as_uint(mine.c.z),
+                                                  (pix.pxy & 0xffffu) & ~7u, (pix.pxy >> 16) & ~7u));
+        }
+        // `rows` rows of sums are taken, the last `fill` of them still rows of x
+        int rows = 0, fill = 0;
+        uint64_t used = 0;
+        auto flush = [&]() {
+            wave_lds_sync();
+            gsx_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            const char* const xb = reinterpret_cast<const char*>(x);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const float4 a = *reinterpret_cast<const float4*>(xb + (read_at ^ (16u * t)));
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, factor[kMoments ? 4 * t : 0], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, factor[kMoments ? 4 * t + 1 : 0], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, factor[kMoments ? 4 * t + 2 : 0], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, factor[kMoments ? 4 * t + 3 : 0], acc, 0, 0, 0);
+            }
+            // lane l holds rows 4 (l / 16) .. + 3 of column l % 16: h and w of two entries
+            if (column < 9u) {
+                float* const to = &sm.sum[wave][(rows - fill + 2 * (int)(lane >> 4)) * kGrad2d + (int)column];
+                to[0] = column < 6u ? acc.x : acc.y;
+                to[kGrad2d] = column < 6u ? acc.z : acc.w;
+            }
+            wave_lds_sync();
+            fill = 0;
+        };
+        // a pixel that needs no checkpoint of a bucket reads one all the same (the slot exists) and drops it
+        auto checkpoint = [&](int bucket) {
+            return ckpt[checkpoint_slot(range.x, tile, (uint32_t)bstart + (uint32_t)(bucket * kBucket)) * kBlendThreads +
+                        threadIdx.x];
+        };
+        float next_t = 0.0f;
+        if (todo != 0ull) next_t = checkpoint((63 - __builtin_clzll(todo)) / kBucket);
+        while (todo != 0ull) {
+            const int sb = (63 - __builtin_clzll(todo)) / kBucket;
+            uint32_t bits = (uint32_t)(todo >> (sb * kBucket));
+            const int hits = __builtin_popcount(bits);
+            todo &= (1ull << (sb * kBucket)) - 1ull;
+            const uint32_t j0 = (uint32_t)bstart + (uint32_t)(sb * kBucket);
+            float tt = j0 < pix.last ? next_t : 0.0f;
+            if (todo != 0ull) next_t = checkpoint((63 - __builtin_clzll(todo)) / kBucket);
+            // forward replay of the bucket from its checkpoint (render.c:1476-1515), two entries' G at a time
+            int k[kBucket];
+            float tb[kBucket], gv[kBucket];
+            uint64_t taken[kBucket];  // the pixels that take the entry
+            auto replay = [&](int q, bool ok, float gq, float alpha) {
+                ok = ok & ((uint32_t)bstart + (uint32_t)k[q] < pix.last);
+                tb[q] = tt;
+                taken[q] = wave_ballot(ok);
+                gv[q] = ok ? gq : 0.0f;
+                tt = ok ? tt * (1.0f - alpha) : tt;
+            };
+#pragma unroll
+            for (int q = 0; q < kBucket; q += 2) {
+                if (q >= hits) break;  // uniform
+                k[q] = sb * kBucket + __builtin_ctz(bits);
+                bits &= bits - 1u;
+                float g0, a0, g1, a1;
+                if (q + 1 < hits) {  // uniform
+                    k[q + 1] = sb * kBucket + __builtin_ctz(bits);
+                    bits &= bits - 1u;
+                    const bool ok0 = blend_alpha<!kMoments>(sm.entry[k[q]], pix.fpx, pix.fpy, pix.pxy, sm.exp2, g0, a0);
+                    const bool ok1 = blend_alpha<!kMoments>(sm.entry[k[q + 1]], pix.fpx, pix.fpy, pix.pxy, sm.exp2, g1, a1);
+                    replay(q, ok0, g0, a0);
+                    replay(q + 1, ok1, g1, a1);
+                } else {
+                    const bool ok0 = blend_alpha<!kMoments>(sm.entry[k[q]], pix.fpx, pix.fpy, pix.pxy, sm.exp2, g0, a0);
+                    replay(q, ok0, g0, a0);
+                }
+            }
+            // back to front over the bucket (render.c:1559-1666 per contribution)
+#pragma unroll
+            for (int q = kBucket - 1; q >= 0; --q) {
+                if (q >= hits) continue;  // uniform
+                if (taken[q] == 0ull) continue;  // uniform: no pixel of this wave
+                used |= 1ull << k[q];
+                const BlendEntry& en = sm.entry[k[q]];
+                const float4 eb = en.b;
+                const float cb = en.c.x;
+                const float gval = gv[q];
+                const float raw = eb.y * gval;
+                const float alpha = fminf(kMaxFragmentAlpha, raw);
+                const float t_before = tb[q];
+                // A lane that does not contribute holds G = 0, hence alpha = 0: its weight w and its
+                // opacity term below are (signed) zeros by arithmetic, and it leaves the suffix
+                // unchanged, so no per-lane select on the contribution is needed (all values are
+                // finite). alpha <= 0.999, so 1 - alpha lies in [0.001, 1]: the CPU's |1 - alpha| > 1e-6
+                // guard always holds.
+                const float w = alpha * t_before;
+                float dalpha;
+                if constexpr (kMoments) {
+                    const float cd = __builtin_fmaf(eb.z, d0, __builtin_fmaf(eb.w, d1, cb * d2));
+                    const float om = 1.0f - alpha;
+                    const float y = __builtin_amdgcn_rcpf(om);
+                    float quot = s0 * y;
+                    quot = __builtin_fmaf(__builtin_fmaf(-om, quot, s0), y, quot);
+                    dalpha = __builtin_fmaf(t_before, cd, -quot);
+                    s0 = __builtin_fmaf(w, cd, s0);
+                } else {
+                    // a correctly rounded division as the CPU's: near-plane Gaussians' covariance
+                    // gradients amplify even 1-ulp differences of this term (no scaling steps are
+                    // needed, and a zero numerator gives a zero quotient)
+                    dalpha = t_before * (eb.z * d0 + eb.w * d1 + cb * d2);
+                    dalpha -= div_rn_normal(s0 * d0 + s1 * d1 + s2 * d2, 1.0f - alpha);
+                    s0 += w * eb.z;
+                    s1 += w * eb.w;
+                    s2 += w * cb;
+                }
+                dalpha = raw < kMaxFragmentAlpha ? dalpha : 0.0f;
+                const float h = dalpha * gval;
+                if constexpr (kMoments) {
+                    const uint32_t at = (uint32_t)fill * (2u * kWave * 4u) + ((4u * lane) ^ ((uint32_t)fill * 32u));
+                    char* const xb = reinterpret_cast<char*>(x);
+                    *reinterpret_cast<float*>(xb + at) = h;
+                    *reinterpret_cast<float*>(xb + ((at ^ 16u) + kWave * 4u)) = w;
+                    ++rows;
+                    if (++fill == kMomentEntries) flush();
+                } else {
+                    const float4 ea = en.a;
+                    const float4 k0 = sm.k[0][k[q]];
+                    const float4 k1 = sm.k[1][k[q]];  // k1.z = 2 k0.y, k1.w = 2 k1.x
+                    const float dx = pix.fpx - ea.x;
+                    const float dy = pix.fpy - ea.y;
+                    const float dpow = dalpha * eb.y * gval;
+                    const float inv_a = -2.0f * ea.z, inv_b = -ea.w, inv_c = -2.0f * eb.x;
+                    const float dia = dpow * (-0.5f * dx * dx);
+                    const float dib = dpow * (-dx * dy);
+                    const float dic = dpow * (-0.5f * dy * dy);
+                    // the mean2d terms may fuse; the covariance terms keep the CPU's rounding
+                    const float v[kGrad2d] = {dpow * __builtin_fmaf(inv_a, dx, inv_b * dy),
+                                              dpow * __builtin_fmaf(inv_b, dx, inv_c * dy),
+                                              dia * k0.x + dib * k0.y + dic * k0.z,
+                                              dia * k1.z + dib * k0.w + dic * k1.w,
+                                              dia * k0.z + dib * k1.x + dic * k1.y,
+                                              w * d0,
+                                              w * d1,
+                                              w * d2,
+                                              h};
+                    float total8;
+                    const float total = wave_sum9(v, total8);
+                    float* const to = &sm.sum[wave][rows * kGrad2d];
+                    if ((lane & 7u) == 0u) to[wave_sum9_index(lane)] = total;
+                    if (lane == 63u) to[8] = total8;
+                    ++rows;
+                }
+            }
+        }
+        if (kMoments && fill > 0) flush();
+        if (lane == 0u) sm.used[wave] = used;
+        __syncthreads();
+        // four threads per entry add the waves' rows and write the partial
+        if ((int)e < count) {
+            const uint64_t mask = sm.used[p];
+            const bool hit = ((mask >> e) & 1ull) != 0ull;
+            const float* const from = &sm.sum[p][(hit ? __popcll((mask >> e) >> 1) : 0) * kGrad2d];
+            float v[kGrad2d];
+#pragma unroll
+            for (int c = 0; c < kGrad2d; ++c) {
+                const float f = from[c];
+                v[c] = hit ? f : 0.0f;
+            }
+            const BlendEntry en = sm.entry[e];
+            if constexpr (kMoments) {
+                // moments about the quadrant's centre -> about the mean: the offset is u + ex, v + ey
+                const float ex = (float)(tx * kTile + 8 * (int)(p & 1u) + 4) - en.a.x;
+                const float ey = (float)(ty * kTile + 8 * (int)(p >> 1) + 4) - en.a.y;
+                const float sx = __builtin_fmaf(ex, v[0], v[1]), sy = __builtin_fmaf(ey, v[0], v[2]);
+                v[3] = __builtin_fmaf(ex, v[1] + sx, v[3]);
+                v[4] = __builtin_fmaf(ex, v[2], __builtin_fmaf(ey, sx, v[4]));
+                v[5] = __builtin_fmaf(ey, v[2] + sy, v[5]);
+                v[1] = sx;
+                v[2] = sy;
+            }
+#pragma unroll
+            for (int c = 0; c < kGrad2d; ++c) v[c] = quad_sum(v[c]);
+            if constexpr (kMoments) {
+                const float4 k0 = cov_coef[2 * (size_t)g_combine];
+                const float4 k1 = cov_coef[2 * (size_t)g_combine + 1];  // k1.z = 2 k0.y, k1.w = 2 k1.x
+                const float op = en.b.y, inv_a = -2.0f * en.a.z, inv_b = -en.a.w, inv_c = -2.0f * en.b.x;
+                const float dia = -0.5f * (op * v[3]), dib = -(op * v[4]), dic = -0.5f * (op * v[5]);
+                const float h = v[0];
+                v[0] = op * __builtin_fmaf(inv_a, v[1], inv_b * v[2]);
+                v[1] = op * __builtin_fmaf(inv_b, v[1], inv_c * v[2]);
+                v[2] = dia * k0.x + dib * k0.y + dic * k0.z;
+                v[3] = dia * k1.z + dib * k0.w + dic * k1.w;
+                v[4] = dia * k0.z + dib * k1.x + dic * k1.y;
+                v[5] = v[6];
+                v[6] = v[7];
+                v[7] = v[8];
+                v[8] = h;
+            }
+            const size_t pos = __float_as_uint(en.c.w);
+            float4* const dst = reinterpret_cast<float4*>(instance_grad) + 2 * pos;
+            if (p == 0) dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+            if (p == 1) dst[1] = make_float4(v[4], v[5], v[6], v[7]);
+            if (p == 2) instance_grad_op[pos] = v[8];
+        }
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kBlendThreads, 5) void blend_backward_kernel(
     const uint2* __restrict__ ranges, const uint32_t* __restrict__ values, const uint32_t* __restrict__ sorted_g,
     const float4* __restrict__ rec, const float4* __restrict__ col, const uint2* __restrict__ cbox,
-    const float4* __restrict__ cov_coef, const float* __restrict__ ckpt,
+    const float4* __restrict__ cov_coef, const float* __restrict__ ckpt, const uint32_t* __restrict__ tile_exact,
     CameraParams cam, const float* __restrict__ grad_rgb, const float* __restrict__ final_t,
     const uint32_t* __restrict__ last_contrib, float* __restrict__ instance_grad,
     float* __restrict__ instance_grad_op, uint32_t* __restrict__ tile_cut, uint8_t* __restrict__ touched,
     SinkZeroing sinks) {
-    __shared__ float4 s_r0[kBackBatch];
-    __shared__ float4 s_r1[kBackBatch];
-    __shared__ float4 s_r2[kBackBatch];
-    __shared__ float4 s_k0[kBackBatch];
-    __shared__ float4 s_k1[kBackBatch];
-    __shared__ uint32_t s_pos[kBackBatch];
-    __shared__ float s_ck[kBatchBuckets][kBlendThreads];
-    __shared__ float s_acc[kRowsPerTile][kBucket][kGrad2d];
-    __shared__ uint64_t s_exp2[GSX_EXPF_BLEND_TABLE_SIZE];
-    __shared__ uint32_t s_max_last;
+    __shared__ BackwardShared sm;
     // every workgroup, the padding ones included, zeroes its slice of the gradient sinks first
     zero_sink_slice(sinks, blockIdx.x);
     const int tiles = cam.tiles_x * cam.tiles_y;
     const int tile = xcd_tile_index(blockIdx.x, tiles);
     if (tile >= tiles) return;
-    if (threadIdx.x < GSX_EXPF_BLEND_TABLE_SIZE) s_exp2[threadIdx.x] = gsx_expf_blend_entry(threadIdx.x);
+    if (threadIdx.x < GSX_EXPF_BLEND_TABLE_SIZE) sm.exp2[threadIdx.x] = gsx_expf_blend_entry(threadIdx.x);
     const int tx = tile % cam.tiles_x, ty = tile / cam.tiles_x;
     const int2 tp = tile_pixel_of_thread((int)threadIdx.x);
     const int px = tx * kTile + tp.x;
     const int py = ty * kTile + tp.y;
-    const int row = threadIdx.x / kTile;  // DPP row of the workgroup (16 lanes)
-    const bool inside = px < cam.width && py < cam.height;
     const uint2 range = ranges[tile];
-    const size_t pix = (size_t)py * (size_t)cam.width + (size_t)px;
-    const size_t plane = (size_t)cam.width * (size_t)cam.height;
-    const float fpx = (float)px + 0.5f;
-    const float fpy = (float)py + 0.5f;
-    const uint32_t pxy = (uint32_t)px | ((uint32_t)py << 16);  // for in_box_packed
-    float t_final = 0.0f, d0 = 0.0f, d1 = 0.0f, d2 = 0.0f;
-    uint32_t last = range.x;
-    if (inside) {
-        t_final = final_t[pix];
-        last = last_contrib[pix];
-        d0 = grad_rgb[pix];
-        d1 = grad_rgb[plane + pix];
-        d2 = grad_rgb[2 * plane + pix];
+    const uint32_t exact = tile_exact[tile];
+    BackwardPixel pix;
+    pix.fpx = (float)px + 0.5f;
+    pix.fpy = (float)py + 0.5f;
+    pix.pxy = (uint32_t)px | ((uint32_t)py << 16);  // for in_box_packed
+    pix.last = range.x;
+    pix.t_final = pix.d0 = pix.d1 = pix.d2 = 0.0f;
+    if (px < cam.width && py < cam.height) {
+        const size_t at = (size_t)py * (size_t)cam.width + (size_t)px;
+        const size_t plane = (size_t)cam.width * (size_t)cam.height;
+        pix.t_final = final_t[at];
+        pix.last = last_contrib[at];
+        pix.d0 = grad_rgb[at];
+        pix.d1 = grad_rgb[plane + at];
+        pix.d2 = grad_rgb[2 * plane + at];
     }
-    // render.c:1552-1557: the suffix starts as T_final * background
-    float s0 = t_final * cam.bg[0], s1 = t_final * cam.bg[1], s2 = t_final * cam.bg[2];
-    if (threadIdx.x == 0) s_max_last = range.x;
+    if (threadIdx.x == 0) sm.max_last = range.x;
+    const uint32_t wave_last = wave_max_u32(pix.last);
     __syncthreads();
-    atomicMax(&s_max_last, last);
+    if (__lane_id() == 0) atomicMax(&sm.max_last, wave_last);
     __syncthreads();
-    const uint32_t end_all = s_max_last;
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wave = threadIdx.x / kWave;
+    const uint32_t end_all = sm.max_last;
     // Entries from zero_from on (whole buckets past the last entry any pixel of the tile reaches)
     // get no partial: their gradient is zero. Positions ascend along the tile's run, so the run's
     // entries with a partial are exactly those whose position is below tile_cut[tile], the
@@ -955,177 +1350,13 @@ __global__ __launch_bounds__(kBlendThreads) void blend_backward_kernel(
         end_all <= range.x ? range.x : range.x + ((end_all - range.x + kBucket - 1) / kBucket) * kBucket;
     if (threadIdx.x == 0) tile_cut[tile] = zero_from < range.y ? values[zero_from] : UINT32_MAX;
     if (end_all <= range.x) return;  // uniform
-
-    // Batches of kBackBatch entries are walked back to front; records and the batch's bucket
-    // checkpoints reach LDS at the start of each batch.
-    const uint32_t first_batch = range.x + ((end_all - 1u - range.x) / kBackBatch) * kBackBatch;
-    for (int64_t bstart = first_batch; bstart >= (int64_t)range.x; bstart -= kBackBatch) {
-        const int count = (int)min((uint32_t)kBackBatch, range.y - (uint32_t)bstart);
-        // the batch's checkpoints load together, ahead of the records (not under branches: a
-        // pixel that needs no checkpoint of a bucket reads the batch's first slot, which exists,
-        // and keeps 0)
-        float ck[kBatchBuckets];
-#pragma unroll
-        for (int b = 0; b < kBatchBuckets; ++b) {
-            const uint32_t j0 = (uint32_t)bstart + (uint32_t)(b * kBucket);
-            const uint32_t js = (inside && j0 < last) ? j0 : (uint32_t)bstart;
-            ck[b] = ckpt[checkpoint_slot(range.x, tile, js) * kBlendThreads + threadIdx.x];
-        }
-        if (threadIdx.x < count) {
-            const uint32_t j = (uint32_t)bstart + threadIdx.x;
-            s_pos[threadIdx.x] = values[j];
-            // sorted_g is written by the TRAIN forward for every batch it loaded, and every entry
-            // below end_all lies in such a batch; entries from end_all on contribute nothing
-            if (j < end_all) {
-                const uint32_t g = sorted_g[j];
-                touched[g] = 1;
-                const float4 geo1 = rec[2 * (size_t)g + 1], c = col[g];
-                const uint2 box = cbox[g];
-                s_r0[threadIdx.x] = rec[2 * (size_t)g + 0];
-                s_r1[threadIdx.x] = make_float4(geo1.x, geo1.y, c.x, c.y);
-                s_r2[threadIdx.x] = make_float4(c.z, __uint_as_float(box.x), __uint_as_float(box.y), c.w);
-                s_k0[threadIdx.x] = cov_coef[2 * (size_t)g + 0];
-                s_k1[threadIdx.x] = cov_coef[2 * (size_t)g + 1];
-            } else {
-                const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                s_r0[threadIdx.x] = z;
-                s_r1[threadIdx.x] = z;
-                s_r2[threadIdx.x] = make_float4(0.0f, __uint_as_float(kEmptyBoxLo), 0.0f, 0.0f);  // no pixel
-                s_k0[threadIdx.x] = z;
-                s_k1[threadIdx.x] = z;
-            }
-        }
-#pragma unroll
-        for (int b = 0; b < kBatchBuckets; ++b) {
-            const uint32_t j0 = (uint32_t)bstart + (uint32_t)(b * kBucket);
-            s_ck[b][threadIdx.x] = (inside && j0 < last) ? ck[b] : 0.0f;
-        }
-        __syncthreads();
-        const int sb_first = (count - 1) / kBucket;
-        for (int sb = sb_first; sb >= 0; --sb) {
-            const uint32_t j0 = (uint32_t)bstart + (uint32_t)(sb * kBucket);
-            if (j0 < end_all) {  // uniform; buckets from end_all on get no partial (tile_cut)
-            const int n_in = min(kBucket, count - sb * kBucket);
-            float tb[kBucket];
-            float gv[kBucket];
-            // forward replay of the bucket from its checkpoint (render.c:1476-1515)
-            {
-                float tt = s_ck[sb][threadIdx.x];
-                const bool pixel_live = inside && j0 < last;
-                const uint64_t pixel_mask = wave_ballot(pixel_live);
-#pragma unroll
-                for (int i = 0; i < kBucket; ++i) {
-                    tb[i] = tt;
-                    gv[i] = 0.0f;
-                    if (i >= n_in) continue;  // uniform
-                    const int kk = sb * kBucket + i;
-                    const float4 r2 = s_r2[kk];
-                    const bool ib = in_box_packed(pxy, __float_as_uint(r2.y), __float_as_uint(r2.z));
-                    const bool before_last = j0 + (uint32_t)i < last;
-                    const bool live = pixel_live & before_last & ib;
-                    if (mask_none(pixel_mask & wave_ballot(before_last) & wave_ballot(ib))) continue;
-                    const float4 r0 = s_r0[kk];
-                    const float4 r1 = s_r1[kk];
-                    const float dx = fpx - r0.x;
-                    const float dy = fpy - r0.y;
-                    float power = -0.5f * (r0.z * dx * dx + r0.w * dx * dy + r1.x * dy * dy);
-                    power = power > 0.0f ? 0.0f : power;
-                    bool ok = live & (power >= kPowerThreshold);
-                    const float gval = gsx_expf_blend(fmaxf(power, kPowerThreshold), s_exp2);
-                    const float alpha = fminf(kMaxFragmentAlpha, r1.y * gval);
-                    ok = ok & (alpha >= kMinAlpha);
-                    gv[i] = ok ? gval : 0.0f;
-                    tt = ok ? tt * (1.0f - alpha) : tt;
-                }
-            }
-            // back to front over the bucket (render.c:1559-1666 per contribution)
-#pragma unroll
-            for (int i = kBucket - 1; i >= 0; --i) {
-                if (i >= n_in) continue;  // uniform
-                const int kk = sb * kBucket + i;
-                // a contribution has G = exp(power) >= exp(-4.5) > 0 and the others keep G = 0
-                if (mask_none(wave_ballot(gv[i] != 0.0f))) {  // uniform: no pixel of this wave
-                    if (lane < 4 * kGrad2d) s_acc[wave * 4 + lane / kGrad2d][i][lane % kGrad2d] = 0.0f;
-                    continue;
-                }
-                const float4 r0 = s_r0[kk];
-                const float4 r1 = s_r1[kk];
-                const float4 r2 = s_r2[kk];
-                const float dx = fpx - r0.x;
-                const float dy = fpy - r0.y;
-                const float gval = gv[i];
-                const float op = r1.y;
-                const float alpha = fminf(kMaxFragmentAlpha, op * gval);
-                const float t_before = tb[i];
-                // A lane that does not contribute holds G = 0, hence alpha = 0: its weight w, dpow
-                // and opacity term below are (signed) zeros by arithmetic, and it leaves the suffix
-                // unchanged, so no per-lane select on the contribution is needed (all values are
-                // finite).
-                const float w = alpha * t_before;
-                float dalpha = t_before * (r1.z * d0 + r1.w * d1 + r2.x * d2);
-                // a correctly rounded division as the CPU's: near-plane Gaussians' covariance
-                // gradients amplify even 1-ulp differences of this term. alpha <= 0.999, so
-                // 1 - alpha lies in [0.001, 1]: the CPU's |1 - alpha| > 1e-6 guard always holds,
-                // the scaling steps of the general division are not needed, and a zero numerator
-                // gives a zero quotient.
-                const float num = s0 * d0 + s1 * d1 + s2 * d2;
-                dalpha -= div_rn_normal(num, 1.0f - alpha);
-                const bool unclamped = op * gval < kMaxFragmentAlpha;
-                const float dg = unclamped ? dalpha * op : 0.0f;
-                const float g_op = unclamped ? dalpha * gval : 0.0f;
-                const float dpow = dg * gval;
-                const float inv_a = r0.z, inv_b = r0.w * 0.5f, inv_c = r1.x;
-                const float dia = dpow * (-0.5f * dx * dx);
-                const float dib = dpow * (-dx * dy);
-                const float dic = dpow * (-0.5f * dy * dy);
-                const float4 k0 = s_k0[kk];
-                const float4 k1 = s_k1[kk];  // k1.z = 2 k0.y, k1.w = 2 k1.x
-                // the mean2d terms may fuse; the covariance terms keep the CPU's rounding, since
-                // near-plane Gaussians' covariance maps are close to singular
-                float v[kGrad2d] = {dpow * __builtin_fmaf(inv_a, dx, inv_b * dy),
-                                    dpow * __builtin_fmaf(inv_b, dx, inv_c * dy),
-                                    dia * k0.x + dib * k0.y + dic * k0.z,
-                                    dia * k1.z + dib * k0.w + dic * k1.w,
-                                    dia * k0.z + dib * k1.x + dic * k1.y,
-                                    w * d0,
-                                    w * d1,
-                                    w * d2,
-                                    g_op};
-                s0 += w * r1.z;
-                s1 += w * r1.w;
-                s2 += w * r2.x;
-                float total8;
-                float scattered = row_reduce_scatter9(v, total8);
-                // both totals are complete before the stores below: otherwise the compiler sinks the
-                // last DPP adds into the masked store blocks, where they cannot fuse
-                asm volatile("" : "+v"(scattered), "+v"(total8));
-                const uint32_t col = threadIdx.x & (kTile - 1);  // lane within the DPP row
-                if ((col & 1u) == 0u) s_acc[row][i][col >> 1] = scattered;
-                if (col == 0u) s_acc[row][i][8] = total8;
-            }
-            __syncthreads();
-            // combine the 16 row partials and write the bucket's per-instance partials
-            for (int o = threadIdx.x; o < n_in * kGrad2d; o += kBlendThreads) {
-                const int e = o / kGrad2d, c = o % kGrad2d;
-                float q[kRowsPerTile];
-#pragma unroll
-                for (int r = 0; r < kRowsPerTile; ++r) q[r] = s_acc[r][e][c];
-#pragma unroll
-                for (int h = kRowsPerTile / 2; h > 0; h >>= 1) {
-#pragma unroll
-                    for (int r = 0; r < h; ++r) q[r] += q[r + h];
-                }
-                const size_t pos = s_pos[sb * kBucket + e];
-                if (c < kGradRecord) {
-                    instance_grad[pos * kGradRecord + c] = q[0];
-                } else {
-                    instance_grad_op[pos] = q[0];
-                }
-            }
-            __syncthreads();
-            }
-        }
-    }
+    const uint32_t part_end = min(zero_from, range.y);  // entries below it get a partial
+    if (__builtin_amdgcn_readfirstlane((int)exact) != 0)
+        blend_backward_walk<false>(sm, pix, range, tile, tx, ty, wave_last, end_all, part_end, values, sorted_g, rec, col,
+                                   cbox, cov_coef, ckpt, cam, instance_grad, instance_grad_op, touched);
+    else
+        blend_backward_walk<true>(sm, pix, range, tile, tx, ty, wave_last, end_all, part_end, values, sorted_g, rec, col,
+                                  cbox, cov_coef, ckpt, cam, instance_grad, instance_grad_op, touched);
 }
 
 // grad2d[g] = sum of the partials over the emission positions [offset[r], offset[r+1]) of g, r its
