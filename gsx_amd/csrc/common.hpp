@@ -610,7 +610,9 @@ gsx_hip_status tile_sort_u32(const uint32_t* tiles, uint32_t* tiles_alt, uint32_
 size_t tile_sort_u32_temp_bytes(int64_t n);
 
 // Exclusive scan of partials[0..count) in place, the total stored at [count], by one workgroup;
-// with arrays > 1, the arrays of count + 1 entries that follow it too (one workgroup each).
-gsx_hip_status scan_partials_in_place(uint32_t* partials, int64_t count, hipStream_t stream, int arrays = 1);
+// with arrays > 1, the arrays of count + 1 entries that follow it too (one workgroup each). totals (may
+// be null; device-visible host memory will do) also receives the arrays' totals.
+gsx_hip_status scan_partials_in_place(uint32_t* partials, int64_t count, hipStream_t stream, int arrays = 1,
+                                      uint32_t* totals = nullptr);
 
 }  // namespace gsx_amd

@@ -54,7 +54,9 @@ __global__ __launch_bounds__(kScanThreads) void scan_reduce_kernel(const uint32_
 // next step's values are loaded before the current step's are written.
 constexpr int kPartialItems = 16;
 // Workgroup b scans the b-th of gridDim.x arrays of count + 1 entries laid out back to back.
-__global__ __launch_bounds__(kScanThreads) void scan_partials_kernel(uint32_t* __restrict__ partials, int64_t count) {
+// totals (may be null): the b-th total, also written there.
+__global__ __launch_bounds__(kScanThreads) void scan_partials_kernel(uint32_t* __restrict__ partials, int64_t count,
+                                                                     uint32_t* __restrict__ totals) {
     constexpr int kWaves = kScanThreads / kWave;
     constexpr int64_t kStep = (int64_t)kScanThreads * kPartialItems;
     __shared__ uint32_t s_wave[kWaves];
@@ -100,7 +102,10 @@ __global__ __launch_bounds__(kScanThreads) void scan_partials_kernel(uint32_t* _
         }
         carry += total;
     }
-    if (threadIdx.x == 0) partials[count] = carry;
+    if (threadIdx.x == 0) {
+        partials[count] = carry;
+        if (totals != nullptr) totals[blockIdx.x] = carry;
+    }
 }
 
 __global__ __launch_bounds__(kScanThreads) void scan_downsweep_kernel(const uint32_t* __restrict__ in, int64_t n,
@@ -567,7 +572,7 @@ gsx_hip_status scan_exclusive_u32(const uint32_t* in, uint32_t* out, int64_t n, 
     int64_t blocks = (n + kScanChunk - 1) / kScanChunk;
     if (blocks < 1) blocks = 1;
     hipLaunchKernelGGL(scan_reduce_kernel, dim3((unsigned)blocks), dim3(kScanThreads), 0, stream, in, n, partials);
-    hipLaunchKernelGGL(scan_partials_kernel, dim3(1), dim3(kScanThreads), 0, stream, partials, blocks);
+    hipLaunchKernelGGL(scan_partials_kernel, dim3(1), dim3(kScanThreads), 0, stream, partials, blocks, nullptr);
     hipLaunchKernelGGL(scan_downsweep_kernel, dim3((unsigned)blocks), dim3(kScanThreads), 0, stream, in, n, partials,
                        out);
     return (gsx_hip_status)hipGetLastError();
@@ -627,8 +632,10 @@ gsx_hip_status gsx_hip_radix_sort_keys_u64(uint64_t* keys, uint64_t* keys_alt, i
 
 namespace gsx_amd {
 
-gsx_hip_status scan_partials_in_place(uint32_t* partials, int64_t count, hipStream_t stream, int arrays) {
-    hipLaunchKernelGGL(scan_partials_kernel, dim3((unsigned)arrays), dim3(kScanThreads), 0, stream, partials, count);
+gsx_hip_status scan_partials_in_place(uint32_t* partials, int64_t count, hipStream_t stream, int arrays,
+                                      uint32_t* totals) {
+    hipLaunchKernelGGL(scan_partials_kernel, dim3((unsigned)arrays), dim3(kScanThreads), 0, stream, partials, count,
+                       totals);
     return (gsx_hip_status)hipGetLastError();
 }
 

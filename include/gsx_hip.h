@@ -437,8 +437,8 @@ gsx_hip_status gsx_hip_adc_context_destroy(gsx_hip_adc_context* context);
  * `capacity` >= count + (max_num_gaussians - count) rows; when rows are pruned the compacted set
  * is written to `out` (same fields bound) and *out_result_in_out = 1, otherwise the result stays
  * in `rows`. The final count is stored in the result's `count`. out_counts[4] = pruned,
- * duplicated, grown (split), reset, as gsx_adc_result. Synchronises the stream twice per refine
- * (candidate and survivor counts).
+ * duplicated, grown (split), reset, as gsx_adc_result. The host waits once per refine, for the
+ * counts (the compaction may still be running when the call returns, ordered on the stream).
  * MCMC (algorithm 2, gsx/src/gsx-cpu/adc/mcmc.c:345-766, dispatched as gsx-cpu/adc.c:515-547):
  * every step before end_refine moves each mean3d by opacity-gated noise shaped by its covariance
  * (6 draws per Gaussian); a refine relocates the rows whose sigmoid(opacity) <= the pruning
@@ -447,8 +447,8 @@ gsx_hip_status gsx_hip_adc_context_destroy(gsx_hip_adc_context* context);
  * place: `capacity` >= that count), with the opacity / scale correction of the relocated sources.
  * Rows are never removed, so the result stays in `rows`; out_counts = relocated (as pruned), 0,
  * relocated + appended (as grown), reset. The draw weights form their cumulative sums in float
- * on the host, in index order, as the CPU and Metal backends do (a sequential float sum has no
- * parallel equivalent with the same rounding); the stream synchronises twice per draw. */
+ * in index order, with every rounding of the CPU and Metal backends' sequential sum, on the device;
+ * the host waits once per refine, for the number of dead rows. */
 gsx_hip_status gsx_hip_adc_step(gsx_hip_adc_context* context, const gsx_hip_adc_params* params, uint64_t global_step,
                                 gsx_hip_gs_rows* rows, int64_t capacity, gsx_hip_gs_rows* out,
                                 int32_t* out_result_in_out, int64_t* out_counts, hipStream_t stream);
