@@ -190,6 +190,11 @@ struct PinnedBuffer {
 // Instance counts from which the tile ranges come from a binary search per tile rather than a
 // pass over the sorted tiles (the search's cost does not grow with the count)
 constexpr int64_t kRangesSearchMin = (int64_t)1 << 25;
+// Images of up to this many tiles keep the tile index of an instance in 16 bits: 30 instead of 48
+// bytes per instance through emission, the two sort passes and the ranges (335M instances of a 1080p
+// image: emission 877 -> 726 us, a sort pass's counts 284 -> 188 and moves 1195 -> 1049, a training step
+// 6.42 -> 5.85 ms; 5M instances: 284 -> 269 us a frame).
+constexpr int32_t kNarrowTiles = 65536;
 // Workgroups of the long-run reduction (4 waves each, each wave 64 list entries at a time): for
 // chunk 0, which every long run has, and per later chunk.
 constexpr unsigned kLongRunBlocks0 = 1024;
@@ -263,6 +268,7 @@ int bits_for(uint32_t v) {
 
 struct gsx_hip_render_context {
     DeviceBuffer rec, cov_coef, ckpt, inst_gauss, inst_tile, tiles_alt, tiles_sorted, vals_alt, vals, tile_cut, tile_exact, touched,
+        tiles_wide,
         inst_grad, tile_count, big_list, offsets, scan_temp, sort_temp, ranges, sorted_g, final_t, last, grad2d,
         depth_keys, depth_keys_alt, rank_g, rank_count, g_rank, long_list, multi_list, counters,
         depth_sort_temp;
@@ -302,6 +308,10 @@ struct gsx_hip_render_context {
     int32_t sort_passes = 0;
     int32_t depth_sort_passes = 0;
     int32_t tile_bits = 0;            // bits of the tile index the sort orders
+    // Tile indices of instances are kept in 16 bits up to kNarrowTiles tiles, else in 32; get_buffers
+    // hands out 32-bit ones (widened into tiles_wide on demand, once per forward)
+    bool narrow_tiles = false;
+    int64_t unwidened = 0;  // 16-bit indices the last completed forward sorted and nobody asked for yet
     uint32_t* sorted_vals = nullptr;  // emission position of each sorted instance
     bool has_train_state = false;
     // Stage timing: a ring of event sets, one set per forward/backward pair, so that a timed
@@ -389,6 +399,50 @@ unsigned state_blocks(int64_t n) {
     // enough workgroups per array to fill the GPU, capped for small sets
     const int64_t b = (n * 3 + 1023) / 1024;
     return (unsigned)std::min<int64_t>(std::max<int64_t>(b, 1), 1024);
+}
+
+// Emission of the counted instances, their stable sort by tile and the tiles' ranges.
+template <typename TileT>
+gsx_hip_status enqueue_tile_lists(gsx_hip_render_context* ctx, const uint32_t* big_count, uint32_t big_blocks,
+                                  unsigned emit_blocks, unsigned pre_blocks, hipStream_t stream) {
+    const int64_t n = ctx->gaussian_count, count = ctx->instance_count;
+    const int32_t tiles = ctx->tile_count_total;
+    if (n > 0) {
+        hipLaunchKernelGGL(emit_kernel<TileT>, dim3(big_blocks + emit_blocks), dim3(256), 0, stream, n,
+                           ctx->rec.as<float4>(), ctx->rank_g.as<uint32_t>(), ctx->rank_count.as<uint32_t>(),
+                           ctx->scan_temp.as<uint32_t>(), ctx->offsets.as<uint32_t>(), ctx->cam.tiles_x,
+                           ctx->big_list.as<uint32_t>(), big_count, big_blocks, ctx->g_rank.as<uint32_t>(),
+                           ctx->inst_gauss.as<uint32_t>(), ctx->inst_tile.as<TileT>(),
+                           ctx->scan_temp.as<uint32_t>() + pre_blocks + 1, ctx->long_list.as<uint32_t>());
+        GSX_HIP_TRY(hipGetLastError(), "emit_kernel");
+    }
+    GSX_TRY(record(ctx, 3, stream));
+    // tile bits in ceil(bits / 8) passes (at least one) of equal digits of 6 to 8 bits (1080p:
+    // 13 bits, 2 x 7)
+    ctx->tile_bits = bits_for((uint32_t)(tiles > 0 ? tiles - 1 : 0));
+    ctx->sort_passes = std::max(1, (ctx->tile_bits + 7) / 8);
+    const int digit_bits = std::max(6, (ctx->tile_bits + ctx->sort_passes - 1) / ctx->sort_passes);
+    GSX_TRY(tile_sort<TileT>(ctx->inst_tile.as<TileT>(), ctx->tiles_alt.as<TileT>(), ctx->tiles_sorted.as<TileT>(),
+                             ctx->vals_alt.as<uint32_t>(), ctx->vals.as<uint32_t>(), count, ctx->tile_bits,
+                             ctx->sort_passes, digit_bits, ctx->sort_temp.ptr, stream));
+    ctx->sorted_vals = ctx->vals.as<uint32_t>();
+    GSX_TRY(record(ctx, 4, stream));
+    if (count >= kRangesSearchMin) {
+        int steps = 0;
+        while (((uint64_t)1 << steps) <= (uint64_t)count) ++steps;  // ceil(log2(count + 1))
+        hipLaunchKernelGGL(tile_ranges_search_kernel<TileT>, dim3(blocks_for(tiles, 256)), dim3(256), 0, stream,
+                           ctx->tiles_sorted.as<TileT>(), (uint32_t)count, (uint32_t)tiles, steps,
+                           ctx->ranges.as<uint2>());
+    } else if (count > 0) {
+        hipLaunchKernelGGL(tile_ranges_kernel<TileT>, dim3(blocks_for((count + 3) / 4, 256)), dim3(256), 0, stream,
+                           ctx->tiles_sorted.as<TileT>(), ctx->offsets.as<uint32_t>() + n, (uint32_t)tiles,
+                           ctx->ranges.as<uint2>());
+    } else {
+        hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for((int64_t)tiles * 2, 256)), dim3(256), 0, stream,
+                           ctx->ranges.as<uint32_t>(), (int64_t)tiles * 2, 0u);
+    }
+    GSX_HIP_TRY(hipGetLastError(), "tile_ranges_kernel");
+    return GSX_HIP_SUCCESS;
 }
 
 gsx_hip_status validate_gaussians(const gsx_hip_gaussians* g) {
@@ -587,7 +641,7 @@ gsx_hip_status gsx_hip_render_context_create(gsx_hip_render_context** out_contex
 gsx_hip_status gsx_hip_render_context_destroy(gsx_hip_render_context* ctx) {
     if (ctx == nullptr) return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "context must be non-null");
     DeviceBuffer* all[] = {&ctx->rec,       &ctx->cov_coef, &ctx->ckpt,      &ctx->inst_gauss, &ctx->inst_tile,
-                           &ctx->tiles_alt, &ctx->tiles_sorted, &ctx->vals_alt, &ctx->vals,
+                           &ctx->tiles_alt, &ctx->tiles_sorted, &ctx->vals_alt, &ctx->vals, &ctx->tiles_wide,
                            &ctx->tile_cut,  &ctx->tile_exact, &ctx->touched,  &ctx->inst_grad,
                            &ctx->tile_count, &ctx->big_list, &ctx->offsets,   &ctx->scan_temp,
                            &ctx->sort_temp,  &ctx->ranges,
@@ -704,7 +758,6 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     const int64_t n = gaussians->count;
     const int32_t tiles = cam.tiles_x * cam.tiles_y;
     const int64_t pixels = (int64_t)cam.width * cam.height;
-    const int tile_bits = bits_for((uint32_t)(tiles > 0 ? tiles - 1 : 0));
     ctx->cam = cam;
     ctx->gs = *gaussians;  // replaced by the snapshot below for a TRAIN forward
     ctx->gaussian_count = n;
@@ -839,58 +892,28 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     const size_t c1 = (size_t)(count > 0 ? count : 1);
     // per instance: its tile (emission order, the sort's input, kept for the backward), the middle
     // pass's tiles and positions, the sorted tiles and positions, its Gaussian
-    GSX_TRY(ctx->inst_tile.reserve(c1 * sizeof(uint32_t), "instance_tile", ctx->call_stream));
-    GSX_TRY(ctx->tiles_alt.reserve(c1 * sizeof(uint32_t), "tiles_alt", ctx->call_stream));
-    GSX_TRY(ctx->tiles_sorted.reserve(c1 * sizeof(uint32_t), "tiles_sorted", ctx->call_stream));
+    ctx->narrow_tiles = tiles <= kNarrowTiles;
+    ctx->unwidened = 0;
+    const size_t tile_bytes = ctx->narrow_tiles ? sizeof(uint16_t) : sizeof(uint32_t);
+    GSX_TRY(ctx->inst_tile.reserve(c1 * tile_bytes, "instance_tile", ctx->call_stream));
+    GSX_TRY(ctx->tiles_alt.reserve(c1 * tile_bytes, "tiles_alt", ctx->call_stream));
+    GSX_TRY(ctx->tiles_sorted.reserve(c1 * tile_bytes, "tiles_sorted", ctx->call_stream));
     GSX_TRY(ctx->vals_alt.reserve(c1 * sizeof(uint32_t), "vals_alt", ctx->call_stream));
     GSX_TRY(ctx->vals.reserve(c1 * sizeof(uint32_t), "vals", ctx->call_stream));
     GSX_TRY(ctx->inst_gauss.reserve(c1 * sizeof(uint32_t), "instance_gaussian", ctx->call_stream));
     GSX_TRY(ctx->sorted_g.reserve(c1 * sizeof(uint32_t), "sorted_g", ctx->call_stream));
-    GSX_TRY(ctx->sort_temp.reserve(tile_sort_u32_temp_bytes(count), "sort_temp", ctx->call_stream));
+    GSX_TRY(ctx->sort_temp.reserve(tile_sort_temp_bytes(count), "sort_temp", ctx->call_stream));
     if (train) {
         // bucket checkpoints: at most I/kBucket + tiles + 1 slots of 256 floats
         GSX_TRY(ctx->ckpt.reserve(((size_t)count / kBucket + (size_t)tiles + 2) * 256 * sizeof(float),
                                   "checkpoints", ctx->call_stream));
     }
-    if (n > 0) {
-        // one wave per big box; rank workgroups up to one rank past the visible ones
-        const uint32_t big_blocks = (uint32_t)((big_total + kWavesPerBlock - 1) / kWavesPerBlock);
-        const unsigned emit_blocks = std::min(pre_blocks, (unsigned)(visible_total / 256u + 1u));
-        hipLaunchKernelGGL(emit_kernel, dim3(big_blocks + emit_blocks), dim3(256), 0, stream, n, ctx->rec.as<float4>(),
-                           ctx->rank_g.as<uint32_t>(), ctx->rank_count.as<uint32_t>(), ctx->scan_temp.as<uint32_t>(),
-                           ctx->offsets.as<uint32_t>(), cam.tiles_x, ctx->big_list.as<uint32_t>(), big_count,
-                           big_blocks, ctx->g_rank.as<uint32_t>(), ctx->inst_gauss.as<uint32_t>(), ctx->inst_tile.as<uint32_t>(),
-                           ctx->scan_temp.as<uint32_t>() + pre_blocks + 1, ctx->long_list.as<uint32_t>());
-        GSX_HIP_TRY(hipGetLastError(), "emit_kernel");
-    }
-    GSX_TRY(record(ctx, 3, stream));
-    // tile bits in ceil(bits / 8) passes (at least one) of equal digits of 6 to 8 bits (1080p:
-    // 13 bits, 2 x 7)
-    ctx->sort_passes = std::max(1, (tile_bits + 7) / 8);
-    ctx->tile_bits = tile_bits;
-    {
-        const int digit_bits = std::max(6, (tile_bits + ctx->sort_passes - 1) / ctx->sort_passes);
-        GSX_TRY(tile_sort_u32(ctx->inst_tile.as<uint32_t>(), ctx->tiles_alt.as<uint32_t>(),
-                              ctx->tiles_sorted.as<uint32_t>(), ctx->vals_alt.as<uint32_t>(), ctx->vals.as<uint32_t>(),
-                              count, tile_bits, ctx->sort_passes, digit_bits, ctx->sort_temp.ptr, stream));
-        ctx->sorted_vals = ctx->vals.as<uint32_t>();
-    }
-    GSX_TRY(record(ctx, 4, stream));
-    if (count >= kRangesSearchMin) {
-        int steps = 0;
-        while (((uint64_t)1 << steps) <= (uint64_t)count) ++steps;  // ceil(log2(count + 1))
-        hipLaunchKernelGGL(tile_ranges_search_kernel, dim3(blocks_for(tiles, 256)), dim3(256), 0, stream,
-                           ctx->tiles_sorted.as<uint32_t>(), (uint32_t)count, (uint32_t)tiles, steps,
-                           ctx->ranges.as<uint2>());
-    } else if (count > 0) {
-        hipLaunchKernelGGL(tile_ranges_kernel, dim3(blocks_for((count + 3) / 4, 256)), dim3(256), 0, stream,
-                           ctx->tiles_sorted.as<uint32_t>(), ctx->offsets.as<uint32_t>() + n, (uint32_t)tiles,
-                           ctx->ranges.as<uint2>());
-    } else {
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks_for((int64_t)tiles * 2, 256)), dim3(256), 0, stream,
-                           ctx->ranges.as<uint32_t>(), (int64_t)tiles * 2, 0u);
-    }
-    GSX_HIP_TRY(hipGetLastError(), "tile_ranges_kernel");
+    // one wave per big box; rank workgroups up to one rank past the visible ones
+    const uint32_t big_blocks = (uint32_t)((big_total + kWavesPerBlock - 1) / kWavesPerBlock);
+    const unsigned emit_blocks = std::min(pre_blocks, (unsigned)(visible_total / 256u + 1u));
+    GSX_TRY(ctx->narrow_tiles ? enqueue_tile_lists<uint16_t>(ctx, big_count, big_blocks, emit_blocks, pre_blocks, stream)
+                              : enqueue_tile_lists<uint32_t>(ctx, big_count, big_blocks, emit_blocks, pre_blocks, stream));
+    if (ctx->narrow_tiles) ctx->unwidened = count;
     GSX_TRY(record(ctx, 5, stream));
     const int tiles_padded = ((tiles + 7) / 8) * 8;
     hipLaunchKernelGGL(train ? blend_forward_kernel<true> : blend_forward_kernel<false>, dim3((unsigned)tiles_padded),
@@ -957,13 +980,16 @@ gsx_hip_status enqueue_backward(gsx_hip_render_context* ctx, const float* grad_r
     GSX_HIP_TRY(hipGetLastError(), "blend_backward_kernel");
     GSX_TRY(record(ctx, 8, stream));
     if (n > 0) {
-        hipLaunchKernelGGL(reduce_instance_grads_kernel,
-                           dim3(kLongRunBlocks0 + kLongRunBlocks * (kLongChunks - 1) + blocks_for(n, 256)),
-                           dim3(256), 0, stream, n, counters, ctx->offsets.as<uint32_t>(), ctx->rank_g.as<uint32_t>(),
-                           ctx->long_list.as<uint32_t>(), ctx->scan_temp.as<uint32_t>() + 2 * (size_t)pre_blocks + 1,
-                           ctx->multi_list.as<uint32_t>(), counters + 4, kLongRunBlocks0, kLongRunBlocks, long_chunk,
-                           ctx->inst_grad.as<float>(), inst_grad_op, ctx->inst_tile.as<uint32_t>(),
-                           ctx->tile_cut.as<uint32_t>(), ctx->touched.as<uint8_t>(), ctx->grad2d.as<float>());
+        const auto launch_reduce = [&](auto kernel, const auto* instance_tile) {
+            hipLaunchKernelGGL(kernel, dim3(kLongRunBlocks0 + kLongRunBlocks * (kLongChunks - 1) + blocks_for(n, 256)),
+                               dim3(256), 0, stream, n, counters, ctx->offsets.as<uint32_t>(), ctx->rank_g.as<uint32_t>(),
+                               ctx->long_list.as<uint32_t>(), ctx->scan_temp.as<uint32_t>() + 2 * (size_t)pre_blocks + 1,
+                               ctx->multi_list.as<uint32_t>(), counters + 4, kLongRunBlocks0, kLongRunBlocks, long_chunk,
+                               ctx->inst_grad.as<float>(), inst_grad_op, instance_tile, ctx->tile_cut.as<uint32_t>(),
+                               ctx->touched.as<uint8_t>(), ctx->grad2d.as<float>());
+        };
+        if (ctx->narrow_tiles) launch_reduce(reduce_instance_grads_kernel<uint16_t>, ctx->inst_tile.as<uint16_t>());
+        else launch_reduce(reduce_instance_grads_kernel<uint32_t>, ctx->inst_tile.as<uint32_t>());
         GSX_HIP_TRY(hipGetLastError(), "reduce_instance_grads_kernel");
     }
     GSX_TRY(record(ctx, 9, stream));
@@ -1088,9 +1114,22 @@ gsx_hip_status gsx_hip_render_context_get_stats(const gsx_hip_render_context* ct
     return GSX_HIP_SUCCESS;
 }
 
-gsx_hip_status gsx_hip_render_context_get_buffers(const gsx_hip_render_context* ctx, gsx_hip_render_buffers* out) {
-    if (ctx == nullptr || out == nullptr) return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "context/out must be non-null");
-    out->sorted_tiles = ctx->tiles_sorted.as<uint32_t>();
+gsx_hip_status gsx_hip_render_context_get_buffers(const gsx_hip_render_context* context, gsx_hip_render_buffers* out) {
+    if (context == nullptr || out == nullptr) return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "context/out must be non-null");
+    gsx_hip_render_context* ctx = const_cast<gsx_hip_render_context*>(context);  // only its widened copy changes
+    if (ctx->unwidened > 0) {
+        // behind everything queued (whichever stream the forward took, also one that is gone by now), on the
+        // context's own stream, and waited for: the pointer is good for any stream
+        const int64_t count = ctx->unwidened;
+        GSX_HIP_TRY(hipDeviceSynchronize(), "widen tiles sync");
+        GSX_TRY(ctx->tiles_wide.reserve((size_t)count * sizeof(uint32_t), "wide tiles", ctx->check_stream));
+        hipLaunchKernelGGL(widen_tiles_kernel, dim3(std::min(blocks_for(count, 1024), 65536u)), dim3(256), 0,
+                           ctx->check_stream, ctx->tiles_sorted.as<uint16_t>(), count, ctx->tiles_wide.as<uint32_t>());
+        GSX_HIP_TRY(hipGetLastError(), "widen_tiles_kernel");
+        GSX_HIP_TRY(hipStreamSynchronize(ctx->check_stream), "widen tiles sync");
+        ctx->unwidened = 0;
+    }
+    out->sorted_tiles = ctx->narrow_tiles ? ctx->tiles_wide.as<uint32_t>() : ctx->tiles_sorted.as<uint32_t>();
     out->sorted_values = ctx->sorted_vals;
     out->tile_ranges = ctx->ranges.as<uint32_t>();
     out->records = ctx->rec.as<float>();

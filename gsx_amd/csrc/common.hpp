@@ -565,15 +565,33 @@ __device__ inline void radix_upsweep_block(uint32_t blk, const KeyT* __restrict_
         // every key of the chunk is loaded before the first count waits on one (no load sits
         // under a branch: lanes past n re-read key n - 1 and count nothing)
         constexpr int kRounds = kChunk / kSortThreads;
-        KeyT k[kRounds];
-#pragma unroll
-        for (int r = 0; r < kRounds; ++r) k[r] = keys[min(base + (int64_t)r * kSortThreads + threadIdx.x, n - 1)];
+        constexpr int kPerLoad = 16 / (int)sizeof(KeyT);
         uint32_t* my_hist = s_hist + (wave * kCopies + (int)(__lane_id() / (kWave / kCopies))) * kCopyWords;
+        if (sizeof(KeyT) == 2 && base + kChunk <= n) {  // uniform
+            // counts do not depend on the order within a chunk: a whole chunk of 16-bit keys is loaded 8
+            // to a lane (chunks start 16-byte aligned), not 128 bytes to a wave
+            struct alignas(16) Keys {
+                KeyT k[kPerLoad];
+            };
+            const Keys* const src = reinterpret_cast<const Keys*>(keys + base);
+            constexpr int kLoads = kRounds / kPerLoad;
+            Keys v[kLoads > 0 ? kLoads : 1];
 #pragma unroll
-        for (int r = 0; r < kRounds; ++r) {
-            const int64_t i = base + (int64_t)r * kSortThreads + threadIdx.x;
-            if (i < n && (!drop_sentinel || (uint64_t)k[r] != kSentinelKey))
-                atomicAdd(&my_hist[digit_of<kBits>(k[r], shift) & dmask], 1u);
+            for (int r = 0; r < kLoads; ++r) v[r] = src[r * kSortThreads + threadIdx.x];
+#pragma unroll
+            for (int r = 0; r < kLoads; ++r)
+#pragma unroll
+                for (int q = 0; q < kPerLoad; ++q) atomicAdd(&my_hist[digit_of<kBits>(v[r].k[q], shift) & dmask], 1u);
+        } else {
+            KeyT k[kRounds];
+#pragma unroll
+            for (int r = 0; r < kRounds; ++r) k[r] = keys[min(base + (int64_t)r * kSortThreads + threadIdx.x, n - 1)];
+#pragma unroll
+            for (int r = 0; r < kRounds; ++r) {
+                const int64_t i = base + (int64_t)r * kSortThreads + threadIdx.x;
+                if (i < n && (!drop_sentinel || (uint64_t)k[r] != kSentinelKey))
+                    atomicAdd(&my_hist[digit_of<kBits>(k[r], shift) & dmask], 1u);
+            }
         }
     }
     __syncthreads();
@@ -603,11 +621,13 @@ size_t radix_sort_keys_u64_compacting_temp_bytes(int64_t n);
 // ceil(b / 8) passes of ceil(b / passes) bits, fewer ballots and bins than 8-bit digits (13-bit
 // tiles: 2 passes of 7). The first pass reads `tiles` (left unchanged) and no values; the result
 // lands in tiles_sorted / vals_sorted (the alternates hold a middle pass). temp holds
-// tile_sort_u32_temp_bytes(n) bytes (the 8-bit need, the largest).
-gsx_hip_status tile_sort_u32(const uint32_t* tiles, uint32_t* tiles_alt, uint32_t* tiles_sorted, uint32_t* vals_alt,
+// tile_sort_temp_bytes(n) bytes (the 8-bit need, the largest).
+// TileT: uint16_t (at most 16 tile bits) or uint32_t.
+template <typename TileT>
+gsx_hip_status tile_sort(const TileT* tiles, TileT* tiles_alt, TileT* tiles_sorted, uint32_t* vals_alt,
                              uint32_t* vals_sorted, int64_t n, int tile_bits, int passes, int digit_bits, void* temp,
                              hipStream_t stream);
-size_t tile_sort_u32_temp_bytes(int64_t n);
+size_t tile_sort_temp_bytes(int64_t n);
 
 // Exclusive scan of partials[0..count) in place, the total stored at [count], by one workgroup;
 // with arrays > 1, the arrays of count + 1 entries that follow it too (one workgroup each). totals (may

@@ -52,8 +52,8 @@ constexpr int kKeptPartVisibleShift = 52;
 // | index (visible depths lie in [near, far], where positive floats order like their bit
 // patterns, so the offset keeps the order in fewer bits; invisible Gaussians get the offset
 // bits(far) - bits(near) + 1 and sort last). Instances are then emitted in that depth order,
-// instance_tile[position] = tile, and the tile indices are sorted stably (u32 keys, the emission
-// positions as values, implicit in the first pass): each tile's run is in (depth, index) order,
+// instance_tile[position] = tile, and the tile indices are sorted stably (16-bit keys up to 65536 tiles,
+// else 32-bit, the emission positions as values, implicit in the first pass): each tile's run is in (depth, index) order,
 // the CPU backend's order, after two passes at 1080p.
 
 __device__ inline uint32_t box_tiles(float4 geo1) {
@@ -154,9 +154,9 @@ __device__ inline uint32_t stage_spans(WaveSpans& w, bool valid, float4 r0, floa
 // Walks the wave's flattened rows. kEmit = false adds each row's kept tiles to kept[owner];
 // kEmit = true writes the kept instances (instance_tile, instance_gaussian) of every row, the
 // rows of a box in order, at base[owner] + the instances of the walked rows before it.
-template <bool kEmit>
+template <bool kEmit, typename TileT>
 __device__ inline void walk_wave_rows(WaveSpans& w, uint32_t wave_rows, int32_t tiles_x,
-                                      uint32_t* __restrict__ instance_gaussian, uint32_t* __restrict__ instance_tile) {
+                                      uint32_t* __restrict__ instance_gaussian, TileT* __restrict__ instance_tile) {
     const uint32_t lane = __lane_id();
     // the owner of item p is the last box starting at or before p, i.e. the last non-empty one
     // (an empty box shares its start with the next box): each non-empty box whose rows start in
@@ -212,7 +212,7 @@ __device__ inline void walk_wave_rows(WaveSpans& w, uint32_t wave_rows, int32_t 
                 if (q < total2) {
                     const uint32_t pos = w.run_pos[run] + q;
                     instance_gaussian[pos] = w.run_g[run];
-                    instance_tile[pos] = w.run_tile[run] + q;
+                    instance_tile[pos] = (TileT)(w.run_tile[run] + q);
                 }
             }
             walked += total2;
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(
     const uint32_t big_slot = wave_append_slot(big_count, big);
     if (big) big_list[big_slot] = (uint32_t)g;
     const uint32_t rows = stage_spans(ws, visible, r0, r1);
-    walk_wave_rows<false>(ws, rows, cam.tiles_x, nullptr, nullptr);
+    walk_wave_rows<false, uint32_t>(ws, rows, cam.tiles_x, nullptr, nullptr);
     const uint32_t kept = ws.kept[__lane_id()];
     if (g < n) tile_count[g] = kept;
     // depth key of every Gaussian (~0 for invisible ones, which the depth sort drops);
@@ -456,11 +456,12 @@ __global__ __launch_bounds__(256) void rank_gather_kernel(int64_t n, const uint3
 // blocking) scans its own 256 counts; offsets[0..n] are stored for the later kernels
 // (offsets[n] = total).
 // ---------------------------------------------------------------------------------------------
+template <typename TileT>
 __device__ inline void emit_block(uint32_t b, int64_t n, int64_t rank_end, const float4* __restrict__ rec,
                                   const uint32_t* __restrict__ rank_gaussian, const uint32_t* __restrict__ rank_count,
                                   const uint32_t* __restrict__ block_prefix, uint32_t* __restrict__ offsets,
                                   int32_t tiles_x, uint32_t* __restrict__ instance_gaussian,
-                                  uint32_t* __restrict__ instance_tile,
+                                  TileT* __restrict__ instance_tile,
                                   const uint32_t* __restrict__ long_prefix, uint32_t* __restrict__ long_list,
                                   WaveSpans* s_spans, uint32_t* s_wave) {
     WaveSpans& ws = s_spans[threadIdx.x / kWave];
@@ -503,18 +504,19 @@ __device__ inline void emit_block(uint32_t b, int64_t n, int64_t rank_end, const
     ws.base[lane] = o - (wave_inclusive_sum_u32(wcnt) - wcnt);
     ws.g[lane] = g;
     const uint32_t rows = stage_spans(ws, walked, r0, r1);
-    walk_wave_rows<true>(ws, rows, tiles_x, instance_gaussian, instance_tile);
+    walk_wave_rows<true, TileT>(ws, rows, tiles_x, instance_gaussian, instance_tile);
 }
 
 // Big boxes: one wave per box of big_list, walking its rows as walk_wave_rows walks a wave's
 // boxes (the box in lane 0, the others empty). It runs beside emit_block in one launch, so it
 // forms the box's offset itself: block_prefix of the rank's 256-rank block plus the counts of the
 // ranks before it in that block. The host sizes the launch with one wave per big box.
+template <typename TileT>
 __device__ inline void big_box_wave(uint32_t i, const uint32_t* __restrict__ big_list, const float4* __restrict__ rec,
                                     int32_t tiles_x, const uint32_t* __restrict__ rank_count,
                                     const uint32_t* __restrict__ block_prefix,
                                     const uint32_t* __restrict__ gaussian_rank,
-                                    uint32_t* __restrict__ instance_gaussian, uint32_t* __restrict__ instance_tile,
+                                    uint32_t* __restrict__ instance_gaussian, TileT* __restrict__ instance_tile,
                                     WaveSpans& ws) {
     const uint32_t lane = __lane_id();
     const uint32_t g = big_list[i];
@@ -527,11 +529,12 @@ __device__ inline void big_box_wave(uint32_t i, const uint32_t* __restrict__ big
     ws.base[lane] = block_prefix[rr >> 8] + wave_reduce_sum_u32(v);
     ws.g[lane] = g;
     const uint32_t rows = stage_spans(ws, lane == 0, r0, r1);
-    walk_wave_rows<true>(ws, rows, tiles_x, instance_gaussian, instance_tile);
+    walk_wave_rows<true, TileT>(ws, rows, tiles_x, instance_gaussian, instance_tile);
 }
 
 // All emission in one launch: workgroups [0, big_blocks) hold one wave per big box, first so
 // that their longer walks start early; the rest are the emission workgroups of the ranks.
+template <typename TileT>
 __global__ __launch_bounds__(256) void emit_kernel(int64_t n, const float4* __restrict__ rec,
                                                    const uint32_t* __restrict__ rank_gaussian,
                                                    const uint32_t* __restrict__ rank_count,
@@ -541,7 +544,7 @@ __global__ __launch_bounds__(256) void emit_kernel(int64_t n, const float4* __re
                                                    const uint32_t* __restrict__ big_count, uint32_t big_blocks,
                                                    const uint32_t* __restrict__ gaussian_rank,
                                                    uint32_t* __restrict__ instance_gaussian,
-                                                   uint32_t* __restrict__ instance_tile,
+                                                   TileT* __restrict__ instance_tile,
                                                    const uint32_t* __restrict__ long_prefix,
                                                    uint32_t* __restrict__ long_list) {
     __shared__ WaveSpans s_spans[kWavesPerBlock];
@@ -571,12 +574,20 @@ __global__ __launch_bounds__(256) void fill_f32_kernel(float* __restrict__ p, in
     if (i < count) p[i] = v;
 }
 
+// The sorted tiles as 32-bit numbers, for a caller that looks at the retained intermediates.
+__global__ __launch_bounds__(256) void widen_tiles_kernel(const uint16_t* __restrict__ in, int64_t count,
+                                                          uint32_t* __restrict__ out) {
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
+        out[i] = in[i];
+}
+
 // [start, end) of each tile's run in the sorted tile indices. Tiles without instances get
 // (0, 0): the thread of the last instance before such a gap (or of the first instance, for the
 // tiles before it) writes them, so no fill of all tiles is needed beforehand. count >= 1 (with
 // no instances the caller fills the ranges). Each thread takes 4 consecutive sorted tiles (one
-// 16-byte load), plus the tiles just before and after them for the boundaries.
-__global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t* __restrict__ sorted_tiles,
+// 8- or 16-byte load), plus the tiles just before and after them for the boundaries.
+template <typename TileT>
+__global__ __launch_bounds__(256) void tile_ranges_kernel(const TileT* __restrict__ sorted_tiles,
                                                           const uint32_t* count_ptr, uint32_t tiles,
                                                           uint2* __restrict__ ranges) {
     const uint32_t count = *count_ptr;
@@ -588,11 +599,12 @@ __global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t* __rest
     const uint32_t t_next = sorted_tiles[min(i0 + m, count - 1u)];
     uint32_t t[4];
     if (m == 4) {
-        const uint4 q = *reinterpret_cast<const uint4*>(sorted_tiles + i0);
-        t[0] = q.x;
-        t[1] = q.y;
-        t[2] = q.z;
-        t[3] = q.w;
+        struct alignas(4 * sizeof(TileT)) Four {
+            TileT t[4];
+        };
+        const Four q = *reinterpret_cast<const Four*>(sorted_tiles + i0);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) t[j] = q.t[j];
     } else {
 #pragma unroll
         for (uint32_t j = 0; j < 4; ++j) t[j] = j < m ? sorted_tiles[i0 + j] : 0u;
@@ -620,7 +632,8 @@ __global__ __launch_bounds__(256) void tile_ranges_kernel(const uint32_t* __rest
 // tile and of the next in the sorted tiles by binary search, the two searches in lockstep
 // (ceil(log2(count + 1)) steps of two loads each, the same for every lane) instead of a pass over
 // every instance. Tiles without instances get (0, 0).
-__global__ __launch_bounds__(256) void tile_ranges_search_kernel(const uint32_t* __restrict__ sorted_tiles,
+template <typename TileT>
+__global__ __launch_bounds__(256) void tile_ranges_search_kernel(const TileT* __restrict__ sorted_tiles,
                                                                  uint32_t count, uint32_t tiles, int steps,
                                                                  uint2* __restrict__ ranges) {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1405,8 +1418,9 @@ struct InstancePartial {
     float4 a, b;
     float op;
 };
+template <typename TileT>
 __device__ inline InstancePartial load_partial(const float4* __restrict__ rec4, const float* __restrict__ instance_grad_op,
-                                               const uint32_t* __restrict__ instance_tile,
+                                               const TileT* __restrict__ instance_tile,
                                                const uint32_t* __restrict__ tile_cut, uint32_t p) {
     InstancePartial v;
     const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
@@ -1425,9 +1439,10 @@ __device__ inline InstancePartial load_partial(const float4* __restrict__ rec4, 
 // Chunk k of the long run [b, e) of Gaussian g, summed by the whole wave (b, e, g, k wave-uniform).
 // A run of one chunk gets its sums in grad2d, a longer one its chunk's sums at the chunk's first
 // position.
+template <typename TileT>
 __device__ inline void reduce_run_chunk(uint32_t b, uint32_t e, uint32_t g, uint32_t k, uint32_t chunk,
                                         float* __restrict__ instance_grad, float* __restrict__ instance_grad_op,
-                                        const uint32_t* __restrict__ instance_tile,
+                                        const TileT* __restrict__ instance_tile,
                                         const uint32_t* __restrict__ tile_cut, float* __restrict__ grad2d) {
     const uint32_t lane = __lane_id();
     const float4* rec4 = reinterpret_cast<const float4*>(instance_grad);
@@ -1473,10 +1488,11 @@ __device__ inline void reduce_run_chunk(uint32_t b, uint32_t e, uint32_t g, uint
 // Chunk k of the long runs of the wave's lanes (run [b, e) of Gaussian g where `live`): the
 // touched ones are summed by the wave one after another (the untouched ones have no sums: the
 // projection backward skips their Gaussians).
+template <typename TileT>
 __device__ inline void reduce_wave_long_runs(bool live, uint32_t b, uint32_t e, uint32_t g, uint32_t k,
                                              uint32_t chunk, float* __restrict__ instance_grad,
                                              float* __restrict__ instance_grad_op,
-                                             const uint32_t* __restrict__ instance_tile,
+                                             const TileT* __restrict__ instance_tile,
                                              const uint32_t* __restrict__ tile_cut,
                                              const uint8_t* __restrict__ touched, float* __restrict__ grad2d) {
     const bool hit = live && touched[g] != 0;
@@ -1489,11 +1505,12 @@ __device__ inline void reduce_wave_long_runs(bool live, uint32_t b, uint32_t e, 
     }
 }
 
+template <typename TileT>
 __device__ inline void reduce_short_block(uint32_t blk, int64_t n, const uint32_t* __restrict__ depth_count,
                                           const uint32_t* __restrict__ offsets,
                                           const uint32_t* __restrict__ rank_gaussian, uint32_t chunk,
                                           float* __restrict__ instance_grad, float* __restrict__ instance_grad_op,
-                                          const uint32_t* __restrict__ instance_tile,
+                                          const TileT* __restrict__ instance_tile,
                                           const uint32_t* __restrict__ tile_cut, const uint8_t* __restrict__ touched,
                                           float* __restrict__ grad2d, float4 (*s_rec)[2 * kShortPiece],
                                           float (*s_op)[kShortPiece]) {
@@ -1557,12 +1574,13 @@ __device__ inline void reduce_short_block(uint32_t blk, int64_t n, const uint32_
 // Chunk k of the runs on `list`, by the gx * 4 waves of the workgroups of column k: lane l of
 // wave w takes entries w + W (l + 64 j), j = 0, 1, ... (W waves), so neighbouring entries go to
 // different waves.
+template <typename TileT>
 __device__ inline void reduce_long_block(uint32_t x, uint32_t k, uint32_t gx, const uint32_t* __restrict__ list,
                                          const uint32_t* __restrict__ list_count,
                                          const uint32_t* __restrict__ offsets,
                                          const uint32_t* __restrict__ rank_gaussian, uint32_t chunk,
                                          float* __restrict__ instance_grad, float* __restrict__ instance_grad_op,
-                                         const uint32_t* __restrict__ instance_tile,
+                                         const TileT* __restrict__ instance_tile,
                                          const uint32_t* __restrict__ tile_cut, const uint8_t* __restrict__ touched,
                                          float* __restrict__ grad2d) {
     const uint32_t count = *list_count;
@@ -1587,13 +1605,14 @@ __device__ inline void reduce_long_block(uint32_t x, uint32_t k, uint32_t gx, co
 // Both reductions in one launch: workgroups [0, gx0) take chunk 0 of the long runs, the next
 // gx * (kLongChunks - 1) chunks 1.. of the runs longer than one chunk (x = index % gx, chunk
 // k = 1 + index / gx), the rest the short runs of the ranks (256 each).
+template <typename TileT>
 __global__ __launch_bounds__(256) void reduce_instance_grads_kernel(
     int64_t n, const uint32_t* __restrict__ depth_count, const uint32_t* __restrict__ offsets,
     const uint32_t* __restrict__ rank_gaussian, const uint32_t* __restrict__ long_list,
     const uint32_t* __restrict__ long_count, const uint32_t* __restrict__ multi_list,
     const uint32_t* __restrict__ multi_count, uint32_t gx0, uint32_t gx, uint32_t chunk,
     float* __restrict__ instance_grad,
-    float* __restrict__ instance_grad_op, const uint32_t* __restrict__ instance_tile,
+    float* __restrict__ instance_grad_op, const TileT* __restrict__ instance_tile,
     const uint32_t* __restrict__ tile_cut, const uint8_t* __restrict__ touched, float* __restrict__ grad2d) {
     __shared__ float4 s_rec[kWavesPerBlock][2 * kShortPiece];
     __shared__ float s_op[kWavesPerBlock][kShortPiece];

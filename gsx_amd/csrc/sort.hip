@@ -22,7 +22,7 @@ constexpr int kScanChunk = kScanThreads * kScanItems;  // 1024 elements per bloc
 
 constexpr int kSortChunk = 4096;  // keys per chunk (one upsweep / downsweep workgroup), public sorts
 constexpr int kRadixBits = 8;     // digit width of the public sorts
-// Chunks of the tile sort's passes (tile_sort_u32): 4096 keys below kLargeTileSort keys, 8192
+// Chunks of the tile sort's passes (tile_sort): 4096 keys below kLargeTileSort keys, 8192
 // from there on (runs of a digit twice as long per workgroup: each workgroup's writes meet half as
 // many distinct places of the output per byte, and the histograms and row scans halve; below it
 // the larger chunk leaves too few workgroups to fill the GPU). The downsweep runs chunk / 8
@@ -265,9 +265,9 @@ __device__ inline uint32_t digit_exclusive_scan(uint32_t v, uint32_t* s_wave, ui
     return wave_base + incl - v;
 }
 
-// KeyT: uint64_t or uint32_t keys. kPairs with vals_in == nullptr: each key's value is its input
+// KeyT: uint64_t, uint32_t or uint16_t keys. kPairs with vals_in == nullptr: each key's value is its input
 // position (the first pass of the tile sort, whose values are the emission positions). kNarrow:
-// n * sizeof(KeyT) <= 2^32, so every output byte offset fits in 32 bits. kThreads: workgroup size
+// n * max(sizeof(KeyT), 4) <= 2^32, so every output byte offset fits in 32 bits. kThreads: workgroup size
 // (kChunk / kThreads keys per thread). Register target: 8 waves per SIMD, except for 64-bit keys
 // with values, whose 54 KB of LDS admits two workgroups (4 waves per SIMD) per CU anyway.
 template <bool kPairs, int kBits, int kChunk, typename KeyT = uint64_t, bool kNarrow = false,
@@ -281,9 +281,9 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     constexpr int kDownWaveKeys = kChunk / kWaves;  // keys ranked by one wave
     constexpr int kDownRounds = kDownWaveKeys / kWave;
     static_assert(kDownRounds >= 1 && kDownWaveKeys % kWave == 0, "whole rounds per wave");
-    // the reordered chunk: 32-bit keys with values as one 64-bit entry per key (one scatter
+    // the reordered chunk: 16- and 32-bit keys with values as one 64-bit entry per key (one scatter
     // store instead of two), otherwise keys (and values) in arrays of their own
-    constexpr bool kPack = kPairs && sizeof(KeyT) == 4;
+    constexpr bool kPack = kPairs && sizeof(KeyT) <= 4;
     __shared__ uint64_t s_kv[kPack ? kChunk : 1];
     __shared__ KeyT s_keys[kPack ? 1 : kChunk];
     __shared__ uint32_t s_vals[(kPairs && !kPack) ? kChunk : 1];
@@ -425,7 +425,7 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
         const int i = (int)threadIdx.x + j * kThreads;
         if (kPack) {
             const uint64_t kv = s_kv[i];
-            ok[j] = (KeyT)(uint32_t)kv;
+            ok[j] = (KeyT)kv;
             ov[j] = (uint32_t)(kv >> 32);
         } else {
             ok[j] = s_keys[i];
@@ -648,8 +648,8 @@ gsx_hip_status radix_sort_keys_u64_compacting(uint64_t* keys, uint64_t* keys_alt
                                                                          stream);
 }
 
-template <int kBits, int kChunk>
-gsx_hip_status tile_sort_passes(const uint32_t* tiles, uint32_t* tiles_alt, uint32_t* tiles_sorted, uint32_t* vals_alt,
+template <int kBits, int kChunk, typename TileT>
+gsx_hip_status tile_sort_passes(const TileT* tiles, TileT* tiles_alt, TileT* tiles_sorted, uint32_t* vals_alt,
                                 uint32_t* vals_sorted, int64_t n, int tile_bits, int passes, void* temp,
                                 hipStream_t stream) {
     constexpr int kBins = 1 << kBits;
@@ -659,25 +659,25 @@ gsx_hip_status tile_sort_passes(const uint32_t* tiles, uint32_t* tiles_alt, uint
     uint32_t* hist = static_cast<uint32_t*>(temp);
     uint32_t* offsets = hist + hist_count;
     uint32_t* totals = offsets + hist_count;
-    const uint32_t* kin = tiles;
+    const TileT* kin = tiles;
     const uint32_t* vin = nullptr;  // first pass: the values are the input positions
     for (int k = 0; k < passes; ++k) {
         // the last pass lands in the sorted arrays, the one before it in the alternates, ...
         const bool to_sorted = (passes - 1 - k) % 2 == 0;
-        uint32_t* kout = to_sorted ? tiles_sorted : tiles_alt;
+        TileT* kout = to_sorted ? tiles_sorted : tiles_alt;
         uint32_t* vout = to_sorted ? vals_sorted : vals_alt;
         const int shift = k * kBits;
         const int width = tile_bits - shift < kBits ? tile_bits - shift : kBits;
         const uint32_t dmask = width > 0 ? (1u << width) - 1u : 0u;
-        hipLaunchKernelGGL((radix_upsweep_kernel<kBits, kChunk, uint32_t>), dim3(sort_chunk_grid(chunks)),
+        hipLaunchKernelGGL((radix_upsweep_kernel<kBits, kChunk, TileT>), dim3(sort_chunk_grid(chunks)),
                            dim3(kSortThreads), 0, stream, kin, n, nullptr, false, shift, dmask, chunks, hist);
         launch_rowscan(kBins, hist, chunks, offsets, totals, stream);
         if (narrow_offsets(n, sizeof(uint32_t))) {
-            hipLaunchKernelGGL((radix_downsweep_kernel<true, kBits, kChunk, uint32_t, true, kChunk / 8>),
+            hipLaunchKernelGGL((radix_downsweep_kernel<true, kBits, kChunk, TileT, true, kChunk / 8>),
                                dim3(sort_chunk_grid(chunks)), dim3(kChunk / 8), 0, stream, kin, vin, n, nullptr,
                                false, shift, dmask, chunks, offsets, totals, kout, vout, nullptr);
         } else {
-            hipLaunchKernelGGL((radix_downsweep_kernel<true, kBits, kChunk, uint32_t, false, kChunk / 8>),
+            hipLaunchKernelGGL((radix_downsweep_kernel<true, kBits, kChunk, TileT, false, kChunk / 8>),
                                dim3(sort_chunk_grid(chunks)), dim3(kChunk / 8), 0, stream, kin, vin, n, nullptr,
                                false, shift, dmask, chunks, offsets, totals, kout, vout, nullptr);
         }
@@ -687,16 +687,17 @@ gsx_hip_status tile_sort_passes(const uint32_t* tiles, uint32_t* tiles_alt, uint
     return (gsx_hip_status)hipGetLastError();
 }
 
-gsx_hip_status tile_sort_u32(const uint32_t* tiles, uint32_t* tiles_alt, uint32_t* tiles_sorted, uint32_t* vals_alt,
+template <typename TileT>
+gsx_hip_status tile_sort(const TileT* tiles, TileT* tiles_alt, TileT* tiles_sorted, uint32_t* vals_alt,
                              uint32_t* vals_sorted, int64_t n, int tile_bits, int passes, int digit_bits, void* temp,
-                             hipStream_t stream) {
+                         hipStream_t stream) {
     if (n < 0 || n > (int64_t)UINT32_MAX || passes < 1 || tile_bits < 0 || tile_bits > passes * digit_bits ||
-        tiles == tiles_sorted || tiles == tiles_alt) {
+        tiles == tiles_sorted || tiles == tiles_alt || tile_bits > (int)(8 * sizeof(TileT))) {
         return GSX_HIP_ERROR_INVALID_ARGUMENT;
     }
     if (n == 0) return GSX_HIP_SUCCESS;
 #define GSX_TILE_SORT(B, C) \
-    tile_sort_passes<B, C>(tiles, tiles_alt, tiles_sorted, vals_alt, vals_sorted, n, tile_bits, passes, temp, stream)
+    tile_sort_passes<B, C, TileT>(tiles, tiles_alt, tiles_sorted, vals_alt, vals_sorted, n, tile_bits, passes, temp, stream)
     const bool large = n >= kLargeTileSort;
     switch (digit_bits) {
         case 6: return large ? GSX_TILE_SORT(6, kDigitsChunkLarge) : GSX_TILE_SORT(6, kDigitsChunk);
@@ -706,8 +707,12 @@ gsx_hip_status tile_sort_u32(const uint32_t* tiles, uint32_t* tiles_alt, uint32_
     }
 #undef GSX_TILE_SORT
 }
+template gsx_hip_status tile_sort<uint16_t>(const uint16_t*, uint16_t*, uint16_t*, uint32_t*, uint32_t*, int64_t, int,
+                                            int, int, void*, hipStream_t);
+template gsx_hip_status tile_sort<uint32_t>(const uint32_t*, uint32_t*, uint32_t*, uint32_t*, uint32_t*, int64_t, int,
+                                            int, int, void*, hipStream_t);
 
-size_t tile_sort_u32_temp_bytes(int64_t n) { return radix_temp_bytes<8, kDigitsChunk>(n); }
+size_t tile_sort_temp_bytes(int64_t n) { return radix_temp_bytes<8, kDigitsChunk>(n); }
 
 
 size_t radix_sort_keys_u64_compacting_temp_bytes(int64_t n) {
