@@ -294,11 +294,7 @@ struct gsx_hip_render_context {
     gsx_hip_gaussians live{};
     gsx_hip_camera camera{};
     int32_t train_mode = GSX_HIP_FORWARD_INFERENCE;
-    // counters: [0] visible Gaussians (depth keys), [1] unused, [2 + big_slot] big boxes
-    // of the next forward (each forward's preprocess clears the other slot for its successor),
-    // [4] runs of more than one long-run chunk
-    bool counters_ready = false;
-    int big_slot = 0;
+    // counters: [0] visible Gaussians (depth keys)
     CameraParams cam{};
     gsx_hip_gaussians gs{};
     int64_t instance_count = 0;
@@ -403,17 +399,22 @@ unsigned state_blocks(int64_t n) {
 
 // Emission of the counted instances, their stable sort by tile and the tiles' ranges.
 template <typename TileT>
-gsx_hip_status enqueue_tile_lists(gsx_hip_render_context* ctx, const uint32_t* big_count, uint32_t big_blocks,
-                                  unsigned emit_blocks, unsigned pre_blocks, hipStream_t stream) {
+gsx_hip_status enqueue_tile_lists(gsx_hip_render_context* ctx, uint32_t big_total, unsigned emit_blocks,
+                                  unsigned pre_blocks, hipStream_t stream) {
     const int64_t n = ctx->gaussian_count, count = ctx->instance_count;
     const int32_t tiles = ctx->tile_count_total;
     if (n > 0) {
+        // a wave per big box, so that a few spread over the GPU; with more boxes than fill it, several a
+        // wave, which then shares the set-up and the last, mostly empty step of 64 rows
+        // (112k boxes among 335M instances: 735 us one a wave, 695 us seven)
+        const uint32_t big_per_wave = std::min(8u, big_total / 16384u + 1u);
+        const uint32_t big_block = big_per_wave * kWavesPerBlock, big_blocks = (big_total + big_block - 1) / big_block;
         hipLaunchKernelGGL(emit_kernel<TileT>, dim3(big_blocks + emit_blocks), dim3(256), 0, stream, n,
                            ctx->rec.as<float4>(), ctx->rank_g.as<uint32_t>(), ctx->rank_count.as<uint32_t>(),
-                           ctx->scan_temp.as<uint32_t>(), ctx->offsets.as<uint32_t>(), ctx->cam.tiles_x,
-                           ctx->big_list.as<uint32_t>(), big_count, big_blocks, ctx->g_rank.as<uint32_t>(),
-                           ctx->inst_gauss.as<uint32_t>(), ctx->inst_tile.as<TileT>(),
-                           ctx->scan_temp.as<uint32_t>() + pre_blocks + 1, ctx->long_list.as<uint32_t>());
+                           ctx->scan_temp.as<uint32_t>(), (size_t)pre_blocks + 1, ctx->offsets.as<uint32_t>(),
+                           ctx->cam.tiles_x, ctx->big_list.as<uint2>(), big_blocks, big_per_wave, ctx->inst_gauss.as<uint32_t>(),
+                           ctx->inst_tile.as<TileT>(), long_chunk_of(tiles), ctx->long_list.as<uint32_t>(),
+                           ctx->multi_list.as<uint32_t>());
         GSX_HIP_TRY(hipGetLastError(), "emit_kernel");
     }
     GSX_TRY(record(ctx, 3, stream));
@@ -771,11 +772,12 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     if (train) GSX_TRY(ctx->touched.reserve(n1, "touched", ctx->call_stream));
     if (train) GSX_TRY(ctx->tile_exact.reserve((size_t)tiles * sizeof(uint32_t), "tile_exact", ctx->call_stream));
     GSX_TRY(ctx->tile_count.reserve(n1 * sizeof(uint32_t), "tile_count", ctx->call_stream));
-    GSX_TRY(ctx->counters.reserve(8 * sizeof(uint32_t), "counters", ctx->call_stream));
-    GSX_TRY(ctx->big_list.reserve(n1 * sizeof(uint32_t), "big_list", ctx->call_stream));
+    GSX_TRY(ctx->counters.reserve(sizeof(uint32_t), "counters", ctx->call_stream));
+    GSX_TRY(ctx->big_list.reserve(n1 * sizeof(uint2), "big_ranks", ctx->call_stream));
     GSX_TRY(ctx->offsets.reserve((size_t)(n + 1) * sizeof(uint32_t), "offsets", ctx->call_stream));
-    // per 256-rank workgroup: its tile-count sum, then its long-run count (two scanned arrays)
-    GSX_TRY(ctx->scan_temp.reserve(2 * ((size_t)blocks_for(n, 256) + 1) * sizeof(uint32_t), "rank_block_sums", ctx->call_stream));
+    // per 256-rank workgroup: its tile-count sum, then its counts of long runs, of big boxes and of
+    // runs of several chunks (four scanned arrays)
+    GSX_TRY(ctx->scan_temp.reserve(4 * ((size_t)blocks_for(n, 256) + 1) * sizeof(uint32_t), "rank_block_sums", ctx->call_stream));
     GSX_TRY(ctx->long_list.reserve(n1 * sizeof(uint32_t), "long_list", ctx->call_stream));
     GSX_TRY(ctx->depth_keys.reserve(n1 * sizeof(uint64_t), "depth_keys", ctx->call_stream));
     GSX_TRY(ctx->depth_keys_alt.reserve(n1 * sizeof(uint64_t), "depth_keys_alt", ctx->call_stream));
@@ -790,7 +792,6 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     uint32_t* counters = ctx->counters.as<uint32_t>();
     const unsigned pre_blocks = blocks_for(n, 256);
     GSX_TRY(ctx->kept_parts.reserve((size_t)pre_blocks * sizeof(unsigned long long), "kept_parts"));
-    uint32_t* big_count = counters + 2 + ctx->big_slot;
 
     // depth keys of the visible Gaussians: (bits(depth) - bits(near)) << index_bits | index (see
     // KeyLayout), at most 31 + 32 bits, so never the all-ones key that marks invisible ones
@@ -827,11 +828,6 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     }
     ctx->train_mode = train;
     if (n > 0) {
-        if (!ctx->counters_ready) {
-            hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, stream, counters, (int64_t)8, 0u);
-            GSX_HIP_TRY(hipGetLastError(), "fill_u32_kernel");
-            ctx->counters_ready = true;
-        }
         hipLaunchKernelGGL(preprocess_kernel, dim3(pre_blocks), dim3(256), 0, stream, snap, n, gaussians->mean3d,
                            gaussians->rotation, gaussians->logscale, gaussians->opacity, gaussians->sh0,
                            gaussians->sh1, gaussians->sh2, gaussians->sh3, (int)gaussians->sh_degree, cam,
@@ -839,14 +835,11 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
                            reinterpret_cast<uint2*>(ctx->rec.as<float4>() + 3 * n),
                            train ? ctx->cov_coef.as<float4>() : nullptr,
                            ctx->tile_count.as<uint32_t>(), train ? visible_counter : nullptr,
-                           ctx->big_list.as<uint32_t>(), big_count, counters + 1, counters + 2 + (ctx->big_slot ^ 1),
-                           counters + 4,
                            static_cast<unsigned long long*>(ctx->kept_parts.dev), ctx->depth_keys.as<uint64_t>(),
                            near_bits,
                            depth_max, index_bits, big_flag ? kBigKeyFlag : 0ull, count_shift,
                            train ? ctx->touched.as<uint8_t>() : nullptr);
         GSX_HIP_TRY(hipGetLastError(), "preprocess_kernel");
-        ctx->big_slot ^= 1;  // the slot this preprocess cleared
     }
     // the counting kernels leave the instance count as per-workgroup partials in host memory;
     // the depth order and the count scan are queued behind them, so the GPU keeps working while
@@ -864,12 +857,13 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
         hipLaunchKernelGGL(rank_gather_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, stream, n, counters,
                            sorted_depth, (uint64_t)((1ull << index_bits) - 1ull), big_flag, count_shift,
                            (uint32_t)((1ull << count_bits) - 1ull), ctx->tile_count.as<uint32_t>(),
+                           ctx->rec.as<float4>(),
                            ctx->rank_g.as<uint32_t>(), ctx->rank_count.as<uint32_t>(), ctx->g_rank.as<uint32_t>(),
                            long_chunk_of(tiles),
-                           ctx->multi_list.as<uint32_t>(), counters + 4, ctx->scan_temp.as<uint32_t>());
+                           ctx->big_list.as<uint2>(), ctx->scan_temp.as<uint32_t>());
         GSX_HIP_TRY(hipGetLastError(), "rank_gather_kernel");
         // exclusive scan of the 256-rank sums; emit_keys_kernel completes the offsets
-        GSX_TRY(scan_partials_in_place(ctx->scan_temp.as<uint32_t>(), pre_blocks, stream, 2));
+        GSX_TRY(scan_partials_in_place(ctx->scan_temp.as<uint32_t>(), pre_blocks, stream, 4));
     }
     GSX_TRY(record(ctx, 2, stream));
     GSX_HIP_TRY(hipEventSynchronize(ctx->count_ev), "instance count sync");
@@ -908,11 +902,10 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
         GSX_TRY(ctx->ckpt.reserve(((size_t)count / kBucket + (size_t)tiles + 2) * 256 * sizeof(float),
                                   "checkpoints", ctx->call_stream));
     }
-    // one wave per big box; rank workgroups up to one rank past the visible ones
-    const uint32_t big_blocks = (uint32_t)((big_total + kWavesPerBlock - 1) / kWavesPerBlock);
+    // rank workgroups up to one rank past the visible ones
     const unsigned emit_blocks = std::min(pre_blocks, (unsigned)(visible_total / 256u + 1u));
-    GSX_TRY(ctx->narrow_tiles ? enqueue_tile_lists<uint16_t>(ctx, big_count, big_blocks, emit_blocks, pre_blocks, stream)
-                              : enqueue_tile_lists<uint32_t>(ctx, big_count, big_blocks, emit_blocks, pre_blocks, stream));
+    GSX_TRY(ctx->narrow_tiles ? enqueue_tile_lists<uint16_t>(ctx, (uint32_t)big_total, emit_blocks, pre_blocks, stream)
+                              : enqueue_tile_lists<uint32_t>(ctx, (uint32_t)big_total, emit_blocks, pre_blocks, stream));
     if (ctx->narrow_tiles) ctx->unwidened = count;
     GSX_TRY(record(ctx, 5, stream));
     const int tiles_padded = ((tiles + 7) / 8) * 8;
@@ -984,7 +977,8 @@ gsx_hip_status enqueue_backward(gsx_hip_render_context* ctx, const float* grad_r
             hipLaunchKernelGGL(kernel, dim3(kLongRunBlocks0 + kLongRunBlocks * (kLongChunks - 1) + blocks_for(n, 256)),
                                dim3(256), 0, stream, n, counters, ctx->offsets.as<uint32_t>(), ctx->rank_g.as<uint32_t>(),
                                ctx->long_list.as<uint32_t>(), ctx->scan_temp.as<uint32_t>() + 2 * (size_t)pre_blocks + 1,
-                               ctx->multi_list.as<uint32_t>(), counters + 4, kLongRunBlocks0, kLongRunBlocks, long_chunk,
+                               ctx->multi_list.as<uint32_t>(),
+                               ctx->scan_temp.as<uint32_t>() + 4 * (size_t)pre_blocks + 3, kLongRunBlocks0, kLongRunBlocks, long_chunk,
                                ctx->inst_grad.as<float>(), inst_grad_op, instance_tile, ctx->tile_cut.as<uint32_t>(),
                                ctx->touched.as<uint8_t>(), ctx->grad2d.as<float>());
         };

@@ -379,19 +379,6 @@ __device__ inline uint64_t lanemask_lt() {
     return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
-// Slot of each lane with `take` in a list whose length is *count: one atomic add per wave (by
-// the lowest taking lane, a vector atomic) instead of one per lane; every lane of the wave must
-// call it. Lanes without `take` get an unspecified value.
-__device__ inline uint32_t wave_append_slot(uint32_t* count, bool take) {
-    const uint64_t mask = __ballot(take);
-    if (mask == 0ull) return 0u;
-    const uint32_t leader = (uint32_t)__builtin_ctzll(mask);
-    uint32_t base = 0u;
-    if (__lane_id() == leader) base = atomicAdd(count, (uint32_t)__popcll(mask));
-    base = (uint32_t)__builtin_amdgcn_readlane((int)base, (int)leader);
-    return base + (uint32_t)__popcll(mask & lanemask_lt());
-}
-
 // Inclusive prefix sum over the 64 lanes of a wave (DPP row shifts, then the two row broadcasts);
 // every lane must be active.
 __device__ inline uint32_t wave_inclusive_sum_u32(uint32_t v) {

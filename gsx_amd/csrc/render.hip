@@ -39,7 +39,7 @@ constexpr int kBlendThreads = kTilePixels;  // 256: one pixel per thread, 4 wave
 // the runs of a step, 64 instances per sub-step, with a second owner search over the runs.
 // ---------------------------------------------------------------------------------------------
 constexpr int kWavesPerBlock = 4;
-// Boxes of more tiles than this are emitted by a wave of their own (big_box_wave): in depth order
+// Boxes of more tiles than this are emitted by waves of their own (big_boxes_wave): in depth order
 // the near, large boxes are neighbours, and a wave holding many full-image boxes would serialise
 // their instances. Counting walks every box in the waves (rows are few).
 constexpr uint32_t kBigTiles = 1024;
@@ -78,148 +78,207 @@ constexpr uint32_t kEmptyBoxLo = 0xffffffffu;
 // corners of the 3-sigma box and, for all but the most opaque Gaussians, its rim, where every pixel
 // fails the CPU's power or alpha cut; fewer pixels, and fewer waves of a tile, meet the entry.
 // Preprocess stores it per visible Gaussian; key emission keeps using the record's box.
-__device__ inline uint2 contribution_box_packed(float4 r0, float4 r1) {
+// k receives the Gaussian's span constants (span_of's), shared with the count of its tiles.
+__device__ inline uint2 contribution_box_packed(float4 r0, float4 r1, gsx_tile_span& k) {
     const uint32_t bx = __float_as_uint(r1.z), by = __float_as_uint(r1.w);
     int xa, xb, ya, yb;
-    gsx_contribution_box(r0.x, r0.y, r0.z, r0.w * 0.5f, r1.x, r1.y, (int)(bx & 0xffffu), (int)(bx >> 16),
-                         (int)(by & 0xffffu), (int)(by >> 16), &xa, &xb, &ya, &yb);
+    gsx_contribution_box_and_span(r0.x, r0.y, r0.z, r0.w * 0.5f, r1.x, r1.y, (int)(bx & 0xffffu), (int)(bx >> 16),
+                                  (int)(by & 0xffffu), (int)(by >> 16), &k, &xa, &xb, &ya, &yb);
     if (xa > xb || ya > yb) return make_uint2(kEmptyBoxLo, 0u);
     return make_uint2((uint32_t)xa | ((uint32_t)ya << 16), (uint32_t)(xb - xa) | ((uint32_t)(yb - ya) << 16));
 }
 
 // Kept run of tile row ty of a box: len tiles from tile0 (len = 0 when none).
-__device__ inline void row_run(const gsx_tile_span& k, uint32_t bx, uint32_t by, int ty, int32_t tiles_x,
+__device__ inline void row_run(const gsx_tile_span& k, uint32_t bx, uint32_t by, uint32_t ty, int32_t tiles_x,
                                uint32_t& len, uint32_t& tile0) {
     const int x0 = (int)(bx & 0xffffu), x1 = (int)(bx >> 16), y0 = (int)(by & 0xffffu), y1 = (int)(by >> 16);
-    const int py0 = max(ty * kTile, y0), py1 = min(ty * kTile + kTile - 1, y1);
+    const int py0 = max((int)ty * kTile, y0), py1 = min((int)ty * kTile + kTile - 1, y1);
     int xa, xb;
     gsx_tile_band_columns(&k, x0, x1, py0, py1, &xa, &xb);
-    len = 0u;
-    tile0 = 0u;
-    if (xa <= xb) {
-        len = (uint32_t)(xb / kTile - xa / kTile + 1);
-        tile0 = (uint32_t)ty * (uint32_t)tiles_x + (uint32_t)(xa / kTile);
-    }
+    // (columns of a kept run lie in the box; box coordinates have 16 bits, so both factors have 12)
+    const uint32_t ta = (uint32_t)xa / kTile;
+    len = xa <= xb ? (uint32_t)xb / kTile - ta + 1u : 0u;
+    tile0 = __umul24(ty, (uint32_t)tiles_x) + ta;
 }
 
+// One wave's boxes and the walk over their rows. The boxes with rows are held in lane order without
+// gaps (slots 0, 1, ..), the non-empty runs of a step likewise.
 struct WaveSpans {
-    float mx[kWave], my[kWave], b[kWave], ra[kWave], det[kWave], vr[kWave], aqs[kWave];  // gsx_tile_span
+    float ml[kWave], mh[kWave], my[kWave], b[kWave], ra[kWave], det[kWave], vr[kWave], aqs[kWave];  // gsx_tile_span
     uint32_t bx[kWave], by[kWave];  // box: x0 | x1 << 16, y0 | y1 << 16
-    uint32_t excl[kWave];           // exclusive prefix of the lanes' row counts
-    uint32_t mark[kWave];           // walk step: base + owner at the lane where that owner's rows start
-    uint32_t kept[kWave];           // counting: kept tiles of the lane's box
-    uint32_t base[kWave], g[kWave];  // emission: position of the lane's first instance less the walked
-                                     // instances of the lanes before it; its Gaussian
-    uint32_t run_tile[kWave], run_pos[kWave], run_g[kWave], mark2[kWave];  // emission: a step's runs
+    uint32_t excl[kWave];           // rows of the boxes before it
+    uint32_t kept[kWave];           // counting: kept tiles of the box
+    uint32_t base[kWave], g[kWave];  // emission: position of the box's first instance less the walked
+                                     // instances of the boxes before it; its Gaussian
+    uint2 run[kWave];                // emission: a step's runs (first tile less the run's start, Gaussian)
+    uint32_t run_pos[kWave];         // .. their positions less their starts, where a wave's boxes are apart
+    uint64_t starts[kWave];          // item_starts
 };
 
-// Inclusive prefix maximum over the 64 lanes of a wave (DPP row shifts, then the two row
-// broadcasts), for non-negative values; every lane must be active.
-__device__ inline int wave_inclusive_max(int v) {
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true));  // row_shr:1
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true));  // row_shr:2
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true));  // row_shr:4
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true));  // row_shr:8
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));  // row_bcast:15
-    v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));  // row_bcast:31
-    return v;
-}
-
-// Stores lane's span constants and box (no rows when !valid) and returns the wave's total row
-// count.
-__device__ inline uint32_t stage_spans(WaveSpans& w, bool valid, float4 r0, float4 r1) {
+// The owners of up to 4096 consecutive items (rows of boxes, instances of runs) win, win + 1, ..:
+// every lane names the first item (`start`) of its owner, `any` when it has items. Bit i of the 64
+// words is set when an owner begins at item win + i + 1, so the number of bits below an item (and
+// of those of the windows before it) is its owner's place among the lanes with items: two mask
+// counts per item, where marks and a prefix maximum over the lanes took 15 instructions. Lane j
+// receives word j (the items 64 j .. of the window).
+__device__ inline uint64_t item_starts(WaveSpans& w, bool any, uint32_t start, uint32_t win) {
     const uint32_t lane = __lane_id();
-    uint32_t rows = 0;
-    if (valid) {
-        const gsx_tile_span k = span_of(r0, r1);
-        const uint32_t bx = __float_as_uint(r1.z), by = __float_as_uint(r1.w);
-        w.mx[lane] = k.mx;
-        w.my[lane] = k.my;
-        w.b[lane] = k.b;
-        w.ra[lane] = k.ra;
-        w.det[lane] = k.det;
-        w.vr[lane] = k.vr;
-        w.aqs[lane] = k.aqs;
-        w.bx[lane] = bx;
-        w.by[lane] = by;
-        rows = (by >> 16) / kTile - (by & 0xffffu) / kTile + 1;
-    }
-    w.kept[lane] = 0;
-    const uint32_t incl = wave_inclusive_sum_u32(rows);
-    w.excl[lane] = incl - rows;
+    w.starts[lane] = 0ull;
     wave_lds_sync();
-    return (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+    const uint32_t bit = start - 1u - win;  // wraps past the window for starts up to win
+    if (any && bit < kWave * 64u) atomicOr(reinterpret_cast<uint32_t*>(w.starts) + (bit >> 5), 1u << (bit & 31u));
+    wave_lds_sync();
+    return w.starts[lane];
 }
 
-// Walks the wave's flattened rows. kEmit = false adds each row's kept tiles to kept[owner];
-// kEmit = true writes the kept instances (instance_tile, instance_gaussian) of every row, the
-// rows of a box in order, at base[owner] + the instances of the walked rows before it.
-template <bool kEmit, typename TileT>
-__device__ inline void walk_wave_rows(WaveSpans& w, uint32_t wave_rows, int32_t tiles_x,
-                                      uint32_t* __restrict__ instance_gaussian, TileT* __restrict__ instance_tile) {
+// Owner of the lane's item in the window's j-th 64 items; carry: owners begun before them.
+__device__ inline uint32_t item_owner(uint64_t words, uint32_t j, uint32_t& carry) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)words, (int)j);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(words >> 32), (int)j);
+    const uint32_t owner = __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, carry));
+    carry += (uint32_t)__popc(lo) + (uint32_t)__popc(hi);
+    return owner;
+}
+
+// What a lane keeps of its box while the wave walks: the box's slot, its first row (of the wave's)
+// and whether it has any; the wave's row count.
+struct WalkLane {
+    uint32_t slot, start, wave_rows;
+    bool any;
+};
+
+// Stores the lane's span constants and box (no rows when !valid).
+__device__ inline WalkLane stage_spans(WaveSpans& w, bool valid, const gsx_tile_span& k, float4 r1) {
+    const uint32_t bx = __float_as_uint(r1.z), by = __float_as_uint(r1.w);
+    const uint32_t rows = valid ? (by >> 16) / kTile - (by & 0xffffu) / kTile + 1 : 0u;
+    const uint32_t incl = wave_inclusive_sum_u32(rows);
+    const uint64_t m = wave_ballot(valid);
+    WalkLane l;
+    l.slot = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+    l.start = incl - rows;
+    l.wave_rows = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+    l.any = valid;
+    if (valid) {
+        w.ml[l.slot] = k.ml;
+        w.mh[l.slot] = k.mh;
+        w.my[l.slot] = k.my;
+        w.b[l.slot] = k.b;
+        w.ra[l.slot] = k.ra;
+        w.det[l.slot] = k.det;
+        w.vr[l.slot] = k.vr;
+        w.aqs[l.slot] = k.aqs;
+        w.bx[l.slot] = bx;
+        w.by[l.slot] = by;
+        w.excl[l.slot] = l.start;
+        w.kept[l.slot] = 0;
+    }
+    wave_lds_sync();
+    return l;
+}
+
+// The kept run of row p of the wave's rows, a row of the box in slot `owner`.
+__device__ inline void staged_row_run(const WaveSpans& w, uint32_t owner, uint32_t p, int32_t tiles_x, uint32_t& len,
+                                      uint32_t& tile0) {
+    gsx_tile_span k;
+    k.ml = w.ml[owner];
+    k.mh = w.mh[owner];
+    k.my = w.my[owner];
+    k.b = w.b[owner];
+    k.ra = w.ra[owner];
+    k.det = w.det[owner];
+    k.vr = w.vr[owner];
+    k.aqs = w.aqs[owner];
+    const uint32_t by = w.by[owner];
+    row_run(k, w.bx[owner], by, (by & 0xffffu) / kTile + (p - w.excl[owner]), tiles_x, len, tile0);
+}
+
+// Kept tiles of the lane's box, summed over the wave's flattened rows (64 rows a step).
+__device__ inline uint32_t count_wave_rows(WaveSpans& w, const WalkLane& l, int32_t tiles_x) {
     const uint32_t lane = __lane_id();
-    // the owner of item p is the last box starting at or before p, i.e. the last non-empty one
-    // (an empty box shares its start with the next box): each non-empty box whose rows start in
-    // the step marks that lane with base + its lane, and a prefix maximum over the lanes, carried
-    // from step to step, names every lane's owner (marks of earlier steps fall below base)
-    const uint32_t my_start = w.excl[lane];
-    const uint32_t my_count = (lane + 1 < kWave ? w.excl[lane + 1] : wave_rows) - my_start;
-    w.mark[lane] = UINT32_MAX;
-    uint32_t carry = 0, walked = 0;
-    for (uint32_t base = 0; base < wave_rows; base += kWave) {
+    uint32_t carry = 0;
+    uint64_t words = 0;
+    for (uint32_t base = 0; base < l.wave_rows; base += kWave) {
+        const uint32_t j = (base / kWave) % kWave;
+        if (j == 0) words = item_starts(w, l.any, l.start, base);
+        const uint32_t owner = item_owner(words, j, carry);
         const uint32_t p = base + lane;
-        wave_lds_sync();  // the previous step's reads of the marks are done
-        if (my_count > 0 && my_start - base < (uint32_t)kWave) w.mark[my_start - base] = base + lane;
-        wave_lds_sync();
-        const uint32_t m = w.mark[lane] - base;
-        const uint32_t owner = max(carry, (uint32_t)wave_inclusive_max(m < (uint32_t)kWave ? (int)m : 0));
-        carry = (uint32_t)__builtin_amdgcn_readlane((int)owner, kWave - 1);
-        uint32_t len = 0, tile0 = 0;
-        if (p < wave_rows) {
-            gsx_tile_span k;
-            k.mx = w.mx[owner];
-            k.my = w.my[owner];
-            k.b = w.b[owner];
-            k.ra = w.ra[owner];
-            k.det = w.det[owner];
-            k.vr = w.vr[owner];
-            k.aqs = w.aqs[owner];
-            const uint32_t by = w.by[owner];
-            const int ty = (int)((by & 0xffffu) / kTile + (p - w.excl[owner]));
-            row_run(k, w.bx[owner], by, ty, tiles_x, len, tile0);
-        }
-        if (!kEmit) {
+        if (p < l.wave_rows) {
+            uint32_t len, tile0;
+            staged_row_run(w, owner, p, tiles_x, len, tile0);
             if (len > 0) atomicAdd(&w.kept[owner], len);
-        } else {
-            // the step's runs, numbered q = start2 .. start2 + len - 1 in row order: run r holds
-            // position run_pos[r] + q and tile run_tile[r] + q
-            const uint32_t incl = wave_inclusive_sum_u32(len);
-            const uint32_t start2 = incl - len;
-            const uint32_t total2 = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-            w.run_tile[lane] = tile0 - start2;
-            w.run_pos[lane] = w.base[owner] + walked;
-            w.run_g[lane] = w.g[owner];
-            w.mark2[lane] = UINT32_MAX;
-            uint32_t carry2 = 0;
-            for (uint32_t base2 = 0; base2 < total2; base2 += kWave) {
-                const uint32_t q = base2 + lane;
-                wave_lds_sync();  // the run records are stored, the previous sub-step's marks read
-                if (len > 0 && start2 - base2 < (uint32_t)kWave) w.mark2[start2 - base2] = base2 + lane;
-                wave_lds_sync();
-                const uint32_t m2 = w.mark2[lane] - base2;
-                const uint32_t run = max(carry2, (uint32_t)wave_inclusive_max(m2 < (uint32_t)kWave ? (int)m2 : 0));
-                carry2 = (uint32_t)__builtin_amdgcn_readlane((int)run, kWave - 1);
-                if (q < total2) {
+        }
+    }
+    wave_lds_sync();
+    return l.any ? w.kept[l.slot] : 0u;
+}
+
+// Writes the kept instances (instance_tile, instance_gaussian) of the wave's boxes, the rows of a
+// box in order: instance i of the walk at position base + i of its box, where `base` is each lane's
+// base[] and g its Gaussian. A step takes 64 rows, then writes their instances 64 at a time: where
+// the boxes' positions follow one another (no big box between them), at one scalar address.
+// Vector instructions bound it (about 0.55 wave instructions a ns). Per 64 instances they were ~35
+// (marks, a prefix maximum over the lanes, three reads of the run and two 64-bit addresses) and are
+// ~13, a row's 64 were ~200 and are ~160: 335M instances of a 1080p image 726 -> 695 us (2 GB are
+// written), 5M 36 -> 31.5 us.
+template <typename TileT>
+__device__ inline void emit_wave_rows(WaveSpans& w, const WalkLane& l, uint32_t base_pos, uint32_t gaussian,
+                                      int32_t tiles_x, uint32_t* __restrict__ instance_gaussian,
+                                      TileT* __restrict__ instance_tile) {
+    const uint32_t lane = __lane_id();
+    const uint64_t boxes = wave_ballot(l.any);
+    if (boxes == 0ull) return;  // uniform
+    const uint32_t first_pos = (uint32_t)__builtin_amdgcn_readlane((int)base_pos, __builtin_ctzll(boxes));
+    const bool together = wave_ballot(l.any && base_pos != first_pos) == 0ull;
+    if (l.any) {
+        w.base[l.slot] = base_pos;
+        w.g[l.slot] = gaussian;
+    }
+    wave_lds_sync();
+    uint32_t carry = 0, walked = 0;
+    uint64_t words = 0;
+    for (uint32_t base = 0; base < l.wave_rows; base += kWave) {
+        const uint32_t j = (base / kWave) % kWave;
+        if (j == 0) words = item_starts(w, l.any, l.start, base);
+        const uint32_t owner = item_owner(words, j, carry);
+        const uint32_t p = base + lane;
+        uint32_t len = 0, tile0 = 0;
+        if (p < l.wave_rows) staged_row_run(w, owner, p, tiles_x, len, tile0);
+        const uint32_t incl = wave_inclusive_sum_u32(len);
+        const uint32_t start = incl - len;
+        const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+        const uint64_t rm = wave_ballot(len > 0);
+        const uint32_t slot =
+            __builtin_amdgcn_mbcnt_hi((uint32_t)(rm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)rm, 0u));
+        wave_lds_sync();  // the previous step's reads of the runs are done
+        if (len > 0) {
+            w.run[slot] = make_uint2(tile0 - start, w.g[owner]);
+            w.run_pos[slot] = w.base[owner] + walked;
+        }
+        uint32_t* const out_g = instance_gaussian + (first_pos + walked);
+        TileT* const out_t = instance_tile + (first_pos + walked);
+        uint32_t run_carry = 0;
+        uint64_t run_words = 0;
+        for (uint32_t base2 = 0; base2 < total; base2 += kWave) {
+            const uint32_t j2 = (base2 / kWave) % kWave;
+            if (j2 == 0) run_words = item_starts(w, len > 0, start, base2);
+            const uint32_t run = item_owner(run_words, j2, run_carry);
+            const uint32_t q = base2 + lane;
+            if (q < total) {
+                const uint2 r = w.run[run];
+                if (together) {
+                    // (byte offsets below 2^32: a step's runs are at most 64 rows of at most 4096 tiles)
+                    *reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(out_g) + q * 4u) = r.y;
+                    *reinterpret_cast<TileT*>(reinterpret_cast<char*>(out_t) + q * (uint32_t)sizeof(TileT)) =
+                        (TileT)(r.x + q);
+                } else {
                     const uint32_t pos = w.run_pos[run] + q;
-                    instance_gaussian[pos] = w.run_g[run];
-                    instance_tile[pos] = (TileT)(w.run_tile[run] + q);
+                    instance_gaussian[pos] = r.y;
+                    instance_tile[pos] = (TileT)(r.x + q);
                 }
             }
-            walked += total2;
         }
-        __builtin_amdgcn_wave_barrier();
+        walked += total;
     }
-    wave_lds_sync();
 }
 
 // The parameter gradient sinks (mean3d, rotation, logscale, opacity, sh0..sh3: `arrays` of
@@ -269,21 +328,13 @@ __global__ __launch_bounds__(256) void preprocess_kernel(
     const float* __restrict__ sh1, const float* __restrict__ sh2, const float* __restrict__ sh3, int sh_degree,
     CameraParams cam, float4* __restrict__ rec, float4* __restrict__ col, uint2* __restrict__ cbox,
     float4* __restrict__ cov_coef, uint32_t* __restrict__ tile_count,
-    float* __restrict__ visible_counter, uint32_t* __restrict__ big_list, uint32_t* __restrict__ big_count,
-    uint32_t* __restrict__ clear0, uint32_t* __restrict__ clear1, uint32_t* __restrict__ clear2,
-    unsigned long long* __restrict__ kept_part,
+    float* __restrict__ visible_counter, unsigned long long* __restrict__ kept_part,
     uint64_t* __restrict__ depth_keys, uint32_t depth_base, uint32_t depth_max, int index_bits,
     uint64_t big_key_flag, int count_shift, uint8_t* __restrict__ touched) {
     __shared__ WaveSpans s_spans[kWavesPerBlock];
     __shared__ uint32_t s_kept[kWavesPerBlock], s_big[kWavesPerBlock];
     WaveSpans& ws = s_spans[threadIdx.x / kWave];
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    // counters that later kernels accumulate into start at zero (plain stores, no fill launch)
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        *clear0 = 0u;
-        *clear1 = 0u;
-        *clear2 = 0u;
-    }
     // TRAIN: the blend backward marks the Gaussians it reaches (touched[g] = 1)
     if (touched != nullptr && g < n) touched[g] = 0;
     if (snap.dst[0] != nullptr && g < n) {
@@ -299,6 +350,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(
     }
     bool visible = false;
     float4 r0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), r1 = r0, r2 = r0;
+    gsx_tile_span span = {};
     if (g < n) {
         const Projected p =
             preprocess_one(g, mean3d, rotation, logscale, opacity, sh0, sh1, sh2, sh3, sh_degree, cam, true);
@@ -316,7 +368,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(
             rec[2 * g + 0] = r0;
             rec[2 * g + 1] = r1;
             col[g] = r2;
-            cbox[g] = contribution_box_packed(r0, r1);
+            cbox[g] = contribution_box_packed(r0, r1, span);
             if (cov_coef != nullptr) {
                 // d(conic)/d(cov2d) coefficients with the CPU's rounding (render.c:1578-1579,
                 // 1647-1655): the backward applies them per contribution, as the CPU does,
@@ -333,13 +385,11 @@ __global__ __launch_bounds__(256) void preprocess_kernel(
             }
         }
     }
+    // emitted by big_boxes_wave; rank_gather_kernel lists them. (Appending them here to one list, an
+    // atomic per wave on its length, serialised the kernel where a scene holds many: 112k of 6M
+    // Gaussians, 790 us against 350 without the list.)
     const bool big = visible && box_tiles(r1) > kBigTiles;
-    // emitted by big_box_wave; one atomic per wave (a scene can hold millions of big boxes)
-    const uint32_t big_slot = wave_append_slot(big_count, big);
-    if (big) big_list[big_slot] = (uint32_t)g;
-    const uint32_t rows = stage_spans(ws, visible, r0, r1);
-    walk_wave_rows<false, uint32_t>(ws, rows, cam.tiles_x, nullptr, nullptr);
-    const uint32_t kept = ws.kept[__lane_id()];
+    const uint32_t kept = count_wave_rows(ws, stage_spans(ws, visible, span, r1), cam.tiles_x);
     if (g < n) tile_count[g] = kept;
     // depth key of every Gaussian (~0 for invisible ones, which the depth sort drops);
     // big_key_flag (kBigKeyFlag or 0, see there) marks the big boxes for rank_gather_kernel;
@@ -378,7 +428,7 @@ __global__ __launch_bounds__(256) void preprocess_kernel(
     }
 }
 
-// Marks a big box's depth key (big_box_wave needs its rank). Used only when the sorted depth
+// Marks a big box's depth key (big_boxes_wave needs its rank). Used only when the sorted depth
 // bits end below bit 63, which holds for fewer than 2^31 Gaussians.
 constexpr uint64_t kBigKeyFlag = 1ull << 63;
 
@@ -387,60 +437,72 @@ constexpr uint64_t kBigKeyFlag = 1ull << 63;
 constexpr uint32_t kLaneRun = 32;
 
 // After the depth sort of the V visible Gaussians (V = *depth_count): the Gaussian of every
-// depth rank, its kept-tile count, the rank of each big box and of each Gaussian whose count
-// exceeds long_chunk (the only ranks looked up by Gaussian: by big-box emission and by the
-// projection backward for runs of several chunks; every Gaussian's when flagged_only is false)
-// and the list of ranks whose count exceeds long_chunk (the backward sums long runs in chunks of
-// that many positions). Ranks V..n-1 get count 0 and no Gaussian. Each workgroup also stores the
-// sum of its 256 counts in block_sums[block] and its number of counts above kLaneRun in
-// block_sums[gridDim.x + 1 + block], the first steps of the offsets scan and of the long-run
-// list (emit_block finishes both).
+// depth rank, its kept-tile count, and the rank of each Gaussian whose count exceeds long_chunk
+// (the only ranks looked up by Gaussian: by the projection backward, for runs of several chunks).
+// Ranks V..n-1 get count 0 and no Gaussian. The ranks of a workgroup's big boxes, each with the sum
+// of the workgroup's counts before it, go to big_ranks[256 block ..], in order. Each workgroup also stores four numbers of its 256 ranks, the
+// first steps of the scans that emission completes: block_sums[block] the sum of the counts, and
+// behind each other in arrays of gridDim.x + 1 the number of counts above kLaneRun, of big boxes
+// and of counts above long_chunk. (The lists of big boxes and of runs of several chunks took an
+// atomic on one length per wave before: 181 us at 6M ranks with 112k such boxes, half of them serial.)
 __global__ __launch_bounds__(256) void rank_gather_kernel(int64_t n, const uint32_t* __restrict__ depth_count,
                                                           const uint64_t* __restrict__ sorted_depth_keys,
-                                                          uint64_t index_mask, bool flagged_only,
+                                                          uint64_t index_mask, bool big_flag,
                                                           int count_shift, uint32_t count_mask,
                                                           const uint32_t* __restrict__ tile_count,
+                                                          const float4* __restrict__ rec,
                                                           uint32_t* __restrict__ rank_gaussian,
                                                           uint32_t* __restrict__ rank_count,
                                                           uint32_t* __restrict__ gaussian_rank,
                                                           uint32_t long_chunk,
-                                                          uint32_t* __restrict__ multi_list,
-                                                          uint32_t* __restrict__ multi_count,
+                                                          uint2* __restrict__ big_ranks,
                                                           uint32_t* __restrict__ block_sums) {
     __shared__ uint32_t s_sum[kWavesPerBlock];
-    __shared__ uint32_t s_long[kWavesPerBlock];
+    __shared__ uint32_t s_marks[kWavesPerBlock];  // long runs, big boxes, runs of several chunks: a byte each
     const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t c = 0;
+    bool big = false;
     if (r < n) {
         if (r < (int64_t)*depth_count) {
             const uint64_t key = sorted_depth_keys[r];
             const uint32_t g = (uint32_t)(key & index_mask);
             c = count_shift > 0 ? (uint32_t)(key >> count_shift) & count_mask : tile_count[g];
+            big = c > 0 && (big_flag ? (key & kBigKeyFlag) != 0 : box_tiles(rec[2 * (size_t)g + 1]) > kBigTiles);
             rank_gaussian[r] = g;
-            if (!flagged_only || (key & kBigKeyFlag) != 0 || c > long_chunk) gaussian_rank[g] = (uint32_t)r;
+            if (c > long_chunk) gaussian_rank[g] = (uint32_t)r;
         }
         rank_count[r] = c;
     }
-    // runs of several chunks are listed (rare: their boxes span more than long_chunk tiles); one
-    // atomic per wave that has any (c is 0 past the visible ranks)
-    const uint32_t multi_slot = wave_append_slot(multi_count, c > long_chunk);
-    if (c > long_chunk) multi_list[multi_slot] = (uint32_t)r;
     const uint32_t wave_sum = wave_reduce_sum_u32(c);
-    const uint32_t wave_long = (uint32_t)__popcll(__ballot(c > kLaneRun));
+    const uint64_t longs_m = wave_ballot(c > kLaneRun), bigs = wave_ballot(big), multis_m = wave_ballot(c > long_chunk);
     if (__lane_id() == 0) {
         s_sum[threadIdx.x / kWave] = wave_sum;
-        s_long[threadIdx.x / kWave] = wave_long;
+        s_marks[threadIdx.x / kWave] = (uint32_t)__popcll(longs_m) | ((uint32_t)__popcll(bigs) << 8) |
+                                       ((uint32_t)__popcll(multis_m) << 16);
     }
     __syncthreads();
+    if (bigs != 0ull) {  // uniform in the wave
+        uint32_t at = blockIdx.x * blockDim.x, before = wave_inclusive_sum_u32(c) - c;
+        for (int w = 0; w < (int)(threadIdx.x / kWave); ++w) {
+            at += (s_marks[w] >> 8) & 0xffu;
+            before += s_sum[w];
+        }
+        if (big) big_ranks[at + (uint32_t)__popcll(bigs & lanemask_lt())] = make_uint2((uint32_t)r, before);
+    }
     if (threadIdx.x == 0) {
-        uint32_t sum = 0, longs = 0;
+        uint32_t sum = 0, longs = 0, big_total = 0, multis = 0;
 #pragma unroll
         for (int w = 0; w < kWavesPerBlock; ++w) {
             sum += s_sum[w];
-            longs += s_long[w];
+            longs += s_marks[w] & 0xffu;
+            big_total += (s_marks[w] >> 8) & 0xffu;
+            multis += s_marks[w] >> 16;
         }
+        const size_t stride = (size_t)gridDim.x + 1;
         block_sums[blockIdx.x] = sum;
-        block_sums[gridDim.x + 1 + blockIdx.x] = longs;
+        block_sums[stride + blockIdx.x] = longs;
+        block_sums[2 * stride + blockIdx.x] = big_total;
+        block_sums[3 * stride + blockIdx.x] = multis;
     }
 }
 
@@ -462,8 +524,8 @@ __device__ inline void emit_block(uint32_t b, int64_t n, int64_t rank_end, const
                                   const uint32_t* __restrict__ block_prefix, uint32_t* __restrict__ offsets,
                                   int32_t tiles_x, uint32_t* __restrict__ instance_gaussian,
                                   TileT* __restrict__ instance_tile,
-                                  const uint32_t* __restrict__ long_prefix, uint32_t* __restrict__ long_list,
-                                  WaveSpans* s_spans, uint32_t* s_wave) {
+                                  size_t prefix_stride, uint32_t long_chunk, uint32_t* __restrict__ long_list,
+                                  uint32_t* __restrict__ multi_list, WaveSpans* s_spans, uint32_t* s_wave) {
     WaveSpans& ws = s_spans[threadIdx.x / kWave];
     const int64_t r = (int64_t)b * blockDim.x + threadIdx.x;
     // the rank's count and Gaussian load together, then its whole record (one wait each)
@@ -478,17 +540,23 @@ __device__ inline void emit_block(uint32_t b, int64_t n, int64_t rank_end, const
     // offsets[n] (the instance total, read by the ranges pass) from the last rank launched: the
     // launch covers the visible ranks and at least one more, whose counts are 0
     if (r == rank_end - 1) offsets[n] = o + cnt;
-    // the long-run list in rank order: long_prefix[b] (scanned per-workgroup counts of
-    // rank_gather_kernel) + the rank's place among the workgroup's long runs (s_wave is free
-    // again after the scan's last barrier)
+    // the lists of long runs and of runs of several chunks, in rank order: the workgroup's scanned
+    // start + the rank's place among the workgroup's (s_wave is free again after the scan's last
+    // barrier)
     {
-        const bool is_long = cnt > kLaneRun;
-        const uint64_t lm = __ballot(is_long);
-        if (__lane_id() == 0) s_wave[threadIdx.x / kWave] = (uint32_t)__popcll(lm);
+        const bool is_long = cnt > kLaneRun, is_multi = cnt > long_chunk;
+        const uint64_t lm = wave_ballot(is_long), mm = wave_ballot(is_multi);
+        if (__lane_id() == 0)
+            s_wave[threadIdx.x / kWave] = (uint32_t)__popcll(lm) | ((uint32_t)__popcll(mm) << 16);
         __syncthreads();
-        uint32_t at = long_prefix[b] + (uint32_t)__popcll(lm & lanemask_lt());
-        for (int w = 0; w < (int)(threadIdx.x / kWave); ++w) at += s_wave[w];
-        if (is_long) long_list[at] = (uint32_t)r;
+        uint32_t before = 0;  // both counts: at most 192 each
+        for (int w = 0; w < (int)(threadIdx.x / kWave); ++w) before += s_wave[w];
+        if (is_long)
+            long_list[block_prefix[prefix_stride + b] + (before & 0xffffu) + (uint32_t)__popcll(lm & lanemask_lt())] =
+                (uint32_t)r;
+        if (is_multi)
+            multi_list[block_prefix[3 * prefix_stride + b] + (before >> 16) + (uint32_t)__popcll(mm & lanemask_lt())] =
+                (uint32_t)r;
     }
     float4 r0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), r1 = r0;
     if (cnt > 0) {
@@ -500,68 +568,88 @@ __device__ inline void emit_block(uint32_t b, int64_t n, int64_t rank_end, const
     // before it (the counting walk's identical runs gave the counts)
     const bool walked = cnt > 0 && box_tiles(r1) <= kBigTiles;
     const uint32_t wcnt = walked ? cnt : 0u;
-    const uint32_t lane = __lane_id();
-    ws.base[lane] = o - (wave_inclusive_sum_u32(wcnt) - wcnt);
-    ws.g[lane] = g;
-    const uint32_t rows = stage_spans(ws, walked, r0, r1);
-    walk_wave_rows<true, TileT>(ws, rows, tiles_x, instance_gaussian, instance_tile);
+    const uint32_t base_pos = o - (wave_inclusive_sum_u32(wcnt) - wcnt);
+    emit_wave_rows<TileT>(ws, stage_spans(ws, walked, span_of(r0, r1), r1), base_pos, g, tiles_x, instance_gaussian,
+                          instance_tile);
 }
 
-// Big boxes: one wave per box of big_list, walking its rows as walk_wave_rows walks a wave's
-// boxes (the box in lane 0, the others empty). It runs beside emit_block in one launch, so it
-// forms the box's offset itself: block_prefix of the rank's 256-rank block plus the counts of the
-// ranks before it in that block. The host sizes the launch with one wave per big box.
+// Big boxes first .. first + per_wave - 1 (in rank order, those below big_prefix[blocks]): a wave walks
+// their rows as emit_block walks a wave's boxes. It runs beside emit_block in one launch, so each lane
+// finds its box's place itself: box i is the (i - big_prefix[b])-th of block b's, the last block with
+// big_prefix[b] <= i, and its offset block_prefix[b] plus the counts before it in the block. (The
+// lanes past per_wave search along, so that the walk runs with the whole wave.)
 template <typename TileT>
-__device__ inline void big_box_wave(uint32_t i, const uint32_t* __restrict__ big_list, const float4* __restrict__ rec,
-                                    int32_t tiles_x, const uint32_t* __restrict__ rank_count,
-                                    const uint32_t* __restrict__ block_prefix,
-                                    const uint32_t* __restrict__ gaussian_rank,
-                                    uint32_t* __restrict__ instance_gaussian, TileT* __restrict__ instance_tile,
-                                    WaveSpans& ws) {
+__device__ inline void big_boxes_wave(uint32_t first, uint32_t per_wave, const uint2* __restrict__ big_ranks,
+                                      const uint32_t* __restrict__ big_prefix, uint32_t blocks,
+                                      const float4* __restrict__ rec, int32_t tiles_x,
+                                      const uint32_t* __restrict__ rank_gaussian,
+                                      const uint32_t* __restrict__ rank_count,
+                                      const uint32_t* __restrict__ block_prefix,
+                                      uint32_t* __restrict__ instance_gaussian, TileT* __restrict__ instance_tile,
+                                      WaveSpans& ws) {
     const uint32_t lane = __lane_id();
-    const uint32_t g = big_list[i];
+    const uint32_t total = big_prefix[blocks];
+    if (first >= total) return;  // uniform
+    const bool mine = lane < per_wave && first + lane < total;
+    const uint32_t i = mine ? first + lane : first;
+    uint32_t block = 0, span = blocks;  // the block is one of block .. block + span - 1
+    if (per_wave == 1u) {  // uniform: the wave compares 64 counts at a time (3 loads in turn for 6M ranks,
+                           // where halving takes 15: 3 us of a launch with a few big boxes)
+        while (span > 1) {
+            const uint32_t step = (span + kWave - 1) / kWave;
+            const uint32_t at = lane * step;  // (lane 0 always counts)
+            const uint64_t m = wave_ballot(at < span && big_prefix[min(block + at, blocks)] <= i);
+            const uint32_t last = ((uint32_t)__popcll(m) - 1u) * step;
+            block += last;
+            span = min(step, span - last);
+        }
+    } else {
+        while (span > 1) {
+            const uint32_t half = span / 2;
+            if (big_prefix[block + half] <= i) block += half;
+            span -= half;
+        }
+    }
+    const uint2 rank = big_ranks[block * 256u + (i - big_prefix[block])];
+    const uint32_t g = rank_gaussian[rank.x];
+    const uint32_t cnt = mine ? rank_count[rank.x] : 0u;
     const float4 r0 = rec[2 * (size_t)g + 0], r1 = rec[2 * (size_t)g + 1];
-    const uint32_t rr = gaussian_rank[g];
-    const uint32_t b0 = rr & ~255u;
-    uint32_t v = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < 256; k += kWave) v += b0 + k + lane < rr ? rank_count[b0 + k + lane] : 0u;
-    ws.base[lane] = block_prefix[rr >> 8] + wave_reduce_sum_u32(v);
-    ws.g[lane] = g;
-    const uint32_t rows = stage_spans(ws, lane == 0, r0, r1);
-    walk_wave_rows<true, TileT>(ws, rows, tiles_x, instance_gaussian, instance_tile);
+    // (less the instances of the wave's boxes before it, as in emit_block)
+    const uint32_t base_pos = block_prefix[block] + rank.y - (wave_inclusive_sum_u32(cnt) - cnt);
+    emit_wave_rows<TileT>(ws, stage_spans(ws, mine, span_of(r0, r1), r1), base_pos, g, tiles_x, instance_gaussian,
+                          instance_tile);
 }
 
-// All emission in one launch: workgroups [0, big_blocks) hold one wave per big box, first so
-// that their longer walks start early; the rest are the emission workgroups of the ranks.
+// All emission in one launch: workgroups [0, big_blocks) hold the waves of big boxes, first so
+// that their longer walks start early, big_per_wave boxes each; the rest are the emission workgroups of the ranks.
+// block_prefix: rank_gather_kernel's four arrays of `prefix_stride` entries, scanned.
 template <typename TileT>
 __global__ __launch_bounds__(256) void emit_kernel(int64_t n, const float4* __restrict__ rec,
                                                    const uint32_t* __restrict__ rank_gaussian,
                                                    const uint32_t* __restrict__ rank_count,
-                                                   const uint32_t* __restrict__ block_prefix,
+                                                   const uint32_t* __restrict__ block_prefix, size_t prefix_stride,
                                                    uint32_t* __restrict__ offsets, int32_t tiles_x,
-                                                   const uint32_t* __restrict__ big_list,
-                                                   const uint32_t* __restrict__ big_count, uint32_t big_blocks,
-                                                   const uint32_t* __restrict__ gaussian_rank,
+                                                   const uint2* __restrict__ big_ranks, uint32_t big_blocks,
+                                                   uint32_t big_per_wave,
                                                    uint32_t* __restrict__ instance_gaussian,
-                                                   TileT* __restrict__ instance_tile,
-                                                   const uint32_t* __restrict__ long_prefix,
-                                                   uint32_t* __restrict__ long_list) {
+                                                   TileT* __restrict__ instance_tile, uint32_t long_chunk,
+                                                   uint32_t* __restrict__ long_list,
+                                                   uint32_t* __restrict__ multi_list) {
     __shared__ WaveSpans s_spans[kWavesPerBlock];
     __shared__ uint32_t s_wave[kWavesPerBlock];
     if (blockIdx.x < big_blocks) {
-        // no workgroup barrier on this path: each wave takes its own box
-        const uint32_t i = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
-        if (i < *big_count)
-            big_box_wave(i, big_list, rec, tiles_x, rank_count, block_prefix, gaussian_rank, instance_gaussian,
-                         instance_tile, s_spans[threadIdx.x / kWave]);
+        // no workgroup barrier on this path: each wave takes its own boxes
+        const uint32_t w = blockIdx.x * kWavesPerBlock + threadIdx.x / kWave;
+        big_boxes_wave(w * big_per_wave, big_per_wave, big_ranks, block_prefix + 2 * prefix_stride,
+                       (uint32_t)prefix_stride - 1u, rec, tiles_x, rank_gaussian, rank_count, block_prefix,
+                       instance_gaussian, instance_tile, s_spans[threadIdx.x / kWave]);
         return;
     }
     // the rank workgroups cover ranks [0, rank_end): the visible ones and at least one past them
     // (ranks of invisible Gaussians emit nothing, and no kernel reads their offsets)
     const int64_t rank_end = min(n, (int64_t)(gridDim.x - big_blocks) * blockDim.x);
     emit_block(blockIdx.x - big_blocks, n, rank_end, rec, rank_gaussian, rank_count, block_prefix, offsets, tiles_x,
-               instance_gaussian, instance_tile, long_prefix, long_list, s_spans, s_wave);
+               instance_gaussian, instance_tile, prefix_stride, long_chunk, long_list, multi_list, s_spans, s_wave);
 }
 
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* __restrict__ p, int64_t count, uint32_t v) {
@@ -1393,7 +1481,7 @@ __global__ __launch_bounds__(kBlendThreads, 5) void blend_backward_kernel(
 //    cover nearly every tile) are cut into at most kLongChunks chunks of `chunk` positions, and
 //    one wave sums a chunk (DPP tree, reduce_run_chunk). reduce_long_block takes chunk 0 of every
 //    long run (long_list, in rank order, written by emit_block) and chunks 1.. of the runs longer
-//    than one chunk (multi_list, from rank_gather_kernel), the entries dealt round-robin over the
+//    than one chunk (multi_list, in rank order), the entries dealt round-robin over the
 //    waves: the near, large Gaussians are neighbours in depth order, and a wave of their own
 //    would serialise them. A run of one chunk is done; the others leave each chunk's sums in
 //    place at its first position, and projection_backward_kernel adds them in chunk order.

@@ -35,6 +35,21 @@ GSX_HD float gsx_cull_minf(float a, float b) { return fminf(a, b); }
 GSX_HD float gsx_cull_maxf(float a, float b) { return fmaxf(a, b); }
 GSX_HD float gsx_cull_absf(float a) { return fabsf(a); }
 #endif
+/* Correctly rounded square root of x >= 2^-80 (or +inf). On the GPU without the scaling and the class
+ * test that sqrtf spends on smaller arguments (half its 18 instructions): the hardware root s is
+ * within one unit in the last place, and x <= s (s - ulp) or x > s (s + ulp) tell the neighbour
+ * that is nearer (Tuckerman's test). */
+#if defined(__HIP_DEVICE_COMPILE__)
+GSX_HD float gsx_cull_sqrtf(float x)
+{
+    const float s = __builtin_amdgcn_sqrtf(x);
+    const float below = gsx_f32_from_bits(gsx_f32_bits(s) - 1u), above = gsx_f32_from_bits(gsx_f32_bits(s) + 1u);
+    const float r = GSX_FMAF(-below, s, x) <= 0.0f ? below : s;
+    return GSX_FMAF(-above, s, x) > 0.0f ? above : r;
+}
+#else
+GSX_HD float gsx_cull_sqrtf(float x) { return sqrtf(x); }
+#endif
 GSX_HD float gsx_cull_clampf(float v, float lo, float hi) { return gsx_cull_minf(gsx_cull_maxf(v, lo), hi); }
 
 /* Natural logarithm of a positive normal float from IEEE operations only, so the CPU and the
@@ -91,14 +106,19 @@ GSX_HD float gsx_tile_qcut(float opacity)
  *   the remaining roundings (of -B v + sqrt(D), of the product with 1 / A) are below
  *          3 eps (sqrt(kappa) + 1) sqrt(Q / A), and the factor widens the span by at least
  *          2^-15 sqrt(Q / A), 8 times more.
- * A pixel column x is kept when its centre offset fl(fl(x + 0.5) - mx), the value the kernels
- * evaluate, lies in [u-, u+]; fl is monotone, so the kept columns are one interval, found from
- * floor / ceil of mx + u -/+ 0.5 and one exact check on each side. A Gaussian whose form is not
+ * D is held above 2^-80, which only widens the span.
+ * A pixel column x may be contributed to when its centre offset fl(fl(x + 0.5) - mx), the value the
+ * kernels evaluate, lies in [u-, u+]. Kept are the columns from ceil(mx - 0.5 - m + u-) to
+ * floor(mx - 0.5 + m + u+), m = 2^-6 + 2^-21 |mx|: the roundings of the offset, of mx - 0.5 -/+ m and of
+ * the sum are below 2^-22 |mx| + 2^-7 for columns below 2^16. (An exact check of the column on each
+ * side instead kept 0.1% fewer tiles and cost 30 of a row's 200 vector instructions.)
+ * A Gaussian whose form is not
  * positive definite, whose kappa exceeds 2^16 (det then carries more than 1% rounding) or whose
  * mean lies beyond 2^21 pixels, or any non-finite constant, keeps every column of its box:
- * aqs = +inf, det = vr = B = 0 and ra = 1 make every band span the box without a branch. */
+ * aqs = +inf, det = vr = B = 0, ra = 1 and a mean of 0 make every band span the box without a branch. */
 typedef struct gsx_tile_span {
-    float mx, my; /* mean2d */
+    float ml, mh; /* mx - 0.5 less and plus the margin m */
+    float my;     /* mean2d y */
     float b;      /* inv_b */
     float ra;     /* 1 / inv_a */
     float det;    /* inv_a inv_c - inv_b^2 */
@@ -106,34 +126,58 @@ typedef struct gsx_tile_span {
     float aqs;    /* inv_a Q with the rounding allowance */
 } gsx_tile_span;
 
-/* Constants of the Gaussian with conic (inv_a, inv_b, inv_c), activated opacity `opacity` and
- * inclusive pixel box [x0, x1] x [y0, y1]. */
-GSX_HD gsx_tile_span gsx_tile_span_make(float mx, float my, float inv_a, float inv_b, float inv_c, float opacity,
+/* The part of a Gaussian's constants that its row spans and its column spans share: Q, det, A C and
+ * the rounding allowance of aqs. */
+typedef struct gsx_tile_form {
+    float q;     /* Q */
+    float ac;    /* inv_a inv_c */
+    float det;   /* inv_a inv_c - inv_b^2 */
+    float slack; /* 2^-14 + kappa 2^-19 */
+} gsx_tile_form;
+
+GSX_HD gsx_tile_form gsx_tile_form_make(float mx, float my, float inv_a, float inv_b, float inv_c, float opacity,
     int x0, int x1, int y0, int y1)
 {
-    gsx_tile_span k;
+    gsx_tile_form f;
     const float A = inv_a, B = inv_b, C = inv_c;
     const float dx0 = ((float)x0 + 0.5f) - mx, dx1 = ((float)x1 + 0.5f) - mx;
     const float dy0 = ((float)y0 + 0.5f) - my, dy1 = ((float)y1 + 0.5f) - my;
     const float X = gsx_cull_maxf(gsx_cull_absf(dx0), gsx_cull_absf(dx1));
     const float Y = gsx_cull_maxf(gsx_cull_absf(dy0), gsx_cull_absf(dy1));
     const float S = gsx_cull_absf(A) * X * X + 2.0f * gsx_cull_absf(B) * X * Y + gsx_cull_absf(C) * Y * Y;
-    const float Q = gsx_tile_qcut(opacity) + (1e-5f * S + 1e-3f);
-    const float ac = A * C;
-    const float det = ac - B * B;
-    const float kappa = ac / det;
-    const float slack = 6.103515625e-05f + kappa * 1.9073486328125e-06f; /* 2^-14 + kappa 2^-19 */
 
-    k.mx = mx;
+    f.q = gsx_tile_qcut(opacity) + (1e-5f * S + 1e-3f);
+    f.ac = A * C;
+    f.det = f.ac - B * B;
+    f.slack = 6.103515625e-05f + (f.ac / f.det) * 1.9073486328125e-06f;
+    return f;
+}
+
+/* Constants of the Gaussian whose form is f = gsx_tile_form_make(...). With x and y (and inv_a and
+ * inv_c) exchanged they are those of its column spans: f is the same up to the rounding of S, which
+ * the allowance covers 40 times over. */
+GSX_HD gsx_tile_span gsx_tile_span_of_form(const gsx_tile_form *f, float mx, float my, float inv_a, float inv_b,
+    float inv_c)
+{
+    gsx_tile_span k;
+    const float A = inv_a, B = inv_b, C = inv_c;
+
+    const float margin = 0.015625f + 4.76837158203125e-07f * gsx_cull_absf(mx);
+
+    k.ml = (mx - 0.5f) - margin;
+    k.mh = (mx - 0.5f) + margin;
     k.my = my;
     k.b = B;
     k.ra = 1.0f / A;
-    k.det = det;
-    k.vr = -B * sqrtf(Q / (det * C));
-    k.aqs = (A * Q) * (1.0f + slack);
+    k.det = f->det;
+    k.vr = -B * sqrtf(f->q / (f->det * C));
+    k.aqs = (A * f->q) * (1.0f + f->slack);
     /* the comparisons are false for NaN, which therefore keeps every column too */
-    if(!(A > 0.0f && C > 0.0f && det > 0.0f && det * 65536.0f >= ac && gsx_cull_absf(mx) < 2097152.0f &&
+    if(!(A > 0.0f && C > 0.0f && f->det > 0.0f && f->det * 65536.0f >= f->ac && gsx_cull_absf(mx) < 2097152.0f &&
            gsx_cull_absf(my) < 2097152.0f && gsx_cull_absf(k.vr) <= 3.0e38f && k.aqs <= 3.0e38f && k.ra <= 3.0e38f)) {
+        k.ml = 0.0f;
+        k.mh = 0.0f;
+        k.my = 0.0f;
         k.b = 0.0f;
         k.ra = 1.0f;
         k.det = 0.0f;
@@ -141,6 +185,16 @@ GSX_HD gsx_tile_span gsx_tile_span_make(float mx, float my, float inv_a, float i
         k.aqs = __builtin_inff();
     }
     return k;
+}
+
+/* Constants of the Gaussian with conic (inv_a, inv_b, inv_c), activated opacity `opacity` and
+ * inclusive pixel box [x0, x1] x [y0, y1]. */
+GSX_HD gsx_tile_span gsx_tile_span_make(float mx, float my, float inv_a, float inv_b, float inv_c, float opacity,
+    int x0, int x1, int y0, int y1)
+{
+    const gsx_tile_form f = gsx_tile_form_make(mx, my, inv_a, inv_b, inv_c, opacity, x0, x1, y0, y1);
+
+    return gsx_tile_span_of_form(&f, mx, my, inv_a, inv_b, inv_c);
 }
 
 /* The pixel columns [*xa, *xb] of the box [x0, x1] whose centres may receive a contribution in
@@ -151,39 +205,17 @@ GSX_HD void gsx_tile_band_columns(const gsx_tile_span *k, int x0, int x1, int py
     const float vh = gsx_cull_clampf(k->vr, v0, v1);
     const float vl = gsx_cull_clampf(k->vr, -v1, -v0);
     const float dh = k->aqs - (k->det * vh) * vh;
-    const float dl = gsx_cull_maxf(k->aqs - (k->det * vl) * vl, 0.0f);
-    const float uh = (sqrtf(dh) - k->b * vh) * k->ra;
-    const float ul = -((sqrtf(dl) - k->b * vl) * k->ra);
-    const float sh = (k->mx + uh) - 0.5f, sl = (k->mx + ul) - 0.5f;
-    int c;
+    const float dl = k->aqs - (k->det * vl) * vl;
+    const float uh = (gsx_cull_sqrtf(gsx_cull_maxf(dh, 8.27180613e-25f)) - k->b * vh) * k->ra;
+    const float ul = -((gsx_cull_sqrtf(gsx_cull_maxf(dl, 8.27180613e-25f)) - k->b * vl) * k->ra);
 
     if(dh < 0.0f) { /* the band misses the set */
         *xa = 1;
         *xb = 0;
         return;
     }
-    /* last column whose centre offset is at most uh */
-    if(!(sh < (float)x1)) {
-        c = x1;
-    } else if(!(sh >= (float)x0 - 1.0f)) {
-        c = x0 - 1;
-    } else {
-        c = (int)floorf(sh);
-        if(c + 1 <= x1 && (((float)(c + 1) + 0.5f) - k->mx) <= uh) c += 1;
-        if(c >= x0 && !((((float)c + 0.5f) - k->mx) <= uh)) c -= 1;
-    }
-    *xb = c;
-    /* first column whose centre offset is at least ul */
-    if(!(sl > (float)x0)) {
-        c = x0;
-    } else if(!(sl <= (float)x1 + 1.0f)) {
-        c = x1 + 1;
-    } else {
-        c = (int)ceilf(sl);
-        if(c - 1 >= x0 && (((float)(c - 1) + 0.5f) - k->mx) >= ul) c -= 1;
-        if(c <= x1 && !((((float)c + 0.5f) - k->mx) >= ul)) c += 1;
-    }
-    *xa = c;
+    *xb = (int)floorf(gsx_cull_maxf(gsx_cull_minf(k->mh + uh, (float)x1), (float)x0 - 1.0f));
+    *xa = (int)ceilf(gsx_cull_minf(gsx_cull_maxf(k->ml + ul, (float)x0), (float)x1 + 1.0f));
 }
 
 /* The pixel rectangle [*xa, *xb] x [*ya, *yb] of the box [x0, x1] x [y0, y1] that holds every
@@ -191,15 +223,25 @@ GSX_HD void gsx_tile_band_columns(const gsx_tile_span *k, int x0, int x1, int py
  * test with the whole box as one band, the rows from the same test with the roles of x and y
  * exchanged (q(u, v) is the same form with A and C swapped, and the rounding allowances are
  * symmetric in u and v). Empty when *xa > *xb or *ya > *yb. The blend kernels test pixels
- * against this rectangle instead of the 3-sigma box: a pixel outside it fails the CPU's cuts. */
+ * against this rectangle instead of the 3-sigma box: a pixel outside it fails the CPU's cuts.
+ * *k receives the row-span constants (gsx_tile_span_make's), which the tile lists need as well. */
+GSX_HD void gsx_contribution_box_and_span(float mx, float my, float inv_a, float inv_b, float inv_c, float opacity, int x0,
+    int x1, int y0, int y1, gsx_tile_span *k, int *xa, int *xb, int *ya, int *yb)
+{
+    const gsx_tile_form f = gsx_tile_form_make(mx, my, inv_a, inv_b, inv_c, opacity, x0, x1, y0, y1);
+    const gsx_tile_span ky = gsx_tile_span_of_form(&f, my, mx, inv_c, inv_b, inv_a);
+
+    *k = gsx_tile_span_of_form(&f, mx, my, inv_a, inv_b, inv_c);
+    gsx_tile_band_columns(k, x0, x1, y0, y1, xa, xb);
+    gsx_tile_band_columns(&ky, y0, y1, x0, x1, ya, yb);
+}
+
 GSX_HD void gsx_contribution_box(float mx, float my, float inv_a, float inv_b, float inv_c, float opacity, int x0,
     int x1, int y0, int y1, int *xa, int *xb, int *ya, int *yb)
 {
-    const gsx_tile_span kx = gsx_tile_span_make(mx, my, inv_a, inv_b, inv_c, opacity, x0, x1, y0, y1);
-    const gsx_tile_span ky = gsx_tile_span_make(my, mx, inv_c, inv_b, inv_a, opacity, y0, y1, x0, x1);
+    gsx_tile_span k;
 
-    gsx_tile_band_columns(&kx, x0, x1, y0, y1, xa, xb);
-    gsx_tile_band_columns(&ky, y0, y1, x0, x1, ya, yb);
+    gsx_contribution_box_and_span(mx, my, inv_a, inv_b, inv_c, opacity, x0, x1, y0, y1, &k, xa, xb, ya, yb);
 }
 
 /* Nonzero when some pixel centre of the inclusive pixel rectangle [px0, px1] x [py0, py1] may
