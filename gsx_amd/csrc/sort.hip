@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -270,8 +271,9 @@ __device__ inline uint32_t digit_exclusive_scan(uint32_t v, uint32_t* s_wave, ui
 // n * max(sizeof(KeyT), 4) <= 2^32, so every output byte offset fits in 32 bits. kThreads: workgroup size
 // (kChunk / kThreads keys per thread). Register target: 8 waves per SIMD, except for 64-bit keys
 // with values, whose 54 KB of LDS admits two workgroups (4 waves per SIMD) per CU anyway.
+// kFirst: vals_in is null (and is then known to be).
 template <bool kPairs, int kBits, int kChunk, typename KeyT = uint64_t, bool kNarrow = false,
-          int kThreads = kDownThreads>
+          int kThreads = kDownThreads, bool kFirst = false>
 __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) void radix_downsweep_kernel(
     const KeyT* __restrict__ keys_in, const uint32_t* __restrict__ vals_in, int64_t n,
     const uint32_t* __restrict__ n_dev, bool drop_sentinel, int shift, uint32_t dmask, int64_t num_chunks,
@@ -284,7 +286,14 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     // the reordered chunk: 16- and 32-bit keys with values as one 64-bit entry per key (one scatter
     // store instead of two), otherwise keys (and values) in arrays of their own
     constexpr bool kPack = kPairs && sizeof(KeyT) <= 4;
-    __shared__ uint64_t s_kv[kPack ? kChunk : 1];
+    // .. and 16-bit keys in the first pass as key | place in the chunk << 16: the place gives the value.
+    // The scattered stores of this reorder bound the first pass where emission leaves neighbours of 128
+    // digits side by side (335M keys, 7 bits: 1235 us with 8 bytes per key, 780 with 4; chunks of 16384
+    // keys, which 4 bytes would allow, 940).
+    constexpr bool kPackPlace = kPack && kFirst && sizeof(KeyT) == 2;
+    static_assert(!kPackPlace || kChunk <= 65536, "16-bit places");
+    using EntryT = std::conditional_t<kPackPlace, uint32_t, uint64_t>;
+    __shared__ EntryT s_kv[kPack ? kChunk : 1];
     __shared__ KeyT s_keys[kPack ? 1 : kChunk];
     __shared__ uint32_t s_vals[(kPairs && !kPack) ? kChunk : 1];
     constexpr int kBins = 1 << kBits;
@@ -300,10 +309,14 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     static_assert(!kCnt16 || kChunk <= 65536, "16-bit counters");
     __shared__ uint32_t s_cnt32[kWaves][kHalf];
     using CntT = std::conditional_t<kCnt16, uint16_t, uint32_t>;
-    auto cnt = [&](int w, uint32_t d) -> CntT& {
-        if constexpr (kCnt16) return reinterpret_cast<uint16_t*>(&s_cnt32[w][0])[2 * (d % kHalf) + d / kHalf];
-        else return s_cnt32[w][d];
+    const auto cnt_offset = [&](int w, uint32_t d) -> uint32_t {  // bytes
+        return (uint32_t)w * (kHalf * 4u) + (kCnt16 ? (d % kHalf) * 4u + (d / kHalf) * 2u : d * 4u);
     };
+    static_assert(sizeof(s_cnt32) <= 65536, "a counter's offset fits beside a rank");
+    const auto cnt_at = [&](uint32_t offset) -> CntT& {
+        return *reinterpret_cast<CntT*>(reinterpret_cast<char*>(&s_cnt32[0][0]) + offset);
+    };
+    const auto cnt = [&](int w, uint32_t d) -> CntT& { return cnt_at(cnt_offset(w, d)); };
     // output position of the reordered chunk's position 0 as counted in each digit: the digit's
     // run starts at s_out[d] + (its start in the reordered chunk) (modulo 2^32)
     __shared__ uint32_t s_out[kBins];
@@ -317,6 +330,10 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     if (n_dev != nullptr) n = min(n, (int64_t)*n_dev);
     if (base >= n) return;  // uniform: a chunk past the live count has nothing to move
     const int chunk_count = (int)min((int64_t)kChunk, n - base);
+    // a whole chunk whose keys all move (every one but the last, where no key is dropped) needs no test
+    // of any of its keys (with the counters addressed once a key and ranks by mask counts: 709 -> ~480
+    // vector instructions a wave of 512 keys; 335M keys, second pass of 6 bits, 930 -> 775 us)
+    const bool whole = !drop_sentinel && chunk_count == kChunk;
     // this chunk's digit offsets and the digit totals, loaded with the keys (threads past kBins
     // re-read digit kBins - 1 and ignore it)
     const int td = min((int)threadIdx.x, kBins - 1);
@@ -325,53 +342,64 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     for (int i = threadIdx.x; i < kWaves * kHalf; i += kThreads) (&s_cnt32[0][0])[i] = 0;
     __syncthreads();
     // 1. per wave: stable ranks among equal digits (rank = keys of the digit before it in this
-    //    wave's eighth of the chunk), packed as digit << 16 | rank
-    const uint64_t lt = lanemask_lt();
+    //    wave's eighth of the chunk), packed as offset of the digit's counter << 16 | rank
+    const int digit_width = __popc(dmask);
+    const auto digit = [&](KeyT k) -> uint32_t {
+        if constexpr (sizeof(KeyT) <= 4) return __builtin_amdgcn_ubfe((uint32_t)k, (uint32_t)shift, (uint32_t)digit_width);
+        else return digit_of<kBits>(k, shift) & dmask;
+    };
     KeyT key[kDownRounds];
     uint32_t val[kDownRounds];
     uint32_t dr[kDownRounds];
+    const auto rank_keys = [&](auto all) {
+        constexpr bool kAll = decltype(all)::value;
+        const int first = wave * kDownWaveKeys + lane;
 #pragma unroll
-    for (int r = 0; r < kDownRounds; ++r) {
-        const int local = wave * kDownWaveKeys + r * kWave + lane;
-        const bool valid = local < chunk_count;
-        key[r] = valid ? keys_in[base + local] : (KeyT)0;
-        if (kPairs) val[r] = vals_in == nullptr ? (uint32_t)(base + local) : (valid ? vals_in[base + local] : 0u);
-        else val[r] = 0u;
-    }
-#pragma unroll
-    for (int r = 0; r < kDownRounds; ++r) {
-        const int local = wave * kDownWaveKeys + r * kWave + lane;
-        const bool valid = local < chunk_count && !(drop_sentinel && (uint64_t)key[r] == kSentinelKey);
-        const uint32_t d = digit_of<kBits>(key[r], shift) & dmask;
-        const uint64_t vm = wave_ballot(valid);
-        // per digit bit: the bit as 0 / all ones (a signed bit-field extract) and the wave's ballot
-        // of it; the lanes that agree with this lane in bit b are ~(ballot ^ ext), folded into the
-        // peer mask with one three-input bitwise operation per half (truth table 0x90:
-        // p & ~(m ^ e))
-        uint32_t ext[kBits];
-        uint64_t m[kBits];
-#pragma unroll
-        for (int b = 0; b < kBits; ++b) {
-            ext[b] = (uint32_t)((int32_t)(d << (31 - b)) >> 31);
-            asm volatile("" : "+v"(ext[b]));  // the ballot compares the extracted bit itself
+        for (int r = 0; r < kDownRounds; ++r) {
+            const int local = first + r * kWave;
+            const bool valid = kAll || local < chunk_count;
+            key[r] = valid ? (keys_in + base)[local] : (KeyT)0;
+            if (kPackPlace) val[r] = (uint32_t)local;
+            else if (kPairs) val[r] = kFirst || vals_in == nullptr ? (uint32_t)base + (uint32_t)local : (valid ? (vals_in + base)[local] : 0u);
+            else val[r] = 0u;
         }
 #pragma unroll
-        for (int b = 0; b < kBits; ++b) m[b] = wave_ballot(ext[b] != 0u);
-        uint32_t plo = (uint32_t)vm, phi = (uint32_t)(vm >> 32);
+        for (int r = 0; r < kDownRounds; ++r) {
+            const bool valid =
+                kAll || (first + r * kWave < chunk_count && !(drop_sentinel && (uint64_t)key[r] == kSentinelKey));
+            const uint32_t d = digit(key[r]);
+            // per digit bit: the bit as 0 / all ones (a signed bit-field extract) and the wave's ballot
+            // of it; the lanes that agree with this lane in bit b are ~(ballot ^ ext), folded into the
+            // peer mask with one three-input bitwise operation per half (truth table 0x90:
+            // p & ~(m ^ e))
+            uint32_t ext[kBits];
+            uint64_t m[kBits];
 #pragma unroll
-        for (int b = 0; b < kBits; ++b) {
-            plo = __builtin_amdgcn_bitop3_b32(plo, (uint32_t)m[b], ext[b], 0x90);
-            phi = __builtin_amdgcn_bitop3_b32(phi, (uint32_t)(m[b] >> 32), ext[b], 0x90);
+            for (int b = 0; b < kBits; ++b) {
+                ext[b] = (uint32_t)((int32_t)(d << (31 - b)) >> 31);
+                asm volatile("" : "+v"(ext[b]));  // the ballot compares the extracted bit itself
+            }
+#pragma unroll
+            for (int b = 0; b < kBits; ++b) m[b] = wave_ballot(ext[b] != 0u);
+            const uint64_t vm = kAll ? ~0ull : wave_ballot(valid);
+            uint32_t plo = (uint32_t)vm, phi = (uint32_t)(vm >> 32);
+#pragma unroll
+            for (int b = 0; b < kBits; ++b) {
+                plo = __builtin_amdgcn_bitop3_b32(plo, (uint32_t)m[b], ext[b], 0x90);
+                phi = __builtin_amdgcn_bitop3_b32(phi, (uint32_t)(m[b] >> 32), ext[b], 0x90);
+            }
+            const uint32_t c = cnt_offset(wave, d);
+            const uint32_t before = cnt_at(c);  // read by all lanes before the leader updates
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi(phi, __builtin_amdgcn_mbcnt_lo(plo, before));
+            if (valid && rank == before) cnt_at(c) = (CntT)(before + (uint32_t)__popc(plo) + (uint32_t)__popc(phi));
+            __builtin_amdgcn_wave_barrier();
+            dr[r] = valid ? (c << 16) | rank : 0xffffffffu;
+            // formed here, so that the peer masks die with the round (not kept alive for the reorder)
+            asm volatile("" : "+v"(dr[r]));
         }
-        const uint64_t peers = (uint64_t)plo | ((uint64_t)phi << 32);
-        const uint32_t before = cnt(wave, d);  // read by all lanes before the leader updates
-        const uint32_t rank = (uint32_t)__popcll(peers & lt);
-        if (valid && rank == 0) cnt(wave, d) = (CntT)(before + (uint32_t)__popcll(peers));
-        __builtin_amdgcn_wave_barrier();
-        dr[r] = valid ? (d << 16) | (before + rank) : 0xffffffffu;
-        // formed here, so that the peer masks die with the round (not kept alive for the reorder)
-        asm volatile("" : "+v"(dr[r]));
-    }
+    };
+    if (whole) rank_keys(std::true_type{});
+    else rank_keys(std::false_type{});
     __syncthreads();
     // 2. threads 0..255 = digits: wave starts inside the digit, digit starts inside the chunk,
     //    and the digit's output position for this chunk
@@ -401,10 +429,10 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     // 3. reorder the chunk by digit in LDS
 #pragma unroll
     for (int r = 0; r < kDownRounds; ++r) {
-        if (dr[r] != 0xffffffffu) {
-            const uint32_t pos = (uint32_t)cnt(wave, dr[r] >> 16) + (dr[r] & 0xffffu);
+        if (whole || dr[r] != 0xffffffffu) {
+            const uint32_t pos = (uint32_t)cnt_at(dr[r] >> 16) + (dr[r] & 0xffffu);
             if (kPack) {
-                s_kv[pos] = (uint64_t)key[r] | ((uint64_t)val[r] << 32);
+                s_kv[pos] = (EntryT)key[r] | ((EntryT)val[r] << (4 * sizeof(EntryT)));
             } else {
                 s_keys[pos] = key[r];
                 if (kPairs) s_vals[pos] = val[r];
@@ -424,9 +452,9 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     for (int j = 0; j < kOutRounds; ++j) {
         const int i = (int)threadIdx.x + j * kThreads;
         if (kPack) {
-            const uint64_t kv = s_kv[i];
+            const EntryT kv = s_kv[i];
             ok[j] = (KeyT)kv;
-            ov[j] = (uint32_t)(kv >> 32);
+            ov[j] = (uint32_t)(kv >> (4 * sizeof(EntryT))) + (kPackPlace ? (uint32_t)base : 0u);
         } else {
             ok[j] = s_keys[i];
             ov[j] = kPairs ? s_vals[i] : 0u;
@@ -435,12 +463,12 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
 #pragma unroll
     for (int j = 0; j < kOutRounds; ++j) {
         const int i = (int)threadIdx.x + j * kThreads;
-        opos[j] = s_out[digit_of<kBits>(ok[j], shift) & dmask] + (uint32_t)i;
+        opos[j] = s_out[digit(ok[j])] + (uint32_t)i;
     }
 #pragma unroll
     for (int j = 0; j < kOutRounds; ++j) {
         const int i = (int)threadIdx.x + j * kThreads;
-        if (i < kept_count) {
+        if (whole || i < kept_count) {
             if (kNarrow) {
                 *reinterpret_cast<KeyT*>(reinterpret_cast<char*>(keys_out) + (uint32_t)(opos[j] * sizeof(KeyT))) =
                     ok[j];
@@ -648,17 +676,32 @@ gsx_hip_status radix_sort_keys_u64_compacting(uint64_t* keys, uint64_t* keys_alt
                                                                          stream);
 }
 
-template <int kBits, int kChunk, typename TileT>
-gsx_hip_status tile_sort_passes(const TileT* tiles, TileT* tiles_alt, TileT* tiles_sorted, uint32_t* vals_alt,
-                                uint32_t* vals_sorted, int64_t n, int tile_bits, int passes, void* temp,
-                                hipStream_t stream) {
-    constexpr int kBins = 1 << kBits;
-    int64_t chunks = (n + kChunk - 1) / kChunk;
-    if (chunks < 1) chunks = 1;
+// One pass of the tile sort on the kBits bits at `shift` (bits from tile_bits on are 0).
+template <int kBits, int kChunk, typename TileT, bool kFirst>
+void tile_sort_pass(const TileT* kin, const uint32_t* vin, TileT* kout, uint32_t* vout, int64_t n, int tile_bits,
+                    int shift, void* temp, hipStream_t stream) {
+    constexpr int kBins = 1 << kBits, kThreads = kChunk / 8;
+    const int64_t chunks = std::max<int64_t>(1, (n + kChunk - 1) / kChunk);
     const int64_t hist_count = chunks * kBins;
     uint32_t* hist = static_cast<uint32_t*>(temp);
     uint32_t* offsets = hist + hist_count;
     uint32_t* totals = offsets + hist_count;
+    const int width = std::min(kBits, tile_bits - shift);
+    const uint32_t dmask = width > 0 ? (1u << width) - 1u : 0u;
+    hipLaunchKernelGGL((radix_upsweep_kernel<kBits, kChunk, TileT>), dim3(sort_chunk_grid(chunks)),
+                       dim3(kSortThreads), 0, stream, kin, n, nullptr, false, shift, dmask, chunks, hist);
+    launch_rowscan(kBins, hist, chunks, offsets, totals, stream);
+    const auto downsweep = narrow_offsets(n, sizeof(uint32_t))
+                               ? radix_downsweep_kernel<true, kBits, kChunk, TileT, true, kThreads, kFirst>
+                               : radix_downsweep_kernel<true, kBits, kChunk, TileT, false, kThreads, kFirst>;
+    hipLaunchKernelGGL(downsweep, dim3(sort_chunk_grid(chunks)), dim3(kThreads), 0, stream, kin, vin, n, nullptr, false,
+                       shift, dmask, chunks, offsets, totals, kout, vout, nullptr);
+}
+
+template <int kBits, int kChunk, typename TileT>
+gsx_hip_status tile_sort_passes(const TileT* tiles, TileT* tiles_alt, TileT* tiles_sorted, uint32_t* vals_alt,
+                                uint32_t* vals_sorted, int64_t n, int tile_bits, int passes, void* temp,
+                                hipStream_t stream) {
     const TileT* kin = tiles;
     const uint32_t* vin = nullptr;  // first pass: the values are the input positions
     for (int k = 0; k < passes; ++k) {
@@ -667,19 +710,15 @@ gsx_hip_status tile_sort_passes(const TileT* tiles, TileT* tiles_alt, TileT* til
         TileT* kout = to_sorted ? tiles_sorted : tiles_alt;
         uint32_t* vout = to_sorted ? vals_sorted : vals_alt;
         const int shift = k * kBits;
-        const int width = tile_bits - shift < kBits ? tile_bits - shift : kBits;
-        const uint32_t dmask = width > 0 ? (1u << width) - 1u : 0u;
-        hipLaunchKernelGGL((radix_upsweep_kernel<kBits, kChunk, TileT>), dim3(sort_chunk_grid(chunks)),
-                           dim3(kSortThreads), 0, stream, kin, n, nullptr, false, shift, dmask, chunks, hist);
-        launch_rowscan(kBins, hist, chunks, offsets, totals, stream);
-        if (narrow_offsets(n, sizeof(uint32_t))) {
-            hipLaunchKernelGGL((radix_downsweep_kernel<true, kBits, kChunk, TileT, true, kChunk / 8>),
-                               dim3(sort_chunk_grid(chunks)), dim3(kChunk / 8), 0, stream, kin, vin, n, nullptr,
-                               false, shift, dmask, chunks, offsets, totals, kout, vout, nullptr);
+        // a last pass with a bit less to sort takes the narrower kernel (a ballot and two mask operations a
+        // key fewer, half the digits)
+        constexpr int kLess = kBits > 6 ? kBits - 1 : kBits;
+        if (k == 0) {
+            tile_sort_pass<kBits, kChunk, TileT, true>(kin, vin, kout, vout, n, tile_bits, shift, temp, stream);
+        } else if (tile_bits - shift <= kLess) {
+            tile_sort_pass<kLess, kChunk, TileT, false>(kin, vin, kout, vout, n, tile_bits, shift, temp, stream);
         } else {
-            hipLaunchKernelGGL((radix_downsweep_kernel<true, kBits, kChunk, TileT, false, kChunk / 8>),
-                               dim3(sort_chunk_grid(chunks)), dim3(kChunk / 8), 0, stream, kin, vin, n, nullptr,
-                               false, shift, dmask, chunks, offsets, totals, kout, vout, nullptr);
+            tile_sort_pass<kBits, kChunk, TileT, false>(kin, vin, kout, vout, n, tile_bits, shift, temp, stream);
         }
         kin = kout;
         vin = vout;

@@ -11,7 +11,8 @@ torch = pytest.importorskip("torch")
 
 
 @pytest.mark.parametrize("width,height,n", [(16, 16, 40), (4081, 4096, 500), (4096, 4096, 500), (4097, 4096, 500),
-                                            (9000, 2000, 300)])
+                                            (9000, 2000, 300),
+                                            (2800, 2800, 3000)])  # 15 bits: a pass of 8 and one of 7
 def test_sorted_tiles_around_the_narrow_limit(oracle, width, height, n):
     from gsx_amd import scenes
     from gsx_amd.backend import Camera, GaussianTensors, Renderer
