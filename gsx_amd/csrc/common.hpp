@@ -539,7 +539,7 @@ template <int kBits, int kChunk, typename KeyT>
 __device__ inline void radix_upsweep_block(uint32_t blk, const KeyT* __restrict__ keys, int64_t n,
                                            const uint32_t* __restrict__ n_dev, bool drop_sentinel, int shift,
                                            int64_t num_chunks, uint32_t* __restrict__ hist,
-                                           uint32_t* s_hist, uint32_t dmask = (1u << kBits) - 1u) {
+                                           uint32_t* s_hist, uint32_t dmask, bool by_chunk) {
     constexpr int kBins = 1 << kBits;
     constexpr int kCopies = kUpsweepCopies<kBits>;
     constexpr int kCopyWords = kUpsweepCopyWords<kBits>;
@@ -588,7 +588,7 @@ __device__ inline void radix_upsweep_block(uint32_t blk, const KeyT* __restrict_
         uint32_t c = 0;
 #pragma unroll
         for (int h = 0; h < kChunkWaves * kCopies; ++h) c += s_hist[h * kCopyWords + d];
-        hist[(int64_t)d * num_chunks + blk] = c;
+        hist[by_chunk ? (int64_t)blk * kBins + d : (int64_t)d * num_chunks + blk] = c;
     }
 }
 

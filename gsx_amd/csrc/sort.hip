@@ -140,6 +140,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_downsweep_kernel(const uint
 // three passes for 27 depth bits), reduce-then-scan, three launches:
 //   upsweep: digit counts of each chunk (4096 keys, 2048 in the depth order) -> hist[digit][chunk]
 //   rowscan: one workgroup per digit scans its row over the chunks    -> offsets, totals[digit]
+//      (not for a few chunks, see kDirectChunks)
 //   downsweep: 8 waves each rank an eighth of the chunk (rounds of 64 keys) stably with kBits
 //      ballots per round and wave-private digit counters; the chunk is then reordered by digit
 //      in LDS and written out in order, so consecutive lanes store consecutive addresses of one
@@ -155,12 +156,12 @@ __global__ __launch_bounds__(kSortThreads) void radix_upsweep_kernel(const KeyT*
                                                                      const uint32_t* __restrict__ n_dev,
                                                                      bool drop_sentinel, int shift,
                                                                      uint32_t dmask, int64_t num_chunks,
-                                                                     uint32_t* __restrict__ hist) {
+                                                                     bool by_chunk, uint32_t* __restrict__ hist) {
     __shared__ uint32_t s_hist[kUpsweepHistWords<kBits>];
     const int64_t chunk = sort_chunk_of(blockIdx.x, num_chunks);
     if (chunk >= num_chunks) return;  // uniform
     radix_upsweep_block<kBits, kChunk, KeyT>((uint32_t)chunk, keys, n, n_dev, drop_sentinel, shift, num_chunks, hist,
-                                             s_hist, dmask);
+                                             s_hist, dmask, by_chunk);
 }
 
 // Workgroup d: exclusive scan of hist[d][0..num_chunks) into offsets[d][..], row total into
@@ -223,6 +224,12 @@ __global__ __launch_bounds__(kThreads) void radix_rowscan_kernel(const uint32_t*
     }
     if (threadIdx.x == 0) totals[blockIdx.x] = carry;
 }
+
+// Up to this many chunks the row scan is left out: the counts are laid out hist[chunk][digit] and each
+// downsweep workgroup adds up those of its digits, a coalesced load per chunk. The launch that it saves
+// takes 4 us whatever its size; the loads cost a downsweep 0.4 us with 2 chunks, 2.3 with 49 and 4.4
+// with 98 (512 digits).
+constexpr int64_t kDirectChunks = 64;
 
 // Row scan launch for `bins` rows of num_chunks counts.
 inline void launch_rowscan(int bins, const uint32_t* hist, int64_t num_chunks, uint32_t* offsets, uint32_t* totals,
@@ -337,8 +344,11 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     // this chunk's digit offsets and the digit totals, loaded with the keys (threads past kBins
     // re-read digit kBins - 1 and ignore it)
     const int td = min((int)threadIdx.x, kBins - 1);
-    const uint32_t my_total = totals[td];
-    const uint32_t my_offset = offsets[(int64_t)td * num_chunks + chunk];
+    uint32_t my_total = 0, my_offset = 0;
+    if (totals != nullptr) {  // uniform
+        my_total = totals[td];
+        my_offset = offsets[(int64_t)td * num_chunks + chunk];
+    }
     for (int i = threadIdx.x; i < kWaves * kHalf; i += kThreads) (&s_cnt32[0][0])[i] = 0;
     __syncthreads();
     // 1. per wave: stable ranks among equal digits (rank = keys of the digit before it in this
@@ -400,6 +410,22 @@ __global__ __launch_bounds__(kThreads, (kPairs && sizeof(KeyT) == 8) ? 4 : 8) vo
     };
     if (whole) rank_keys(std::true_type{});
     else rank_keys(std::false_type{});
+    if (totals == nullptr) {  // uniform: the counts themselves, [chunk][digit] (kDirectChunks)
+        constexpr int kBatch = 16;
+        const int my_chunk = (int)chunk, chunks = (int)num_chunks;
+        if ((int)threadIdx.x < kBins) {
+            for (int c0 = 0; c0 < chunks; c0 += kBatch) {
+                uint32_t v[kBatch];
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) v[j] = offsets[min(c0 + j, chunks - 1) * kBins + td];
+#pragma unroll
+                for (int j = 0; j < kBatch; ++j) {
+                    my_total += c0 + j < chunks ? v[j] : 0u;
+                    my_offset += c0 + j < my_chunk ? v[j] : 0u;
+                }
+            }
+        }
+    }
     __syncthreads();
     // 2. threads 0..255 = digits: wave starts inside the digit, digit starts inside the chunk,
     //    and the digit's output position for this chunk
@@ -517,6 +543,7 @@ gsx_hip_status radix_sort_u64(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt
     uint32_t* hist = static_cast<uint32_t*>(temp);
     uint32_t* offsets = hist + hist_count;
     uint32_t* totals = offsets + hist_count;
+    const bool direct = chunks <= kDirectChunks;
     int in_alt = 0;
     if (n > 0) {
         for (int shift = begin_bit; shift < end_bit; shift += kBits) {
@@ -530,16 +557,18 @@ gsx_hip_status radix_sort_u64(uint64_t* keys, uint32_t* vals, uint64_t* keys_alt
             const int width = end_bit - shift < kBits ? end_bit - shift : kBits;
             const uint32_t dmask = (1u << width) - 1u;
             hipLaunchKernelGGL((radix_upsweep_kernel<kBits, kChunk>), dim3(sort_chunk_grid(chunks)), dim3(kSortThreads),
-                               0, stream, kin, n, live, drop, shift, dmask, chunks, hist);
-            launch_rowscan(kBins, hist, chunks, offsets, totals, stream);
+                               0, stream, kin, n, live, drop, shift, dmask, chunks, direct, hist);
+            if (!direct) launch_rowscan(kBins, hist, chunks, offsets, totals, stream);
             if (narrow_offsets(n, sizeof(uint64_t))) {
                 hipLaunchKernelGGL((radix_downsweep_kernel<kPairs, kBits, kChunk, uint64_t, true>),
                                    dim3(sort_chunk_grid(chunks)), dim3(kDownThreads), 0, stream, kin, vin, n, live,
-                                   drop, shift, dmask, chunks, offsets, totals, kout, vout, drop ? n_dev : nullptr);
+                                   drop, shift, dmask, chunks, direct ? hist : offsets, direct ? nullptr : totals, kout,
+                                   vout, drop ? n_dev : nullptr);
             } else {
                 hipLaunchKernelGGL((radix_downsweep_kernel<kPairs, kBits, kChunk, uint64_t, false>),
                                    dim3(sort_chunk_grid(chunks)), dim3(kDownThreads), 0, stream, kin, vin, n, live,
-                                   drop, shift, dmask, chunks, offsets, totals, kout, vout, drop ? n_dev : nullptr);
+                                   drop, shift, dmask, chunks, direct ? hist : offsets, direct ? nullptr : totals, kout,
+                                   vout, drop ? n_dev : nullptr);
             }
             in_alt ^= 1;
         }
@@ -686,16 +715,17 @@ void tile_sort_pass(const TileT* kin, const uint32_t* vin, TileT* kout, uint32_t
     uint32_t* hist = static_cast<uint32_t*>(temp);
     uint32_t* offsets = hist + hist_count;
     uint32_t* totals = offsets + hist_count;
+    const bool direct = chunks <= kDirectChunks;
     const int width = std::min(kBits, tile_bits - shift);
     const uint32_t dmask = width > 0 ? (1u << width) - 1u : 0u;
     hipLaunchKernelGGL((radix_upsweep_kernel<kBits, kChunk, TileT>), dim3(sort_chunk_grid(chunks)),
-                       dim3(kSortThreads), 0, stream, kin, n, nullptr, false, shift, dmask, chunks, hist);
-    launch_rowscan(kBins, hist, chunks, offsets, totals, stream);
+                       dim3(kSortThreads), 0, stream, kin, n, nullptr, false, shift, dmask, chunks, direct, hist);
+    if (!direct) launch_rowscan(kBins, hist, chunks, offsets, totals, stream);
     const auto downsweep = narrow_offsets(n, sizeof(uint32_t))
                                ? radix_downsweep_kernel<true, kBits, kChunk, TileT, true, kThreads, kFirst>
                                : radix_downsweep_kernel<true, kBits, kChunk, TileT, false, kThreads, kFirst>;
     hipLaunchKernelGGL(downsweep, dim3(sort_chunk_grid(chunks)), dim3(kThreads), 0, stream, kin, vin, n, nullptr, false,
-                       shift, dmask, chunks, offsets, totals, kout, vout, nullptr);
+                       shift, dmask, chunks, direct ? hist : offsets, direct ? nullptr : totals, kout, vout, nullptr);
 }
 
 template <int kBits, int kChunk, typename TileT>

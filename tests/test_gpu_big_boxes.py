@@ -10,16 +10,18 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 
-# (n, big ones): a workgroup lists 256 ranks, and a search step compares 64 workgroups
+# (n, big ones): a workgroup lists 256 ranks, and a search step compares 64 workgroups; the depth sort
+# scans its counts in a launch of its own from 65 chunks of 2048 on
 @pytest.mark.parametrize("n,big", [(1, 1), (255, 3), (257, 257), (5000, 70), (64 * 256 + 300, 4), (64 * 256, 0),
-                                   (66 * 256 + 1, 130), (20000, 19900)])
+                                   (66 * 256 + 1, 130), (20000, 19900),
+                                   (64 * 2048, 2), (64 * 2048 + 1, 2)])
 def test_big_boxes(oracle, n, big):
     from gsx_amd import scenes
     from gsx_amd.backend import Camera, GaussianTensors, Renderer
     w = scenes.config0(n=n, width=1601, height=1200)
     w.scene.logscale[:] = -6.0 + 0.1 * np.random.default_rng(n).normal(size=w.scene.logscale.shape)
     which = np.random.default_rng(n + 1).choice(n, big, replace=False)
-    w.scene.logscale[which] = 0.5 if n < 20000 else -0.9  # (from 16384 on, waves take several)
+    w.scene.logscale[which] = 0.5 if n != 20000 else -0.9  # (from 16384 on, waves take several)
     w.scene.opacity[which] = -3.0
     cam, g = Camera.from_block(w.camera), GaussianTensors.from_scene(w.scene)
     print(f"[case] big boxes n={n} big={big}", flush=True)
