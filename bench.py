@@ -58,15 +58,15 @@ def algorithmic_bytes(stage, geo, train=True):
         return 8 * n + 12 * vp
     if stage == "emit":
         # per depth rank: count, Gaussian in, offset out; the geometry record of each Gaussian
-        # with tiles in; per instance its tile (4 B) and its Gaussian (4 B) out
-        return 12 * vp + 32 * v + 8 * i
+        # with tiles in; per instance its tile (2 or 4 B) and its Gaussian (4 B) out
+        return 12 * vp + 32 * v + (tile_index_bytes(t) + 4) * i
     if stage == "sort":
-        return sort_bytes(geo["S"], i)
+        return sort_bytes(geo["S"], i, t)
     if stage == "ranges":
         if i >= RANGES_SEARCH_MIN:
-            # per tile two binary searches of ceil(log2(I + 1)) 4-byte probes, one range out
-            return t * (8 * int(i).bit_length() + 8)
-        return 4 * i + 8 * t  # sorted tiles in, one range per tile out
+            # per tile two binary searches of ceil(log2(I + 1)) probes, one range out
+            return t * (2 * tile_index_bytes(t) * int(i).bit_length() + 8)
+        return tile_index_bytes(t) * i + 8 * t  # sorted tiles in, one range per tile out
     if stage == "blend_forward":
         # ranges, reached entries' positions + Gaussians in, each reached Gaussian's record once;
         # image (12 B) + final T + last position out; TRAIN: each reached entry's Gaussian and the
@@ -84,7 +84,7 @@ def algorithmic_bytes(stage, geo, train=True):
         # Gaussians' instances and the reached entries' partials in (the 9-float screen gradients
         # of the touched Gaussians stay in L2 for the projection backward: the counters show no
         # writes, so they are not counted)
-        return 9 * vp + 4 * geo["It"] + 36 * r
+        return 9 * vp + tile_index_bytes(t) * geo["It"] + 36 * r
     if stage == "projection_backward":
         # every Gaussian's touched flag in, the five parameter gradients of the reached Gaussians
         # out (the blend backward has zeroed the others; the reached ones' inputs and screen
@@ -105,13 +105,18 @@ def algorithmic_bytes(stage, geo, train=True):
 RANGES_SEARCH_MIN = 1 << 25
 
 
-def sort_bytes(passes, instances):
-    """Bytes the tile sort moves: per pass each 4-byte tile is read twice (digit counts, then
-    scatter) and written once with its 4-byte position; the first pass reads no positions (they
-    are the input order), the later ones read them once."""
+def tile_index_bytes(tiles):
+    """Bytes the path keeps a tile index in."""
+    return 2 if tiles <= 65536 else 4
+
+
+def sort_bytes(passes, instances, tiles):
+    """HBM bytes the tile sort of `instances` tiles moves in `passes` passes: per pass the tiles in
+    twice (counts, then reorder) and tiles and positions out; positions in from the second pass on."""
     if passes <= 0:
         return 0
-    return instances * (16 * passes + 4 * (passes - 1))
+    width = tile_index_bytes(tiles)
+    return (passes * (3 * width + 4) + (passes - 1) * 4) * instances
 
 
 def render_geometry(lib, renderer, n, width, height):
@@ -735,7 +740,7 @@ def _config4(lib, steps):
     c4 = config_measurement(runner, inputs, 1, max(2, steps // 4))
     st = runner.renderer.stats()
     inst = int(st.instance_count)
-    moved = sort_bytes(int(st.sort_passes), inst)
+    moved = sort_bytes(int(st.sort_passes), inst, int(st.tile_count))
     sort_ms = c4["stage_ms"]["sort"]
     out["c4_sort_stress"] = {"gaussians": w.scene.count, "width": 1920, "height": 1080, **c4, "instances": inst,
                              "sort_passes": int(st.sort_passes),
