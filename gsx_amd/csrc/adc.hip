@@ -895,12 +895,33 @@ RowSet moment_rows(const gsx_hip_gs_rows& r) {
 struct gsx_hip_adc_context {
     gsx_amd_pcg32 rng;
     Scratch scratch;
-    uint32_t* host = nullptr;  // pinned counts that kernels write through host_dev
+    uint32_t* host = nullptr;  // pinned counts that kernels of any device write through host_dev
     uint32_t* host_dev = nullptr;
     hipEvent_t counted = nullptr;  // recorded behind the kernel that writes them
+    int counted_device = -1;       // the device it belongs to
 };
 
 namespace {
+
+// Makes ctx->counted an event of the current device. An event goes with one device and a context with
+// none: it may be stepped on another device than it was made on.
+hipError_t make_counted(gsx_hip_adc_context* ctx) {
+    int device = 0;
+    hipError_t e = hipGetDevice(&device);
+    if (e != hipSuccess || device == ctx->counted_device) return e;
+    if (ctx->counted != nullptr) (void)hipEventDestroy(ctx->counted);
+    ctx->counted = nullptr;
+    ctx->counted_device = -1;
+    e = hipEventCreateWithFlags(&ctx->counted, hipEventDisableTiming);
+    if (e == hipSuccess) ctx->counted_device = device;
+    return e;
+}
+
+gsx_hip_status record_counted(gsx_hip_adc_context* ctx, hipStream_t stream) {
+    ADC_HIP_TRY(make_counted(ctx));
+    ADC_HIP_TRY(hipEventRecord(ctx->counted, stream));
+    return GSX_HIP_SUCCESS;
+}
 
 // MCMC position noise (gsx/src/gsx-cpu/adc/mcmc.c:345-451): none past end_refine or without
 // noise strength; otherwise 6 draws per Gaussian from the context's stream.
@@ -1039,7 +1060,7 @@ gsx_hip_status mcmc_refine(gsx_hip_adc_context* ctx, const gsx_hip_adc_params& p
     ADC_HIP_TRY(hipGetLastError());
     // the scans' totals go straight to host memory: [0] dead rows, [1] live rows with a positive weight
     ADC_TRY(scan_partials_in_place(partials, blocks, stream, 2, ctx->host_dev));
-    ADC_HIP_TRY(hipEventRecord(ctx->counted, stream));
+    ADC_TRY(record_counted(ctx, stream));
     ADC_HIP_TRY(hipEventSynchronize(ctx->counted));
     const int64_t dead_count = ctx->host[0];
     out_counts[0] = dead_count;
@@ -1094,9 +1115,10 @@ gsx_hip_status gsx_hip_adc_context_create(gsx_hip_adc_context** out, uint64_t se
     if (ctx == nullptr) return adc_fail(GSX_HIP_ERROR_OUT_OF_MEMORY, "adc context allocation");
     // gsx_pcg32_init(seed) -> pcg32_init(seed, seed) (gsx/src/gsx-random.c:25, gsx-cpu/adc.c:466)
     gsx_pcg32_seed2(&ctx->rng, seed, seed);
-    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&ctx->host), 4 * sizeof(uint32_t), hipHostMallocDefault);
+    hipError_t e = hipHostMalloc(reinterpret_cast<void**>(&ctx->host), 4 * sizeof(uint32_t),
+                                 hipHostMallocPortable | hipHostMallocMapped);
     if (e == hipSuccess) e = hipHostGetDevicePointer(reinterpret_cast<void**>(&ctx->host_dev), ctx->host, 0);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->counted, hipEventDisableTiming);
+    if (e == hipSuccess) e = make_counted(ctx);
     if (e != hipSuccess) {
         (void)gsx_hip_adc_context_destroy(ctx);
         return adc_fail((gsx_hip_status)e, "adc context creation");
@@ -1196,7 +1218,7 @@ gsx_hip_status gsx_hip_adc_step(gsx_hip_adc_context* ctx, const gsx_hip_adc_para
                            keep_partials);
         ADC_HIP_TRY(hipGetLastError());
         ADC_TRY(scan_partials_in_place(keep_partials, keep_blocks, stream, 1, ctx->host_dev + 2));
-        ADC_HIP_TRY(hipEventRecord(ctx->counted, stream));
+        ADC_TRY(record_counted(ctx, stream));
         // out rows that cannot take the result are an error only if rows are pruned
         const bool out_bound = out->mean3d != nullptr && out->rotation != nullptr && out->logscale != nullptr &&
                                out->opacity != nullptr && out->sh0 != nullptr;

@@ -1,0 +1,78 @@
+"""What the library's host code asks of HIP, on a stand-in for the runtime (fake_hip.c) in a process of its
+own: no GPU is needed or touched, and kernels are counted, not run."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes, os, sys
+sys.path.insert(0, {root!r})
+from gsx_amd import _lib
+fake = ctypes.CDLL({fake!r})
+fake.fake_threads_of.restype = ctypes.c_uint64
+lib = _lib.load(require_device=False)
+P = 0x7000000000  # an address on the device
+"""
+
+
+@pytest.fixture(scope="module")
+def host(tmp_path_factory):
+    """Runs a piece of Python against the library on the stand-in runtime."""
+    fake = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    subprocess.run(["gcc", "-std=c11", "-O1", "-fPIC", "-shared", "-Wall", "-o", fake,
+                    os.path.join(ROOT, "tests", "fake_hip.c")], check=True)
+    preload = ":".join([fake] + ([os.environ["LD_PRELOAD"]] if os.environ.get("LD_PRELOAD") else []))
+
+    def run(code):
+        text = PRELUDE.format(root=ROOT, fake=fake) + textwrap.dedent(code)
+        res = subprocess.run([sys.executable, "-c", text], env={**os.environ, "LD_PRELOAD": preload},
+                             capture_output=True, text=True, timeout=120)
+        assert res.returncode == 0, res.stdout + res.stderr
+    return run
+
+
+ROWS = """
+def rows(count):
+    r = _lib.GsRows()
+    r.count, r.sh_degree = count, 0
+    for f in ("mean3d", "rotation", "logscale", "opacity", "sh0", "grad_acc"):
+        setattr(r, f, P)
+    return r
+
+def step(handle, algorithm, count, capacity, stream=None, out=None, **more):
+    p = _lib.AdcParams()
+    p.algorithm, p.scene_scale, p.refine_every, p.end_refine = algorithm, 1.0, 100, 1000
+    p.max_num_gaussians = capacity
+    for k, v in more.items():
+        setattr(p, k, v)
+    r, o = rows(count), out if out is not None else rows(count)
+    in_out, counts = ctypes.c_int32(0), (ctypes.c_int64 * 4)()
+    _lib.check(lib.gsx_hip_adc_step(handle, ctypes.byref(p), 100, ctypes.byref(r), capacity, ctypes.byref(o),
+                                    ctypes.byref(in_out), counts, stream), "adc step")
+    return r.count, list(counts)
+
+def context():
+    h = ctypes.c_void_p()
+    _lib.check(lib.gsx_hip_adc_context_create(ctypes.byref(h), 3), "create")
+    return h
+"""
+
+
+@pytest.mark.parametrize("algorithm", [0, 2])
+def test_a_density_control_steps_on_another_device(host, algorithm):
+    """Made while device 0 is current and stepped on a stream and the null stream of device 1."""
+    host(ROWS + f"""
+h = context()
+fake.fake_set_totals(1, 1)
+fake.hipSetDevice(1)
+stream = ctypes.c_void_p()
+fake.hipStreamCreateWithFlags(ctypes.byref(stream), 0)
+step(h, {algorithm}, 1000, 1000, stream)
+step(h, {algorithm}, 1000, 1000, None)
+_lib.check(lib.gsx_hip_adc_context_destroy(h), "destroy")
+""")
