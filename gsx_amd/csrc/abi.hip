@@ -268,7 +268,6 @@ int bits_for(uint32_t v) {
 
 struct gsx_hip_render_context {
     DeviceBuffer rec, cov_coef, ckpt, inst_gauss, inst_tile, tiles_alt, tiles_sorted, vals_alt, vals, tile_cut, tile_exact, touched,
-        tiles_wide,
         inst_grad, tile_count, big_list, offsets, scan_temp, sort_temp, ranges, sorted_g, final_t, last, grad2d,
         depth_keys, depth_keys_alt, rank_g, rank_count, g_rank, long_list, multi_list, counters,
         depth_sort_temp;
@@ -305,9 +304,9 @@ struct gsx_hip_render_context {
     int32_t depth_sort_passes = 0;
     int32_t tile_bits = 0;            // bits of the tile index the sort orders
     // Tile indices of instances are kept in 16 bits up to kNarrowTiles tiles, else in 32; get_buffers
-    // hands out 32-bit ones (widened into tiles_wide on demand, once per forward)
+    // hands out 32-bit ones, widened once per forward into vals_alt, which the sort needs no more
     bool narrow_tiles = false;
-    int64_t unwidened = 0;  // 16-bit indices the last completed forward sorted and nobody asked for yet
+    mutable int64_t unwidened = 0;  // its 16-bit indices, while nobody has asked for them
     uint32_t* sorted_vals = nullptr;  // emission position of each sorted instance
     bool has_train_state = false;
     // Stage timing: a ring of event sets, one set per forward/backward pair, so that a timed
@@ -443,6 +442,23 @@ gsx_hip_status enqueue_tile_lists(gsx_hip_render_context* ctx, uint32_t big_tota
                            ctx->ranges.as<uint32_t>(), (int64_t)tiles * 2, 0u);
     }
     GSX_HIP_TRY(hipGetLastError(), "tile_ranges_kernel");
+    return GSX_HIP_SUCCESS;
+}
+
+// The last forward's sorted tiles in 32 bits, into vals_alt (no allocation). Behind everything queued
+// (whichever stream the forward took, also one that is gone by now), on the context's own stream, and
+// waited for: the pointer is good for any stream.
+gsx_hip_status widen_sorted_tiles(const gsx_hip_render_context* ctx) {
+    hipError_t e = hipDeviceSynchronize();
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(widen_tiles_kernel, dim3(std::min(blocks_for(ctx->unwidened, 1024), 65536u)), dim3(256), 0,
+                           ctx->check_stream, ctx->tiles_sorted.as<uint16_t>(), ctx->unwidened,
+                           ctx->vals_alt.as<uint32_t>());
+        e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(ctx->check_stream);
+    GSX_HIP_TRY(e, "widen tiles");
+    ctx->unwidened = 0;
     return GSX_HIP_SUCCESS;
 }
 
@@ -642,7 +658,7 @@ gsx_hip_status gsx_hip_render_context_create(gsx_hip_render_context** out_contex
 gsx_hip_status gsx_hip_render_context_destroy(gsx_hip_render_context* ctx) {
     if (ctx == nullptr) return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "context must be non-null");
     DeviceBuffer* all[] = {&ctx->rec,       &ctx->cov_coef, &ctx->ckpt,      &ctx->inst_gauss, &ctx->inst_tile,
-                           &ctx->tiles_alt, &ctx->tiles_sorted, &ctx->vals_alt, &ctx->vals, &ctx->tiles_wide,
+                           &ctx->tiles_alt, &ctx->tiles_sorted, &ctx->vals_alt, &ctx->vals,
                            &ctx->tile_cut,  &ctx->tile_exact, &ctx->touched,  &ctx->inst_grad,
                            &ctx->tile_count, &ctx->big_list, &ctx->offsets,   &ctx->scan_temp,
                            &ctx->sort_temp,  &ctx->ranges,
@@ -1108,22 +1124,10 @@ gsx_hip_status gsx_hip_render_context_get_stats(const gsx_hip_render_context* ct
     return GSX_HIP_SUCCESS;
 }
 
-gsx_hip_status gsx_hip_render_context_get_buffers(const gsx_hip_render_context* context, gsx_hip_render_buffers* out) {
-    if (context == nullptr || out == nullptr) return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "context/out must be non-null");
-    gsx_hip_render_context* ctx = const_cast<gsx_hip_render_context*>(context);  // only its widened copy changes
-    if (ctx->unwidened > 0) {
-        // behind everything queued (whichever stream the forward took, also one that is gone by now), on the
-        // context's own stream, and waited for: the pointer is good for any stream
-        const int64_t count = ctx->unwidened;
-        GSX_HIP_TRY(hipDeviceSynchronize(), "widen tiles sync");
-        GSX_TRY(ctx->tiles_wide.reserve((size_t)count * sizeof(uint32_t), "wide tiles", ctx->check_stream));
-        hipLaunchKernelGGL(widen_tiles_kernel, dim3(std::min(blocks_for(count, 1024), 65536u)), dim3(256), 0,
-                           ctx->check_stream, ctx->tiles_sorted.as<uint16_t>(), count, ctx->tiles_wide.as<uint32_t>());
-        GSX_HIP_TRY(hipGetLastError(), "widen_tiles_kernel");
-        GSX_HIP_TRY(hipStreamSynchronize(ctx->check_stream), "widen tiles sync");
-        ctx->unwidened = 0;
-    }
-    out->sorted_tiles = ctx->narrow_tiles ? ctx->tiles_wide.as<uint32_t>() : ctx->tiles_sorted.as<uint32_t>();
+gsx_hip_status gsx_hip_render_context_get_buffers(const gsx_hip_render_context* ctx, gsx_hip_render_buffers* out) {
+    if (ctx == nullptr || out == nullptr) return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "context/out must be non-null");
+    if (ctx->unwidened > 0) GSX_TRY(widen_sorted_tiles(ctx));
+    out->sorted_tiles = ctx->narrow_tiles ? ctx->vals_alt.as<uint32_t>() : ctx->tiles_sorted.as<uint32_t>();
     out->sorted_values = ctx->sorted_vals;
     out->tile_ranges = ctx->ranges.as<uint32_t>();
     out->records = ctx->rec.as<float>();

@@ -158,9 +158,9 @@ typedef struct gsx_hip_render_stats {
     int32_t sorted_tile_bytes; /* element size of sorted_tiles (4) */
 } gsx_hip_render_stats;
 
-/* Device pointers of the intermediates a forward retains (valid until the next forward). The first
- * get_buffers after a forward of at most 65536 tiles waits for the device: the path keeps tile indices in
- * 16 bits there, and sorted_tiles is written from them. */
+/* Device pointers of the intermediates a forward retains (valid until the next forward). The path keeps
+ * tile indices in 16 bits up to 65536 tiles: the first get_buffers after such a forward waits for the
+ * device and writes sorted_tiles from them, into memory that the context has. */
 typedef struct gsx_hip_render_buffers {
     const uint32_t* sorted_tiles;  /* [instance_count] tile index of each sorted instance */
     const uint32_t* sorted_values; /* [instance_count] emission position of each sorted instance */

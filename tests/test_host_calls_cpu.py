@@ -76,3 +76,43 @@ step(h, {algorithm}, 1000, 1000, stream)
 step(h, {algorithm}, 1000, 1000, None)
 _lib.check(lib.gsx_hip_adc_context_destroy(h), "destroy")
 """)
+
+
+RENDER = """
+def camera():
+    c = _lib.Camera()
+    c.width, c.height, c.fx, c.fy, c.near_plane, c.far_plane = 64, 48, 50.0, 50.0, 0.1, 100.0
+    c.rot[3] = 1.0
+    return c
+
+def gaussians(count):
+    g = _lib.Gaussians()
+    g.count, g.sh_degree = count, 0
+    for f in ("mean3d", "rotation", "logscale", "opacity", "sh0"):
+        setattr(g, f, P)
+    return g
+
+def forward(handle, count, instances):
+    fake.fake_set_kept(instances)
+    return lib.gsx_hip_render_forward(handle, ctypes.byref(camera()), ctypes.byref(gaussians(count)), 0, P, None, None)
+
+def look(handle):
+    b = _lib.RenderBuffers()
+    _lib.check(lib.gsx_hip_render_context_get_buffers(handle, ctypes.byref(b)), "get buffers")
+    return b.sorted_tiles
+
+h = ctypes.c_void_p()
+_lib.check(lib.gsx_hip_render_context_create(ctypes.byref(h)), "create")
+_lib.check(forward(h, 100, 500), "forward")
+"""
+
+
+def test_a_look_at_the_buffers_allocates_nothing(host):
+    host(RENDER + """
+before = fake.fake_allocations()
+assert look(h) and look(h) == look(h)
+assert fake.fake_allocations() == before
+assert fake.fake_launches_of(b"widen_tiles") == 1
+_lib.check(forward(h, 100, 400), "forward")
+assert look(h) and fake.fake_launches_of(b"widen_tiles") == 2
+""")
