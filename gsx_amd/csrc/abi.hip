@@ -16,6 +16,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <mutex>
 #include <new>
 
 #include "../../include/gsx_hip.h"
@@ -306,6 +307,7 @@ struct gsx_hip_render_context {
     // Tile indices of instances are kept in 16 bits up to kNarrowTiles tiles, else in 32; get_buffers
     // hands out 32-bit ones, widened once per forward into vals_alt, which the sort needs no more
     bool narrow_tiles = false;
+    mutable std::mutex widen_mutex;
     mutable int64_t unwidened = 0;  // its 16-bit indices, while nobody has asked for them
     uint32_t* sorted_vals = nullptr;  // emission position of each sorted instance
     bool has_train_state = false;
@@ -1126,7 +1128,10 @@ gsx_hip_status gsx_hip_render_context_get_stats(const gsx_hip_render_context* ct
 
 gsx_hip_status gsx_hip_render_context_get_buffers(const gsx_hip_render_context* ctx, gsx_hip_render_buffers* out) {
     if (ctx == nullptr || out == nullptr) return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "context/out must be non-null");
-    if (ctx->unwidened > 0) GSX_TRY(widen_sorted_tiles(ctx));
+    {
+        std::lock_guard<std::mutex> lock(ctx->widen_mutex);  // several threads may look at a context
+        if (ctx->unwidened > 0) GSX_TRY(widen_sorted_tiles(ctx));
+    }
     out->sorted_tiles = ctx->narrow_tiles ? ctx->vals_alt.as<uint32_t>() : ctx->tiles_sorted.as<uint32_t>();
     out->sorted_values = ctx->sorted_vals;
     out->tile_ranges = ctx->ranges.as<uint32_t>();

@@ -116,3 +116,14 @@ assert fake.fake_launches_of(b"widen_tiles") == 1
 _lib.check(forward(h, 100, 400), "forward")
 assert look(h) and fake.fake_launches_of(b"widen_tiles") == 2
 """)
+
+
+def test_threads_look_at_the_buffers_at_the_same_time(host):
+    host(RENDER + """
+import threading
+seen = []
+threads = [threading.Thread(target=lambda: seen.append(look(h))) for _ in range(4)]
+[t.start() for t in threads], [t.join() for t in threads]
+assert len(set(seen)) == 1 and seen[0]
+assert fake.fake_launches_of(b"widen_tiles") == 1
+""")
