@@ -309,6 +309,7 @@ struct gsx_hip_render_context {
     bool narrow_tiles = false;
     mutable std::mutex widen_mutex;
     mutable int64_t unwidened = 0;  // its 16-bit indices, while nobody has asked for them
+    int device = 0;                 // the device of the context's events and of check_stream
     uint32_t* sorted_vals = nullptr;  // emission position of each sorted instance
     bool has_train_state = false;
     // Stage timing: a ring of event sets, one set per forward/backward pair, so that a timed
@@ -449,8 +450,11 @@ gsx_hip_status enqueue_tile_lists(gsx_hip_render_context* ctx, uint32_t big_tota
 
 // The last forward's sorted tiles in 32 bits, into vals_alt (no allocation). Behind everything queued
 // (whichever stream the forward took, also one that is gone by now), on the context's own stream, and
-// waited for: the pointer is good for any stream.
+// waited for: the pointer is good for any stream, and for the thread of another device.
 gsx_hip_status widen_sorted_tiles(const gsx_hip_render_context* ctx) {
+    int device = 0;
+    GSX_HIP_TRY(hipGetDevice(&device), "hipGetDevice");
+    if (device != ctx->device) GSX_HIP_TRY(hipSetDevice(ctx->device), "hipSetDevice");
     hipError_t e = hipDeviceSynchronize();
     if (e == hipSuccess) {
         hipLaunchKernelGGL(widen_tiles_kernel, dim3(std::min(blocks_for(ctx->unwidened, 1024), 65536u)), dim3(256), 0,
@@ -459,6 +463,10 @@ gsx_hip_status widen_sorted_tiles(const gsx_hip_render_context* ctx) {
         e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->check_stream);
+    if (device != ctx->device) {
+        const hipError_t back = hipSetDevice(device);
+        if (e == hipSuccess) e = back;
+    }
     GSX_HIP_TRY(e, "widen tiles");
     ctx->unwidened = 0;
     return GSX_HIP_SUCCESS;
@@ -643,7 +651,8 @@ gsx_hip_status gsx_hip_render_context_create(gsx_hip_render_context** out_contex
     *out_context = nullptr;
     gsx_hip_render_context* ctx = new (std::nothrow) gsx_hip_render_context();
     if (ctx == nullptr) return fail(GSX_HIP_ERROR_OUT_OF_MEMORY, "render context allocation failed");
-    hipError_t e = hipEventCreateWithFlags(&ctx->count_ev, hipEventDisableTiming);
+    hipError_t e = hipGetDevice(&ctx->device);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->count_ev, hipEventDisableTiming);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ctx->state_ev, hipEventDisableTiming);
     // fork_ev only orders the comparison's stream after the caller's (device-side): no
     // system-scope fence (its cache flush would idle the GPU before every borrowed backward)

@@ -127,3 +127,13 @@ threads = [threading.Thread(target=lambda: seen.append(look(h))) for _ in range(
 assert len(set(seen)) == 1 and seen[0]
 assert fake.fake_launches_of(b"widen_tiles") == 1
 """)
+
+
+def test_a_look_at_the_buffers_from_another_device(host):
+    host(RENDER + """
+fake.hipSetDevice(1)
+assert look(h)
+device = ctypes.c_int()
+fake.hipGetDevice(ctypes.byref(device))
+assert device.value == 1
+""")
