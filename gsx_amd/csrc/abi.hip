@@ -307,6 +307,7 @@ struct gsx_hip_render_context {
     // Tile indices of instances are kept in 16 bits up to kNarrowTiles tiles, else in 32; get_buffers
     // hands out 32-bit ones, widened once per forward into vals_alt, which the sort needs no more
     bool narrow_tiles = false;
+    bool listed = false;            // the last forward got as far as its sorted lists
     mutable std::mutex widen_mutex;
     mutable int64_t unwidened = 0;  // its 16-bit indices, while nobody has asked for them
     int device = 0;                 // the device of the context's events and of check_stream
@@ -781,6 +782,8 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
         return fail(GSX_HIP_ERROR_INVALID_ARGUMENT, "forward type must be a GSX_HIP_FORWARD_* value");
     }
     ctx->has_train_state = false;
+    ctx->listed = false;
+    ctx->unwidened = 0;
     ctx->call_stream = stream;
     const CameraParams cam = make_camera_params(*camera);
     const int64_t n = gaussians->count;
@@ -914,7 +917,6 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     // per instance: its tile (emission order, the sort's input, kept for the backward), the middle
     // pass's tiles and positions, the sorted tiles and positions, its Gaussian
     ctx->narrow_tiles = tiles <= kNarrowTiles;
-    ctx->unwidened = 0;
     const size_t tile_bytes = ctx->narrow_tiles ? sizeof(uint16_t) : sizeof(uint32_t);
     GSX_TRY(ctx->inst_tile.reserve(c1 * tile_bytes, "instance_tile", ctx->call_stream));
     GSX_TRY(ctx->tiles_alt.reserve(c1 * tile_bytes, "tiles_alt", ctx->call_stream));
@@ -933,6 +935,7 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
     const unsigned emit_blocks = std::min(pre_blocks, (unsigned)(visible_total / 256u + 1u));
     GSX_TRY(ctx->narrow_tiles ? enqueue_tile_lists<uint16_t>(ctx, (uint32_t)big_total, emit_blocks, pre_blocks, stream)
                               : enqueue_tile_lists<uint32_t>(ctx, (uint32_t)big_total, emit_blocks, pre_blocks, stream));
+    ctx->listed = true;
     if (ctx->narrow_tiles) ctx->unwidened = count;
     GSX_TRY(record(ctx, 5, stream));
     const int tiles_padded = ((tiles + 7) / 8) * 8;
@@ -1141,7 +1144,9 @@ gsx_hip_status gsx_hip_render_context_get_buffers(const gsx_hip_render_context* 
         std::lock_guard<std::mutex> lock(ctx->widen_mutex);  // several threads may look at a context
         if (ctx->unwidened > 0) GSX_TRY(widen_sorted_tiles(ctx));
     }
-    out->sorted_tiles = ctx->narrow_tiles ? ctx->vals_alt.as<uint32_t>() : ctx->tiles_sorted.as<uint32_t>();
+    out->sorted_tiles = !ctx->listed       ? nullptr
+                        : ctx->narrow_tiles ? ctx->vals_alt.as<uint32_t>()
+                                            : ctx->tiles_sorted.as<uint32_t>();
     out->sorted_values = ctx->sorted_vals;
     out->tile_ranges = ctx->ranges.as<uint32_t>();
     out->records = ctx->rec.as<float>();

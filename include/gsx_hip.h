@@ -161,7 +161,7 @@ typedef struct gsx_hip_render_stats {
 /* Device pointers of the intermediates a forward retains (valid until the next forward). The path keeps
  * tile indices in 16 bits up to 65536 tiles: the first get_buffers after such a forward waits for the
  * device and writes sorted_tiles from them, into memory that the context has. Threads may look at one
- * context at the same time. */
+ * context at the same time. sorted_tiles is null after a forward that failed before its lists stood. */
 typedef struct gsx_hip_render_buffers {
     const uint32_t* sorted_tiles;  /* [instance_count] tile index of each sorted instance */
     const uint32_t* sorted_values; /* [instance_count] emission position of each sorted instance */

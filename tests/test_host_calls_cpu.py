@@ -137,3 +137,16 @@ device = ctypes.c_int()
 fake.hipGetDevice(ctypes.byref(device))
 assert device.value == 1
 """)
+
+
+def test_no_sorted_tiles_of_an_earlier_forward(host):
+    """A forward that runs out of memory behind its count leaves no sorted tiles, rather than the last one's."""
+    host(RENDER + """
+assert look(h)
+fake.fake_set_no_memory(1)
+assert forward(h, 100, 1 << 30) == _lib.ERROR_OUT_OF_MEMORY
+assert not look(h)
+fake.fake_set_no_memory(0)
+_lib.check(forward(h, 100, 500), "forward")
+assert look(h)
+""")
