@@ -453,15 +453,21 @@ __global__ __launch_bounds__(kAdcThreads) void mcmc_count_kernel(int64_t draws, 
 // starts from, and pairs compose associatively. m only grows: if it ends below 2^24 it never left
 // the binade, and the pair gave every sum exactly; otherwise the addition that leaves it is made in
 // float and the chain goes on in the next binade (at most some 24 times).
+// Totals below 2^-125 count as the binade k = -126 whatever their first bit: m is then below 2^23, the
+// weights are whole ulps and nothing is rounded.
 //  1. float_sum_maps_kernel: the pair of every 1024-element chunk for each binade from kSumLowest up.
 //  2. float_sum_starts_kernel (one workgroup): the total before every chunk, by scans over the chunks'
-//     pairs up to the chunk that leaves the binade, whose sum one wave forms.
+//     pairs up to the chunk that leaves the binade, whose sum one wave forms. Below kSumLowest the
+//     workgroup forms the pairs of its next 16 chunks itself, a wave each: only weights that are
+//     tiny for thousands of rows stay there, and the maps of all binades would cost every other sum
+//     four times step 1. (A refine of 1M rows of weight 1e-13: 0.56 ms; one chunk after the other
+//     2.69, on the host 0.80.)
 //  3. float_sums_kernel: every chunk's sums from its start.
 // 1M weights: 0.14 ms on the device instead of 0.9 ms for the copy out, a host loop and the copy back.
 constexpr int kSumItems = 16;                   // elements per lane
 constexpr int kSumChunk = kSumItems * kWave;    // elements per chunk, one wave
 constexpr uint32_t kSumLimit = 1u << 24;        // m from which the total has left the binade
-constexpr int kSumLowest = -12;                 // lowest binade with pairs (below, chunk by chunk)
+constexpr int kSumLowest = -12;                 // lowest binade whose pairs are formed beforehand
 
 struct SumMap {
     uint32_t even, odd;  // what m grows by from an even and from an odd start, at most kSumLimit
@@ -486,10 +492,16 @@ __device__ inline SumMap sum_map_of(float w, float scale) {
     return SumMap{r, r};
 }
 
-__device__ inline float sum_scale(int k) { return __uint_as_float((uint32_t)(127 + 23 - k) << 23); }
-__device__ inline float sum_value(uint32_t m, int k) {  // m 2^(k-23), m in [2^23, 2^24)
-    return __uint_as_float(((uint32_t)(k + 127) << 23) | (m & 0x7fffffu));
+// k and m of a total (m 2^(k-23)), and the total of an m below 2^24
+__device__ inline int sum_binade(float total) { return max((int)(__float_as_uint(total) >> 23), 1) - 127; }
+__device__ inline uint32_t sum_mantissa(float total, int k) {
+    return __float_as_uint(total) - ((uint32_t)(k + 126) << 23);
 }
+__device__ inline float sum_value(uint32_t m, int k) { return __uint_as_float(((uint32_t)(k + 126) << 23) + m); }
+
+// 1 / ulp of binade k, divided by sum_prescale(k) where it would be above the largest float
+__device__ inline float sum_prescale(int k) { return k < -100 ? 0x1p64f : 1.0f; }
+__device__ inline float sum_scale(int k) { return __uint_as_float((uint32_t)(127 + 23 - k - (k < -100 ? 64 : 0)) << 23); }
 
 // Inclusive composition over the lanes of a wave, lane 0 first.
 __device__ inline SumMap wave_sum_scan(SumMap m) {
@@ -504,15 +516,25 @@ __device__ inline SumMap wave_sum_scan(SumMap m) {
     return m;
 }
 
-// The lane's 16 weights of a chunk, negative ones, NaN and those past count as 0.
+// The lane's 16 weights of a chunk, negative ones, NaN and those past count as 0. weight is 16-byte
+// aligned: with single-float loads, whose lanes lie 64 bytes apart, a step of the sums below kSumLowest
+// spent 8 of its 10 us on addresses.
 __device__ inline void load_sum_chunk(const float* __restrict__ weight, int64_t count, int64_t chunk,
                                       float (&w)[kSumItems]) {
     const int64_t first = chunk * kSumChunk + (int64_t)__lane_id() * kSumItems;
+    if (first + kSumItems <= count) {
+        const float4* const from = reinterpret_cast<const float4*>(weight + first);
 #pragma unroll
-    for (int i = 0; i < kSumItems; ++i) {
-        const float v = first + i < count ? weight[first + i] : 0.0f;
-        w[i] = v > 0.0f ? v : 0.0f;
+        for (int i = 0; i < kSumItems; i += 4) {
+            const float4 v = from[i / 4];
+            w[i] = v.x, w[i + 1] = v.y, w[i + 2] = v.z, w[i + 3] = v.w;
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < kSumItems; ++i) w[i] = first + i < count ? weight[first + i] : 0.0f;
     }
+#pragma unroll
+    for (int i = 0; i < kSumItems; ++i) w[i] = w[i] > 0.0f ? w[i] : 0.0f;
 }
 
 // The sums of a chunk whose lanes hold 16 weights each, from `total`: the lane's own in out, the last
@@ -521,35 +543,31 @@ __device__ inline float sum_chunk(float total, const float (&w)[kSumItems], floa
     const int lane = (int)__lane_id();
     int from = 0;  // lanes before it are done
     while (from < kWave) {
-        const uint32_t bits = __float_as_uint(total);
-        const int k = (int)(bits >> 23) - 127;
-        int next = from;  // the lane to sum in float
-        if (k > -100 && k < 100) {
-            const float scale = sum_scale(k);
-            const uint32_t m0 = (bits & 0x7fffffu) | 0x800000u;
-            SumMap map{0u, 0u};
+        const int k = sum_binade(total);
+        const float pre = sum_prescale(k), scale = sum_scale(k);
+        const uint32_t m0 = sum_mantissa(total, k);
+        SumMap map{0u, 0u};
 #pragma unroll
-            for (int i = 0; i < kSumItems; ++i) map = sum_then(map, sum_map_of(w[i], scale));
-            if (lane < from) map = SumMap{0u, 0u};
-            const SumMap incl = wave_sum_scan(map);
-            const uint32_t end = m0 + ((m0 & 1u) != 0u ? incl.odd : incl.even);
-            uint32_t start = (uint32_t)__shfl_up((int)end, 1, kWave);
-            if (lane == 0) start = m0;
-            const uint64_t left = wave_ballot(end >= kSumLimit);
-            next = left != 0ull ? __builtin_ctzll(left) : kWave;
-            if (lane >= from && lane < next) {
-                uint32_t m = start;
+        for (int i = 0; i < kSumItems; ++i) map = sum_then(map, sum_map_of(w[i] * pre, scale));
+        if (lane < from) map = SumMap{0u, 0u};
+        const SumMap incl = wave_sum_scan(map);
+        const uint32_t end = m0 + ((m0 & 1u) != 0u ? incl.odd : incl.even);
+        uint32_t start = (uint32_t)__shfl_up((int)end, 1, kWave);
+        if (lane == 0) start = m0;
+        const uint64_t left = wave_ballot(end >= kSumLimit);
+        const int next = left != 0ull ? __builtin_ctzll(left) : kWave;  // the lane to sum in float
+        if (lane >= from && lane < next) {
+            uint32_t m = start;
 #pragma unroll
-                for (int i = 0; i < kSumItems; ++i) {
-                    const SumMap e = sum_map_of(w[i], scale);
-                    m += (m & 1u) != 0u ? e.odd : e.even;
-                    out[i] = sum_value(m, k);
-                }
+            for (int i = 0; i < kSumItems; ++i) {
+                const SumMap e = sum_map_of(w[i] * pre, scale);
+                m += (m & 1u) != 0u ? e.odd : e.even;
+                out[i] = sum_value(m, k);
             }
-            const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)(next == kWave ? end : start), min(next, kWave - 1));
-            total = sum_value(m, k);
-            if (next == kWave) break;
         }
+        const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)(next == kWave ? end : start), min(next, kWave - 1));
+        total = sum_value(m, k);
+        if (next == kWave) break;
 #pragma unroll
         for (int i = 0; i < kSumItems; ++i) {
             total += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w[i]), next));
@@ -588,10 +606,9 @@ __global__ __launch_bounds__(kSumStartThreads) void float_sum_starts_kernel(cons
     const int lane = (int)__lane_id(), wave = (int)(threadIdx.x / kWave);
     float total = 0.0f;
     for (int64_t c = 0; c < chunks;) {
-        const uint32_t bits = __float_as_uint(total);
-        const int k = (int)(bits >> 23) - 127;
+        const int k = sum_binade(total);
+        const uint32_t m0 = sum_mantissa(total, k);
         if (k >= kSumLowest && k < kSumLowest + binades) {  // uniform
-            const uint32_t m0 = (bits & 0x7fffffu) | 0x800000u;
             const int64_t i = c + threadIdx.x;
             SumMap map{0u, 0u};
             if (i < chunks) map = maps[(int64_t)(k - kSumLowest) * chunks + i];
@@ -618,10 +635,41 @@ __global__ __launch_bounds__(kSumStartThreads) void float_sum_starts_kernel(cons
                 continue;  // uniform
             }
             c += bad;
+        } else if (c > 0) {  // (weights of use take the total past the lowest binade in the first chunk)
+            const float pre = sum_prescale(k), scale = sum_scale(k);
+            const int64_t i = c + wave;
+            SumMap map{0u, 0u};
+            if (i < chunks) {  // uniform in the wave
+                float w[kSumItems];
+                load_sum_chunk(weight, count, i, w);
+#pragma unroll
+                for (int j = 0; j < kSumItems; ++j) map = sum_then(map, sum_map_of(w[j] * pre, scale));
+            }
+            map = wave_sum_scan(map);
+            if (lane == kWave - 1) s_map[wave] = map;
+            __syncthreads();
+            SumMap before{0u, 0u};
+            for (int w = 0; w < wave; ++w) before = sum_then(before, s_map[w]);
+            const SumMap own = s_map[wave];
+            const uint32_t start = m0 + ((m0 & 1u) != 0u ? before.odd : before.even);
+            const uint32_t end = start + ((start & 1u) != 0u ? own.odd : own.even);
+            if (lane == 0) s_bad[wave] = end >= kSumLimit ? (uint32_t)wave : UINT32_MAX;
+            __syncthreads();
+            uint32_t bad = UINT32_MAX;
+            for (int w = kWaves - 1; w >= 0; --w) bad = s_bad[w] != UINT32_MAX ? s_bad[w] : bad;
+            if (lane == 0 && i < chunks && (uint32_t)wave <= bad) starts[i] = sum_value(start, k);
+            if (lane == 0 && (uint32_t)wave == min(bad, (uint32_t)kWaves - 1u)) s_m = bad != UINT32_MAX ? start : end;
+            __syncthreads();
+            total = sum_value(s_m, k);
+            if (bad == UINT32_MAX) {
+                c += kWaves;
+                continue;  // uniform
+            }
+            c += bad;
         } else if (threadIdx.x == 0) {
             starts[c] = total;
         }
-        // the chunk that leaves the binade (or starts below the lowest)
+        // the chunk that leaves the binade (or the first)
         if (wave == 0) {
             float w[kSumItems], out[kSumItems];
             load_sum_chunk(weight, count, c, w);
