@@ -13,6 +13,8 @@
 // stream, reached with the O(log i) jump of gsx_pcg32_advance, so the fill is one parallel
 // launch instead of the CPU's sequential loop.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
 #include <math.h>
 #include <stdint.h>
 #include <string.h>
@@ -147,20 +149,23 @@ __global__ __launch_bounds__(kThreads) void multinomial_kernel(int32_t* __restri
                                                                uint64_t state, uint64_t inc) {
     // a sample per thread (its stream reached by the workgroup's uniform jump and the thread's short
     // one): the binary searches are chains of dependent loads, so the more in flight the better (100k
-    // samples over 1M categories, 16 per thread: 80 us, 25 workgroups)
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= samples) return;
-    gsx_amd_pcg32 rng{state, inc};
-    gsx_pcg32_advance(&rng, (uint64_t)blockIdx.x * kThreads);
-    gsx_pcg32_advance(&rng, (uint64_t)threadIdx.x);
-    const float draw = gsx_pcg32_next_f32(&rng) * cdf[categories - 1];
-    int64_t lo = 0, hi = categories;
-    while (lo < hi) {
-        const int64_t mid = lo + (hi - lo) / 2;
-        if (draw < cdf[mid]) hi = mid;
-        else lo = mid + 1;
+    // samples over 1M categories, 16 per thread: 80 us, 25 workgroups); a thread takes more only from
+    // 2^32 samples on, which no launch has threads for
+    for (int64_t first = (int64_t)blockIdx.x * kThreads; first < samples; first += (int64_t)gridDim.x * kThreads) {
+        const int64_t i = first + threadIdx.x;
+        if (i >= samples) return;
+        gsx_amd_pcg32 rng{state, inc};
+        gsx_pcg32_advance(&rng, (uint64_t)first);
+        gsx_pcg32_advance(&rng, (uint64_t)threadIdx.x);
+        const float draw = gsx_pcg32_next_f32(&rng) * cdf[categories - 1];
+        int64_t lo = 0, hi = categories;
+        while (lo < hi) {
+            const int64_t mid = lo + (hi - lo) / 2;
+            if (draw < cdf[mid]) hi = mid;
+            else lo = mid + 1;
+        }
+        out[i] = (int32_t)(lo >= categories ? categories - 1 : lo);
     }
-    out[i] = (int32_t)(lo >= categories ? categories - 1 : lo);
 }
 
 // *flag = 1 when an element is inf or NaN (gsx-cpu/core.c:1208-1246).
@@ -484,12 +489,10 @@ gsx_hip_status gsx_hip_multinomial_i32(int32_t* out, int64_t samples, const floa
     if (samples < 0 || categories < 0 || (samples > 0 && categories > 0 && (out == nullptr || cdf == nullptr)))
         return invalid("multinomial: bad arguments");
     if (samples == 0 || categories == 0) return GSX_HIP_SUCCESS;
-    if (samples > (int64_t)UINT32_MAX / 2 * kThreads) {
-        set_last_error("multinomial: too many samples");
-        return GSX_HIP_ERROR_OUT_OF_RANGE;
-    }
-    hipLaunchKernelGGL(multinomial_kernel, dim3((unsigned)((samples + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                       stream, out, samples, cdf, categories, state, inc);
+    // a launch has fewer than 2^32 threads
+    const int64_t blocks = std::min<int64_t>((samples + kThreads - 1) / kThreads, UINT32_MAX / kThreads);
+    hipLaunchKernelGGL(multinomial_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, out, samples, cdf,
+                       categories, state, inc);
     return launch_status("multinomial_kernel");
 }
 

@@ -1,0 +1,64 @@
+"""gsx_hip_multinomial_i32 against a search of the cumulative weights for the pcg32 stream's draws, up to more
+samples than a launch has threads (2^32)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def _pcg32_advance(state, inc, delta):
+    """(state, inc) after delta steps (the linear congruential jump of the pcg32 family)."""
+    mask, mul, plus = 2**64 - 1, 6364136223846793005, inc
+    acc_mul, acc_plus = 1, 0
+    while delta:
+        if delta & 1:
+            acc_mul, acc_plus = acc_mul * mul & mask, (acc_plus * mul + plus) & mask
+        mul, plus = mul * mul & mask, (mul + 1) * plus & mask
+        delta >>= 1
+    return (acc_mul * state + acc_plus) & mask
+
+
+def _draw(out, cdf, state, inc):
+    from gsx_amd import _lib
+    from gsx_amd.backend import ptr, stream_handle
+    _lib.check(_lib.load().gsx_hip_multinomial_i32(ptr(out), out.numel(), ptr(cdf), cdf.numel(), state, inc,
+                                                   stream_handle()), "multinomial")
+
+
+def _uniform(state, inc, count):
+    """Draws of the stream through a fill of the same library, in [0, 1)."""
+    from gsx_amd import _lib
+    from gsx_amd.backend import ptr, stream_handle
+    u = torch.empty(count, device="cuda")
+    _lib.check(_lib.load().gsx_hip_fill_rand_f32(ptr(u), count, state, inc, stream_handle()), "rand")
+    return u.cpu().numpy()
+
+
+STATE, INC = 0x853C49E6748FEA9B, 0xDA3E39CB94B95BDB
+
+
+@pytest.mark.parametrize("samples,categories", [(1, 1), (255, 7), (256, 1000), (257, 1), (100_001, 5000)])
+def test_draws(samples, categories):
+    w = np.random.default_rng(samples).random(categories).astype(np.float32)
+    cdf = np.cumsum(w, dtype=np.float32)
+    out = torch.full((samples,), -1, dtype=torch.int32, device="cuda")
+    print(f"[case] multinomial {samples} of {categories}", flush=True)
+    _draw(out, torch.from_numpy(cdf).cuda(), STATE, INC)
+    want = np.minimum(np.searchsorted(cdf, _uniform(STATE, INC, samples) * cdf[-1], side="right"), categories - 1)
+    assert np.array_equal(out.cpu().numpy(), want)
+
+
+def test_more_samples_than_threads():
+    samples, tail = 2**32 + 5000, 3000
+    cdf = torch.tensor([0.5, 1.25, 1.5, 4.0], device="cuda")
+    out = torch.full((samples,), -1, dtype=torch.int32, device="cuda")
+    print(f"[case] multinomial {samples} of 4", flush=True)
+    _draw(out, cdf, STATE, INC)
+    torch.cuda.synchronize()
+    for first in (0, 2**32 - 256 - 1000, samples - tail):  # a launch has 2^32 - 256 threads
+        state = _pcg32_advance(STATE, INC, first)
+        c = cdf.cpu().numpy()
+        want = np.minimum(np.searchsorted(c, _uniform(state, INC, tail) * c[-1], side="right"), 3)
+        assert np.array_equal(out[first: first + tail].cpu().numpy(), want), first
