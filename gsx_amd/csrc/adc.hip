@@ -752,7 +752,7 @@ __global__ __launch_bounds__(kAdcThreads) void mcmc_relocate_kernel(int64_t draw
 // row dst[j] = row src[j] over the parameter fields (dst = dead_idx for a relocation, or the
 // appended rows n + j when dst is null), and the optimizer moments of row zero[j] (the source of
 // a relocation, the appended row of a growth) cleared. blockIdx.y names the array; consecutive threads
-// take consecutive floats of its rows.
+// take consecutive floats of its rows (and further ones from 2^32 floats on, which no launch has threads for).
 __global__ __launch_bounds__(kAdcThreads) void mcmc_copy_kernel(int64_t draws, int64_t n,
                                                                 const uint32_t* __restrict__ dst,
                                                                 const uint32_t* __restrict__ src, RowSet rows,
@@ -761,14 +761,14 @@ __global__ __launch_bounds__(kAdcThreads) void mcmc_copy_kernel(int64_t draws, i
     const int f = moment ? (int)blockIdx.y - rows.count : (int)blockIdx.y;
     const uint32_t w = (uint32_t)(moment ? moments.w[f] : rows.w[f]);
     float* const a = moment ? moments.f[f] : rows.f[f];
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= draws * w) return;
-    const int64_t j = draws * w <= (int64_t)UINT32_MAX ? (int64_t)((uint32_t)e / w) : e / w;
-    const int64_t c = e - j * w;
-    const int64_t s = src[j];
-    const int64_t t = dst != nullptr ? (int64_t)dst[j] : n + j;
-    if (moment) a[(zero_source_moments ? s : t) * w + c] = 0.0f;
-    else a[t * w + c] = a[s * w + c];
+    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < draws * w; e += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t j = draws * w <= (int64_t)UINT32_MAX ? (int64_t)((uint32_t)e / w) : e / w;
+        const int64_t c = e - j * w;
+        const int64_t s = src[j];
+        const int64_t t = dst != nullptr ? (int64_t)dst[j] : n + j;
+        if (moment) a[(zero_source_moments ? s : t) * w + c] = 0.0f;
+        else a[t * w + c] = a[s * w + c];
+    }
 }
 
 __global__ __launch_bounds__(256) void gather_rows_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
@@ -800,6 +800,9 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint8_t* __restr
 using namespace gsx_amd;
 
 namespace {
+
+// workgroups of the largest launch: HIP refuses 2^32 threads
+constexpr int64_t kAdcMostBlocks = UINT32_MAX / kAdcThreads;
 
 unsigned adc_blocks(int64_t n) {
     int64_t b = (n + kAdcThreads - 1) / kAdcThreads;
@@ -1040,7 +1043,10 @@ gsx_hip_status mcmc_draw(gsx_hip_adc_context* ctx, const McmcDraws& d, float min
                        d.sample, d.src, d.counts, rows->opacity, rows->logscale);
     int widest = 1;
     for (int f = 0; f < prow.count; ++f) widest = prow.w[f] > widest ? prow.w[f] : widest;
-    hipLaunchKernelGGL(mcmc_copy_kernel, dim3(adc_blocks(d.draws * widest), (unsigned)(prow.count + mrow.count)),
+    const int64_t copy_blocks = (d.draws * widest + kAdcThreads - 1) / kAdcThreads;
+    hipLaunchKernelGGL(mcmc_copy_kernel,
+                       dim3((unsigned)(copy_blocks < kAdcMostBlocks ? copy_blocks : kAdcMostBlocks),
+                            (unsigned)(prow.count + mrow.count)),
                        dim3(kAdcThreads), 0, stream, d.draws, n, d.dst, d.src, prow, mrow, d.dst != nullptr ? 1 : 0);
     ADC_HIP_TRY(hipGetLastError());
     return GSX_HIP_SUCCESS;

@@ -159,3 +159,19 @@ def test_multinomial_of_more_samples_than_threads(host, samples):
 _lib.check(lib.gsx_hip_multinomial_i32(P, {samples}, P, 1000, 1, 3, None), "multinomial")
 assert fake.fake_launches_of(b"multinomial") == 1 and 0 < fake.fake_threads_of(b"multinomial") < 2**32
 """)
+
+
+@pytest.mark.parametrize("dead", [1000, 204_522_240, 250_000_000])  # 21 floats a row: the second fills a launch
+def test_relocation_of_more_floats_than_threads(host, dead):
+    host(ROWS + f"""
+def rows(count, few=rows):
+    r = few(count)
+    r.sh_degree = 3
+    r.sh1 = r.sh2 = r.sh3 = P
+    return r
+
+fake.fake_set_totals({dead}, 1)
+_, counts = step(context(), 2, 400_000_000, 400_000_000)
+assert counts[0] == counts[2] == {dead}
+assert fake.fake_launches_of(b"mcmc_copy") == 1 and fake.fake_threads_of(b"mcmc_copy") >= min({dead} * 21, 2**32 - 256)
+""")
