@@ -941,6 +941,19 @@ RowSet moment_rows(const gsx_hip_gs_rows& r) {
     return s;
 }
 
+// Whether two sets bind the same parameter fields and moments (the compaction pairs them in order).
+bool same_fields(const gsx_hip_gs_rows& a, const gsx_hip_gs_rows& b) {
+    const float* const sh[3][2] = {{a.sh1, b.sh1}, {a.sh2, b.sh2}, {a.sh3, b.sh3}};
+    for (int d = 0; d < 3; ++d)
+        if (a.sh_degree > d && (sh[d][0] != nullptr) != (sh[d][1] != nullptr)) return false;
+    for (int k = 0; k < 8; ++k) {
+        if (k >= 5 && a.sh_degree < k - 4) continue;
+        if ((a.first_moment[k] != nullptr) != (b.first_moment[k] != nullptr)) return false;
+        if ((a.second_moment[k] != nullptr) != (b.second_moment[k] != nullptr)) return false;
+    }
+    return true;
+}
+
 }  // namespace
 
 struct gsx_hip_adc_context {
@@ -1279,8 +1292,8 @@ gsx_hip_status gsx_hip_adc_step(gsx_hip_adc_context* ctx, const gsx_hip_adc_para
         gsx_hip_gs_rows to = *out;
         to.sh_degree = rows->sh_degree;
         int d0, d1, d2, d3;
-        const bool out_same = out_bound && param_rows(to, &d0, &d1, &d2, &d3, true).count == prow.count &&
-                              moment_rows(to).count == mrow.count;
+        const bool out_same = out_bound && same_fields(*rows, to) &&
+                              param_rows(to, &d0, &d1, &d2, &d3, true).count == prow.count;
         // the result's statistics restart (gsx/src/gsx-cpu/adc.c:446-452): zeroed, not copied
         const RowSet src = param_rows(*rows, &d0, &d1, &d2, &d3, false);
         if (out_same) {

@@ -175,3 +175,29 @@ _, counts = step(context(), 2, 400_000_000, 400_000_000)
 assert counts[0] == counts[2] == {dead}
 assert fake.fake_launches_of(b"mcmc_copy") == 1 and fake.fake_threads_of(b"mcmc_copy") >= min({dead} * 21, 2**32 - 256)
 """)
+
+
+@pytest.mark.parametrize("change", ["o.sh1, o.absgrad_acc = None, P", "o.sh1, o.sh2 = None, P",
+                                    "o.first_moment[0], o.second_moment[0] = None, P"])
+def test_out_rows_of_other_fields_are_not_written(host, change):
+    """As many fields, but other ones: no compaction into them is queued, and the refine says so."""
+    host(ROWS + f"""
+def rows(count, few=rows):
+    r = few(count)
+    r.sh_degree, r.sh1 = 2, P
+    r.first_moment[0] = P
+    return r
+
+fake.fake_set_totals(5, 0)  # rows kept
+step(context(), 0, 1000, 1000)
+assert fake.fake_launches_of(b"adc_compact") == 1
+o = rows(1000)
+{change}
+try:
+    step(context(), 0, 1000, 1000, out=o)
+except _lib.GsxHipError as e:
+    assert "the same fields" in str(e)
+else:
+    raise AssertionError("accepted")
+assert fake.fake_launches_of(b"adc_compact") == 1
+""")
