@@ -1044,17 +1044,24 @@ constexpr int kGradRecord = 8;  // per-instance partials: channels 0-7 in one 32
 //      dmean2d, d(conic)  are sums of dpow times 1, dx, dy, dx^2, dx dy, dy^2,
 //      dcolor             are sums of w times the pixel's image gradient.
 //    So the sum over a quadrant's 64 pixels is a product of matrices: 16 rows (h and w of 8 entries)
-//    by 64 pixels, times 64 pixels by 9 columns (the monomials of the pixel's offset u, v from the
-//    quadrant's centre, |u|, |v| <= 3.5, and the three image gradients): 16 f32 16x16x4 matrix
-//    instructions per 8 entries. (On gfx950 an f32 matrix instruction takes the vector ALUs' time,
-//    about 7 vector instructions' worth; that is 15 per entry, where the products and their reduction
-//    over lanes took some 60.) Once per entry and tile the moments are moved from the quadrants'
-//    centres to the entry's mean, added over the quadrants, and mapped through the conic and the
-//    d(conic)/d(cov2d) coefficients. The suffix is one scalar, its product with the image gradient.
+//    by 64 pixels, times 64 pixels by 16 columns (the monomials of the pixel's offset from an origin near
+//    the entry's mean, and the three image gradients): 16 f32 16x16x4 matrix instructions per 8 entries.
+//    (On gfx950 an f32 matrix instruction takes the vector ALUs' time, 32 cycles or 8 vector
+//    instructions' worth; that is 16 per entry, where the products and their reduction over lanes took
+//    some 60.) Once per entry and tile the moments are moved from that origin to the entry's mean, added
+//    over the quadrants, and mapped through the conic and the d(conic)/d(cov2d) coefficients. The suffix
+//    is one scalar, its product with the image gradient.
+//    The move cancels: a second moment about a point at distance d from the mean is larger than the one
+//    about the mean by d^2 / sigma^2, and so is its rounding. So the columns hold the moments about four
+//    origins, (+/- 2, +/- 2) from the quadrant's centre, which share enough columns to fit the 16, and an
+//    entry takes those on its mean's side. (About the centre alone, 9 columns, footprints of a pixel or
+//    two lost up to a bit of the scale and rotation gradients: 0.97e-6 -> 1.76e-6 off 64 bits, now 1.03e-6,
+//    5000 of sigma 0.6 to 0.9 on a plane. The selection costs 3% of the kernel.)
 //  * Per contribution. That map amplifies rounding by the eigenvalue ratio of the 2D covariance:
 //    near-plane Gaussians reach ratios of 1e6 and more, where the CPU's gradient is mostly the
-//    rounding of its per-contribution map. A tile with an entry that is not regular forms every term per contribution with the CPU's operations, the suffix colour and its division
-//    included, and sums the nine values over the wave with lane swaps and DPP moves.
+//    rounding of its per-contribution map. A tile with an entry that is not regular forms every term per
+//    contribution with the CPU's operations, the suffix colour and its division included, and sums the
+//    nine values over the wave with lane swaps and DPP moves.
 //
 // Reduction without atomics: every wave leaves one row of nine sums per entry in LDS, four threads
 // per entry combine the four waves' rows, and the tile writes one 9-float partial per reached
@@ -1080,6 +1087,15 @@ constexpr int kBackBatch = 64;
 constexpr int kMomentEntries = 8;  // entries of one matrix product
 
 typedef float gsx_f32x4 __attribute__((ext_vector_type(4)));
+
+// Origins of an entry's moments in a quadrant: (+/- kMomentOrigin, +/- kMomentOrigin) from its centre, on the
+// sides of the entry's mean.
+constexpr float kMomentOrigin = 2.0f;
+
+// Column c of a product's second factor: its place in a row of sums (1, u, v, u^2, u v, v^2, image gradient), and the
+// sides whose entries take it (see blend_backward_walk), a nibble a column.
+__device__ inline uint32_t moment_place(uint32_t c) { return (uint32_t)(0x8764444525231310ull >> (4u * c)) & 15u; }
+__device__ inline uint32_t moment_sides(uint32_t c) { return (uint32_t)(0xfff142833cc55aafull >> (4u * c)) & 15u; }
 
 // Sum over the four lanes of a quad, in every lane.
 __device__ inline float quad_sum(float v) {
@@ -1129,6 +1145,7 @@ struct BackwardShared {
     BlendEntry entry[kBackBatch];  // c.w: the entry's emission position
     uint64_t exp2[GSX_EXPF_BLEND_TABLE_SIZE];
     uint64_t used[kWavesPerTile];
+    alignas(8) uint32_t side[kWavesPerTile][kMomentEntries];  // of a product's entries (see flush)
     uint32_t max_last;
     float sum[kWavesPerTile][(kBackBatch + kMomentEntries) * kGrad2d];
     union {
@@ -1168,8 +1185,9 @@ __device__ inline void blend_backward_walk(BackwardShared& sm, const BackwardPix
     if (kMoments) s0 = s0 * d0 + s1 * d1 + s2 * d2;
 
     // Moments: this lane's column of the products' second factor, one value per step: step s takes the
-    // pixels 16 (lane / 16) + s of the quadrant. Columns 0-5: 1, u, v, u^2, u v, v^2; 6-8: the image
-    // gradient.
+    // pixels 16 (lane / 16) + s of the quadrant. With u, v the pixel's offset from the quadrant's centre
+    // and a = kMomentOrigin the columns are 1; u - a, (u - a)^2, u + a, (u + a)^2; the same of v;
+    // (u - a)(v - a), (u - a)(v + a), (u + a)(v - a), (u + a)(v + a); the image gradient. All are exact.
     float* const x = sm.x[wave];
     const uint32_t column = lane & 15u;
     float factor[kMoments ? 16 : 1];
@@ -1178,18 +1196,19 @@ __device__ inline void blend_backward_walk(BackwardShared& sm, const BackwardPix
         x[kWave + lane] = d1;
         x[2 * kWave + lane] = d2;
         wave_lds_sync();
-        const float* dcol = x + kWave * (min(max((int)column, 6), 8) - 6) + 16 * (lane >> 4);
+        const float* dcol = x + kWave * (max((int)column, 13) - 13) + 16 * (lane >> 4);
+        const float ax = (column - 1u) % 4u < 2u ? kMomentOrigin : -kMomentOrigin;  // columns 1 to 8
+        const float bx = column < 11u ? kMomentOrigin : -kMomentOrigin;             // columns 9 to 12
+        const float by = (column & 1u) != 0u ? kMomentOrigin : -kMomentOrigin;
 #pragma unroll
         for (int s = 0; s < 16; ++s) {
             const float u = (float)(s & 7) - 3.5f, v = (float)(2 * (int)(lane >> 4) + (s >> 3)) - 3.5f;
+            const float t = (column < 5u ? u : v) - ax;
             float f = dcol[s];
-            if (column == 0) f = 1.0f;
-            if (column == 1) f = u;
-            if (column == 2) f = v;
-            if (column == 3) f = u * u;
-            if (column == 4) f = u * v;
-            if (column == 5) f = v * v;
-            factor[s] = column < 9u ? f : 0.0f;
+            if (column < 13u) f = (u - bx) * (v - by);
+            if (column < 9u) f = (column & 1u) != 0u ? t : t * t;
+            if (column == 0u) f = 1.0f;
+            factor[s] = f;
         }
         wave_lds_sync();
     }
@@ -1246,22 +1265,44 @@ __device__ inline void blend_backward_walk(BackwardShared& sm, const BackwardPix
         uint64_t used = 0;
         auto flush = [&]() {
             wave_lds_sync();
-            gsx_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+            // which side of the quadrant's centre each entry's mean lies on: the product's entries are the lowest
+            // `fill` of `used`, the first of them highest. (Formed here by lane = entry: bits collected entry by
+            // entry in scalar registers cost 6% of the kernel, and held vector registers spill.)
+            bool take0, take1;
+            {
+                uint32_t l = __lane_id();
+                asm volatile("" : "+v"(l));
+                const float2 mean = *reinterpret_cast<const float2*>(&sm.entry[l].a);
+                const uint32_t at = (uint32_t)fill - 1u - __builtin_amdgcn_mbcnt_hi((uint32_t)(used >> 32),
+                                                                                   __builtin_amdgcn_mbcnt_lo((uint32_t)used, 0u));
+                const uint32_t side = (mean.x >= (float)((pix.pxy & 0xfff8u) + 4u) ? 1u : 0u) |
+                                      (mean.y >= (float)((pix.pxy >> 16 & 0xfff8u) + 4u) ? 2u : 0u);
+                if (__builtin_amdgcn_inverse_ballot_w64(used) && at < (uint32_t)fill) sm.side[wave][at] = side;
+                wave_lds_sync();
+                const uint2 both = *reinterpret_cast<const uint2*>(&sm.side[wave][2u * (l >> 4)]);
+                const uint32_t sides = moment_sides(l & 15u);
+                take0 = ((sides >> (both.x & 3u)) & 1u) != 0u;
+                take1 = ((sides >> (both.y & 3u)) & 1u) != 0u;
+            }
+            // two chains of 32 pixels, not one of 64: half the rounding of the sums
+            gsx_f32x4 part[2] = {};
             const char* const xb = reinterpret_cast<const char*>(x);
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
                 const float4 a = *reinterpret_cast<const float4*>(xb + (read_at ^ (16u * t)));
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, factor[kMoments ? 4 * t : 0], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, factor[kMoments ? 4 * t + 1 : 0], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, factor[kMoments ? 4 * t + 2 : 0], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, factor[kMoments ? 4 * t + 3 : 0], acc, 0, 0, 0);
+                gsx_f32x4& to = part[t / 2];
+                to = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, factor[kMoments ? 4 * t : 0], to, 0, 0, 0);
+                to = __builtin_amdgcn_mfma_f32_16x16x4f32(a.y, factor[kMoments ? 4 * t + 1 : 0], to, 0, 0, 0);
+                to = __builtin_amdgcn_mfma_f32_16x16x4f32(a.z, factor[kMoments ? 4 * t + 2 : 0], to, 0, 0, 0);
+                to = __builtin_amdgcn_mfma_f32_16x16x4f32(a.w, factor[kMoments ? 4 * t + 3 : 0], to, 0, 0, 0);
             }
+            const gsx_f32x4 acc = part[0] + part[1];
             // lane l holds rows 4 (l / 16) .. + 3 of column l % 16: h and w of two entries
-            if (column < 9u) {
-                float* const to = &sm.sum[wave][(rows - fill + 2 * (int)(lane >> 4)) * kGrad2d + (int)column];
-                to[0] = column < 6u ? acc.x : acc.y;
-                to[kGrad2d] = column < 6u ? acc.z : acc.w;
-            }
+            uint32_t l = __lane_id();
+            asm volatile("" : "+v"(l));
+            float* const to = &sm.sum[wave][(rows - fill + 2 * (int)(l >> 4)) * kGrad2d + (int)moment_place(l & 15u)];
+            if (take0) to[0] = (l & 15u) < 13u ? acc.x : acc.y;
+            if (take1) to[kGrad2d] = (l & 15u) < 13u ? acc.z : acc.w;
             wave_lds_sync();
             fill = 0;
         };
@@ -1402,9 +1443,11 @@ __device__ inline void blend_backward_walk(BackwardShared& sm, const BackwardPix
             }
             const BlendEntry en = sm.entry[e];
             if constexpr (kMoments) {
-                // moments about the quadrant's centre -> about the mean: the offset is u + ex, v + ey
-                const float ex = (float)(tx * kTile + 8 * (int)(p & 1u) + 4) - en.a.x;
-                const float ey = (float)(ty * kTile + 8 * (int)(p >> 1) + 4) - en.a.y;
+                // moments about the entry's origin in the quadrant -> about the mean: the offset is u + ex, v + ey
+                const float qcx = (float)(tx * kTile + 8 * (int)(p & 1u) + 4);
+                const float qcy = (float)(ty * kTile + 8 * (int)(p >> 1) + 4);
+                const float ex = (en.a.x >= qcx ? qcx + kMomentOrigin : qcx - kMomentOrigin) - en.a.x;
+                const float ey = (en.a.y >= qcy ? qcy + kMomentOrigin : qcy - kMomentOrigin) - en.a.y;
                 const float sx = __builtin_fmaf(ex, v[0], v[1]), sy = __builtin_fmaf(ey, v[0], v[2]);
                 v[3] = __builtin_fmaf(ex, v[1] + sx, v[3]);
                 v[4] = __builtin_fmaf(ex, v[2], __builtin_fmaf(ey, sx, v[4]));
