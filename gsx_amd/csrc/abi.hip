@@ -191,7 +191,7 @@ struct PinnedBuffer {
 // Instance counts from which the tile ranges come from a binary search per tile rather than a
 // pass over the sorted tiles (the search's cost does not grow with the count)
 constexpr int64_t kRangesSearchMin = (int64_t)1 << 25;
-// Images of up to this many tiles keep the tile index of an instance in 16 bits: 30 instead of 48
+// Images of up to this many tiles keep the tile index of an instance in 16 bits: 32 instead of 48
 // bytes per instance through emission, the two sort passes and the ranges (335M instances of a 1080p
 // image: emission 877 -> 726 us, a sort pass's counts 284 -> 188 and moves 1195 -> 1049, a training step
 // 6.42 -> 5.85 ms; 5M instances: 284 -> 269 us a frame).
@@ -892,7 +892,7 @@ gsx_hip_status gsx_hip_render_forward(gsx_hip_render_context* ctx, const gsx_hip
                            long_chunk_of(tiles),
                            ctx->big_list.as<uint2>(), ctx->scan_temp.as<uint32_t>());
         GSX_HIP_TRY(hipGetLastError(), "rank_gather_kernel");
-        // exclusive scan of the 256-rank sums; emit_keys_kernel completes the offsets
+        // exclusive scan of the 256-rank sums; emit_kernel completes the offsets
         GSX_TRY(scan_partials_in_place(ctx->scan_temp.as<uint32_t>(), pre_blocks, stream, 4));
     }
     GSX_TRY(record(ctx, 2, stream));

@@ -520,10 +520,11 @@ __device__ inline uint32_t digit_of(KeyT key, int shift) {
 }
 
 // Upsweep of one kChunk-key chunk (workgroup `blk` of kSortThreads threads): its digit counts,
-// counted in wave-private LDS counters, to hist[digit][blk]. n_dev (may be null): live key
+// counted in wave-private LDS counters, to hist[digit][blk], or to hist[blk][digit] (by_chunk: few chunks,
+// whose counts the downsweep adds up itself). n_dev (may be null): live key
 // count, n = min(n, *n_dev); drop_sentinel: keys equal to kSentinelKey are not counted.
 // dmask keeps the digit's bits below the sort's end bit (a last pass narrower than kBits). KeyT:
-// uint64_t (the depth order and the public sorts) or uint32_t (tile indices).
+// uint64_t (the depth order and the public sorts), uint32_t or uint16_t (tile indices).
 // Digit histograms of an upsweep workgroup: per wave, kUpsweepCopies<kBits> copies (one per
 // group of 64 / copies lanes), so that lanes of one wave that count the same digit in the same
 // round mostly add to different words; each copy kBins + 64 / copies words long, so that a digit's

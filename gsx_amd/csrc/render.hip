@@ -13,8 +13,8 @@
 //   geo[2g+1] = {inv_c, opacity, x_min | x_max << 16, y_min | y_max << 16}   (ints as f32 bits)
 //   col[g]    = {color_r, color_g, color_b, depth}
 // Emission and tile counting gather records in depth order, one per Gaussian: they need the
-// geometry only, a 32 B-aligned read. The blends read both and stage them in LDS as
-//   {geo0} {inv_c, opacity, color_r, color_g} {color_b, box lo, box extent, depth}.
+// geometry only, a 32 B-aligned read. The blends read both and stage them in LDS as a BlendEntry,
+// with the contribution box cbox[g] (8 B, behind the colours).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -563,7 +563,7 @@ __device__ inline void emit_block(uint32_t b, int64_t n, int64_t rank_end, const
         r0 = rec[2 * (size_t)g + 0];
         r1 = rec[2 * (size_t)g + 1];
     }
-    // big boxes are emitted by big_rows_block; the walk numbers the wave's other instances
+    // big boxes are emitted by big_boxes_wave; the walk numbers the wave's other instances
     // consecutively, so a lane's base is its offset less the walked instances of the lanes
     // before it (the counting walk's identical runs gave the counts)
     const bool walked = cnt > 0 && box_tiles(r1) <= kBigTiles;
@@ -813,10 +813,10 @@ __device__ inline BlendEntry blend_entry(float4 geo0, float4 geo1, float4 col, u
 // skipped when that bound stays below the cut, max(-4.5, ln(1 / (255 opacity))), by 1e-3 and 1e-5 of
 // the terms' largest sum (40 times the rounding of the power as the pixels evaluate it; the bound's
 // own is about twice that). A conic that is not positive definite by 2^-16 of its terms, and any NaN,
-// keeps the entry. Of the entries whose boxes meet a quadrant 11 to 12% are skipped in scenes of long
-// Gaussians (1M in clusters, 500k in a cube; a test of every pixel would skip 12 to 13%), 7% of round
-// ones on a plane: forward 62 -> 57 us (100k, 640x480), 97 -> 89 (500k,
-// 720p, TRAIN), backward 185 -> 179; the clusters, whose tiles close after some 50 entries, gain nothing.
+// keeps the entry. Of the entries whose boxes meet a quadrant before its pixels close, 12 to 13% are skipped in
+// a cube of long Gaussians (100k and 500k) and 7% of the round ones on a plane: forward 62 -> 57 us (100k,
+// 640x480), 97 -> 89 (500k, 720p, TRAIN), backward 185 -> 179. In the clusters a few near Gaussians close the
+// tiles, and none is skipped.
 __device__ inline bool box_meets_quadrant(const BlendEntry& e, uint32_t qx, uint32_t qy) {
     const uint32_t lo = __float_as_uint(e.c.y), ext = __float_as_uint(e.c.z);
     const uint32_t x0 = lo & 0xffffu, y0 = lo >> 16;
@@ -849,11 +849,17 @@ __device__ inline bool entry_meets_quadrant(const BlendEntry& e, uint32_t qx, ui
 //  * A pixel outside a regular entry's 3-sigma box fails the power cut by itself: it lies at least half
 //    a pixel beyond 3 sigma, where the power is below -4.5 (1 + 1 / (3 sigma)) <= -4.5 (1 + 3e-4), and
 //    the float evaluation is off by less than 6e-5 of it (the form's terms are at most 2 r = 128 times
-//    their sum, each rounded a few times). So its pixels need no box test: 3 instructions of some 40,
+//    their sum, each rounded a few times); the rounding of the box's own radius, below 1e-6 of it, is far less. So its pixels need no box test: 3 instructions of some 40,
 //    left out where a whole tile is regular (blend_backward_kernel's moments: 934 -> 906 us at 1M
 //    Gaussians on a plane; a branch per group in the forward cost more than it saved, 394 -> 417 us).
 //  * The map from moments to covariance gradients loses no more digits than the ratio says
 //    (blend_backward_kernel).
+// The limit: of the entries that a tile's pixels reach, none is above 64 in a cube of 200k or 500k long Gaussians
+// (0.4% are above 16, but in 40% of the tiles, one of which takes a whole tile's time: blend backward 230 us
+// at 16, 179 at 64 and more) and none above 16 on a plane; all are, at any limit up to 16384, where near-plane
+// Gaussians close the tiles (1M in clusters). Only a scene between these would gain from a larger limit:
+// 6M at full HD have 6.1% of the entries and 92% of the tiles above 64 (589 us), 1.2 and 40% above 256 (546),
+// 0.1 and 7% above 1024 (495). There the gradient's error at such ratios is not measured.
 constexpr float kRegularRatio = 64.0f;
 constexpr float kRegularExtent = 1048576.0f;
 __device__ inline bool entry_is_regular(const BlendEntry& e) {
@@ -1056,7 +1062,7 @@ constexpr int kGradRecord = 8;  // per-instance partials: channels 0-7 in one 32
 //    origins, (+/- 2, +/- 2) from the quadrant's centre, which share enough columns to fit the 16, and an
 //    entry takes those on its mean's side. (About the centre alone, 9 columns, footprints of a pixel or
 //    two lost up to a bit of the scale and rotation gradients: 0.97e-6 -> 1.76e-6 off 64 bits, now 1.03e-6,
-//    5000 of sigma 0.6 to 0.9 on a plane. The selection costs 3% of the kernel.)
+//    5000 of sigma 0.6 to 0.8 on a plane. The selection costs 3 to 4% of the kernel.)
 //  * Per contribution. That map amplifies rounding by the eigenvalue ratio of the 2D covariance:
 //    near-plane Gaussians reach ratios of 1e6 and more, where the CPU's gradient is mostly the
 //    rounding of its per-contribution map. A tile with an entry that is not regular forms every term per
@@ -1072,13 +1078,14 @@ constexpr int kGradRecord = 8;  // per-instance partials: channels 0-7 in one 32
 // full-screen Gaussians (present in every tile), and the instances behind saturated pixels cost the
 // backward nothing.
 //
-// Bound by instruction issue (84% of the SIMDs' cycles at 1M Gaussians on a plane, 70 vector
-// instructions per wave and entry plus the products' 15; every term per contribution took 156).
+// Bound by instruction issue (82% of the SIMDs' cycles at 1M Gaussians on a plane, 73 vector
+// instructions per walked quadrant and entry plus the products' 18 such; every term per contribution took 156).
 // With every entry tested by every pixel and every term per contribution, and now: that plane at
-// 1024^2 1309 -> 906 us; 500k in a cube at 720p 283 -> 182 us; 1M clustered at full HD (per
-// contribution) 170 -> 163 us. f32 products for the per-contribution sums too were slower (255 us:
-// 8 matrix instructions per entry instead of 24 lane operations), as was sharing both forms in one
-// walk (191 us: 105 registers). 64-entry batches took 1052 us where 32 took 1174: fewer barriers.
+// 1024^2 1233 -> 892 us; 500k in a cube at 720p 268 -> 184 us; 1M clustered at full HD (per contribution, all
+// tiles) 222 -> 227 us: that walk alone would fit 6 waves per SIMD, and both in one kernel leave 5.
+// f32 products for the per-contribution sums too were slower (255 us: 8 matrix instructions per entry
+// instead of 24 lane operations), as was sharing both forms in one walk (191 us: 105 registers).
+// 64-entry batches took 1052 us where 32 took 1174: fewer barriers.
 // ---------------------------------------------------------------------------------------------
 constexpr int kWavesPerTile = kBlendThreads / kWave;
 
@@ -1092,8 +1099,9 @@ typedef float gsx_f32x4 __attribute__((ext_vector_type(4)));
 // sides of the entry's mean.
 constexpr float kMomentOrigin = 2.0f;
 
-// Column c of a product's second factor: its place in a row of sums (1, u, v, u^2, u v, v^2, image gradient), and the
-// sides whose entries take it (see blend_backward_walk), a nibble a column.
+// Column c of a product's second factor (blend_backward_walk): its place in a row of sums (1, u, v, u^2, u v, v^2,
+// image gradient), and a bit for each of the four sides whose entries take it (bit x + 2 y, x and y 1 where
+// the mean lies on the + side). A nibble a column.
 __device__ inline uint32_t moment_place(uint32_t c) { return (uint32_t)(0x8764444525231310ull >> (4u * c)) & 15u; }
 __device__ inline uint32_t moment_sides(uint32_t c) { return (uint32_t)(0xfff142833cc55aafull >> (4u * c)) & 15u; }
 
@@ -1267,7 +1275,8 @@ __device__ inline void blend_backward_walk(BackwardShared& sm, const BackwardPix
             wave_lds_sync();
             // which side of the quadrant's centre each entry's mean lies on: the product's entries are the lowest
             // `fill` of `used`, the first of them highest. (Formed here by lane = entry: bits collected entry by
-            // entry in scalar registers cost 6% of the kernel, and held vector registers spill.)
+            // entry in scalar registers cost 6% of the kernel; a lane's place and sides held in a register gain
+            // nothing, and spill others.)
             bool take0, take1;
             {
                 uint32_t l = __lane_id();
@@ -1647,7 +1656,6 @@ __device__ inline void reduce_run_chunk(uint32_t b, uint32_t e, uint32_t g, uint
     instance_grad_op[cb] = acc[8];
 }
 
-// The +0 sums of chunk k of a long run that no tile reached, stored by one lane.
 // Chunk k of the long runs of the wave's lanes (run [b, e) of Gaussian g where `live`): the
 // touched ones are summed by the wave one after another (the untouched ones have no sums: the
 // projection backward skips their Gaussians).

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kSortThreads) void radix_upsweep_kernel(const KeyT*
 // totals[d]. A step covers kThreads * kRowItems counts; wave w takes the step's w-th run of
 // 64 * kRowItems, as kRowItems coalesced groups of 64 (one count per lane), each scanned with DPP
 // and carried into the next. The next step's counts are loaded before the current step's scan,
-// so the row's serial steps overlap their loads. Long rows (config 4's tile sort: 82k chunks) run
+// so the row's serial steps overlap their loads. Long rows (config 4's tile sort: 41k chunks) run
 // 1024 threads, short ones 256.
 template <int kThreads>
 __global__ __launch_bounds__(kThreads) void radix_rowscan_kernel(const uint32_t* __restrict__ hist,
