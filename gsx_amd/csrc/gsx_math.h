@@ -600,4 +600,24 @@ GSX_HD void gsx_pcg32_advance(gsx_amd_pcg32 *rng, uint64_t delta)
     rng->state = acc_mult * rng->state + acc_plus;
 }
 
+/* The jump by `delta` draws of the streams with this increment: state -> mult * state + plus. */
+typedef struct gsx_pcg32_jump {
+    uint64_t mult, plus;
+} gsx_pcg32_jump;
+
+GSX_HD gsx_pcg32_jump gsx_pcg32_jump_by(uint64_t inc, uint64_t delta)
+{
+    gsx_amd_pcg32 zero, one;
+    gsx_pcg32_jump jump;
+
+    zero.state = 0u;
+    one.state = 1u;
+    zero.inc = one.inc = inc;
+    gsx_pcg32_advance(&zero, delta);
+    gsx_pcg32_advance(&one, delta);
+    jump.mult = one.state - zero.state;
+    jump.plus = zero.state;
+    return jump;
+}
+
 #endif /* GSX_AMD_MATH_H */

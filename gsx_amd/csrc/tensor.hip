@@ -39,6 +39,13 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kRandPerThread = 16;  // consecutive draws per lane of the rand-like fills
+// Categories up to which a multinomial launch has at most kMultinomialBlocks workgroups. The sums of that few stay in
+// a CU's 32 KB cache and finding the draw costs as much as the search, so a thread finds its place in the stream
+// once for many samples (16M samples of 4: 318 -> 42 us, of 1000: 326 -> 137, of 8192: 330 -> 254; of 32768
+// 397 -> 437). With more a search waits on memory, and a thread per sample keeps most of them in flight (16M of
+// 65536: 502 us, 554 with many a thread; 100k samples of 1M: 10, and 56 with 16 a thread).
+constexpr int64_t kMultinomialFew = 8192;
+constexpr int64_t kMultinomialBlocks = 4096;
 
 unsigned grid_for(int64_t n, int64_t per_block) {
     int64_t b = (n + per_block - 1) / per_block;
@@ -143,21 +150,20 @@ __global__ __launch_bounds__(kThreads) void randint_scatter_kernel(const uint32_
 }
 
 // multinomial: sample i from draw i, u * cdf[last], first category whose cdf exceeds it
-// (gsx-cpu/core.c:1118-1206).
+// (gsx-cpu/core.c:1118-1206). A thread takes the samples i, i + gridDim.x * kThreads, ...: it finds its place in
+// the stream once and goes on by `step`, the jump by that many draws (see kMultinomialFew; from 2^32 samples on no
+// launch has a thread for each).
 __global__ __launch_bounds__(kThreads) void multinomial_kernel(int32_t* __restrict__ out, int64_t samples,
                                                                const float* __restrict__ cdf, int64_t categories,
-                                                               uint64_t state, uint64_t inc) {
-    // a sample per thread (its stream reached by the workgroup's uniform jump and the thread's short
-    // one): the binary searches are chains of dependent loads, so the more in flight the better (100k
-    // samples over 1M categories, 16 per thread: 80 us, 25 workgroups); a thread takes more only from
-    // 2^32 samples on, which no launch has threads for
-    for (int64_t first = (int64_t)blockIdx.x * kThreads; first < samples; first += (int64_t)gridDim.x * kThreads) {
-        const int64_t i = first + threadIdx.x;
-        if (i >= samples) return;
-        gsx_amd_pcg32 rng{state, inc};
-        gsx_pcg32_advance(&rng, (uint64_t)first);
-        gsx_pcg32_advance(&rng, (uint64_t)threadIdx.x);
-        const float draw = gsx_pcg32_next_f32(&rng) * cdf[categories - 1];
+                                                               uint64_t state, uint64_t inc, gsx_pcg32_jump step) {
+    int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x;
+    if (i >= samples) return;
+    gsx_amd_pcg32 rng{state, inc};
+    gsx_pcg32_advance(&rng, (uint64_t)i);
+    const float total = cdf[categories - 1];
+    for (;;) {
+        gsx_amd_pcg32 here = rng;
+        const float draw = gsx_pcg32_next_f32(&here) * total;
         int64_t lo = 0, hi = categories;
         while (lo < hi) {
             const int64_t mid = lo + (hi - lo) / 2;
@@ -165,6 +171,9 @@ __global__ __launch_bounds__(kThreads) void multinomial_kernel(int32_t* __restri
             else lo = mid + 1;
         }
         out[i] = (int32_t)(lo >= categories ? categories - 1 : lo);
+        i += (int64_t)gridDim.x * kThreads;
+        if (i >= samples) return;
+        rng.state = step.mult * rng.state + step.plus;
     }
 }
 
@@ -489,10 +498,11 @@ gsx_hip_status gsx_hip_multinomial_i32(int32_t* out, int64_t samples, const floa
     if (samples < 0 || categories < 0 || (samples > 0 && categories > 0 && (out == nullptr || cdf == nullptr)))
         return invalid("multinomial: bad arguments");
     if (samples == 0 || categories == 0) return GSX_HIP_SUCCESS;
-    // a launch has fewer than 2^32 threads
-    const int64_t blocks = std::min<int64_t>((samples + kThreads - 1) / kThreads, UINT32_MAX / kThreads);
+    // (a launch has fewer than 2^32 threads)
+    const int64_t most = categories <= kMultinomialFew ? kMultinomialBlocks : UINT32_MAX / kThreads;
+    const int64_t blocks = std::min<int64_t>((samples + kThreads - 1) / kThreads, most);
     hipLaunchKernelGGL(multinomial_kernel, dim3((unsigned)blocks), dim3(kThreads), 0, stream, out, samples, cdf,
-                       categories, state, inc);
+                       categories, state, inc, gsx_pcg32_jump_by(inc, (uint64_t)blocks * kThreads));
     return launch_status("multinomial_kernel");
 }
 

@@ -152,11 +152,12 @@ assert look(h)
 """)
 
 
+@pytest.mark.parametrize("categories", [1000, 1_000_000])  # many samples a thread, and one
 @pytest.mark.parametrize("samples", [1, 2**32 - 256, 2**32 - 255, 2**32, 2**34])
-def test_multinomial_of_more_samples_than_threads(host, samples):
+def test_multinomial_of_more_samples_than_threads(host, samples, categories):
     """A launch of 2^32 threads is refused: beyond that a thread draws several samples."""
     host(f"""
-_lib.check(lib.gsx_hip_multinomial_i32(P, {samples}, P, 1000, 1, 3, None), "multinomial")
+_lib.check(lib.gsx_hip_multinomial_i32(P, {samples}, P, {categories}, 1, 3, None), "multinomial")
 assert fake.fake_launches_of(b"multinomial") == 1 and 0 < fake.fake_threads_of(b"multinomial") < 2**32
 """)
 
