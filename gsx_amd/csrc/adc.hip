@@ -549,30 +549,44 @@ __device__ inline float sum_chunk(float total, const float (&w)[kSumItems], floa
     const int lane = (int)__lane_id();
     int from = 0;  // lanes before it are done
     while (from < kWave) {
-        const int k = sum_binade(total);
-        const float pre = sum_prescale(k), scale = sum_scale(k);
-        const uint32_t m0 = sum_mantissa(total, k);
-        SumMap map{0u, 0u};
+        int next;  // the lane to sum in float
+        // (uniform) nothing up to the first weight, which leaves whatever binade: no pairs to scan (a refine of 200
+        // rows: 139 us with them, 132 so)
+        if (total == 0.0f) {
+            bool any = false;
 #pragma unroll
-        for (int i = 0; i < kSumItems; ++i) map = sum_then(map, sum_map_of(w[i] * pre, scale));
-        if (lane < from) map = SumMap{0u, 0u};
-        const SumMap incl = wave_sum_scan(map);
-        const uint32_t end = m0 + ((m0 & 1u) != 0u ? incl.odd : incl.even);
-        uint32_t start = (uint32_t)__shfl_up((int)end, 1, kWave);
-        if (lane == 0) start = m0;
-        const uint64_t left = wave_ballot(end >= kSumLimit);
-        const int next = left != 0ull ? __builtin_ctzll(left) : kWave;  // the lane to sum in float
-        if (lane >= from && lane < next) {
-            uint32_t m = start;
+            for (int i = 0; i < kSumItems; ++i) any |= w[i] > 0.0f;
+            const uint64_t some = wave_ballot(any);
+            next = some != 0ull ? __builtin_ctzll(some) : kWave;
 #pragma unroll
-            for (int i = 0; i < kSumItems; ++i) {
-                const SumMap e = sum_map_of(w[i] * pre, scale);
-                m += (m & 1u) != 0u ? e.odd : e.even;
-                out[i] = sum_value(m, k);
+            for (int i = 0; i < kSumItems; ++i)
+                if (lane < next) out[i] = 0.0f;
+        } else {
+            const int k = sum_binade(total);
+            const float pre = sum_prescale(k), scale = sum_scale(k);
+            const uint32_t m0 = sum_mantissa(total, k);
+            SumMap map{0u, 0u};
+#pragma unroll
+            for (int i = 0; i < kSumItems; ++i) map = sum_then(map, sum_map_of(w[i] * pre, scale));
+            if (lane < from) map = SumMap{0u, 0u};
+            const SumMap incl = wave_sum_scan(map);
+            const uint32_t end = m0 + ((m0 & 1u) != 0u ? incl.odd : incl.even);
+            uint32_t start = (uint32_t)__shfl_up((int)end, 1, kWave);
+            if (lane == 0) start = m0;
+            const uint64_t left = wave_ballot(end >= kSumLimit);
+            next = left != 0ull ? __builtin_ctzll(left) : kWave;
+            if (lane >= from && lane < next) {
+                uint32_t m = start;
+#pragma unroll
+                for (int i = 0; i < kSumItems; ++i) {
+                    const SumMap e = sum_map_of(w[i] * pre, scale);
+                    m += (m & 1u) != 0u ? e.odd : e.even;
+                    out[i] = sum_value(m, k);
+                }
             }
+            const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)(next == kWave ? end : start), min(next, kWave - 1));
+            total = sum_value(m, k);
         }
-        const uint32_t m = (uint32_t)__builtin_amdgcn_readlane((int)(next == kWave ? end : start), min(next, kWave - 1));
-        total = sum_value(m, k);
         if (next == kWave) break;
 #pragma unroll
         for (int i = 0; i < kSumItems; ++i) {
