@@ -860,6 +860,11 @@ __device__ inline bool entry_meets_quadrant(const BlendEntry& e, uint32_t qx, ui
 // Gaussians close the tiles (1M in clusters). Only a scene between these would gain from a larger limit:
 // 6M at full HD have 6.1% of the entries and 92% of the tiles above 64 (589 us), 1.2 and 40% above 256 (546),
 // 0.1 and 7% above 1024 (495). There the gradient's error at such ratios is not measured.
+// A tile of fewer than kMomentPixels pixels (at an image's edge) forms every term per contribution all the same: moments
+// of a single pixel near an entry's mean leave little of themselves when moved there, and such pixels are then all that
+// a gradient comes from (images of 1x1, any scene: 0.5e-6 -> 7.3e-6 off 64 bits in the middle and 1.9e-3 at worst;
+// of 2x2 0.6 -> 0.8e-6, of 4x4 and of 49x50 no more than before). Beside whole tiles the few cost nothing.
+constexpr int kMomentPixels = 64;
 constexpr float kRegularRatio = 64.0f;
 constexpr float kRegularExtent = 1048576.0f;
 __device__ inline bool entry_is_regular(const BlendEntry& e) {
@@ -909,13 +914,14 @@ __global__ __launch_bounds__(kBlendThreads) void blend_forward_kernel(
     constexpr int kGroup = kTrain ? 2 : 4;
     __shared__ BlendEntry s_entry[kBlendThreads];
     __shared__ uint64_t s_exp2[GSX_EXPF_BLEND_TABLE_SIZE];
-    __shared__ uint32_t s_exact;  // TRAIN: an entry that a wave looked at is not regular
+    __shared__ uint32_t s_exact;  // TRAIN: few pixels, or an entry that a wave looked at is not regular
     const int tiles = cam.tiles_x * cam.tiles_y;
     const int tile = xcd_tile_index(blockIdx.x, tiles);
     if (tile >= tiles) return;
     if (threadIdx.x < GSX_EXPF_BLEND_TABLE_SIZE) s_exp2[threadIdx.x] = gsx_expf_blend_entry(threadIdx.x);
-    if (kTrain && threadIdx.x == 0) s_exact = 0u;
     const int tx = tile % cam.tiles_x, ty = tile / cam.tiles_x;
+    if (kTrain && threadIdx.x == 0)
+        s_exact = min(cam.width - tx * kTile, kTile) * min(cam.height - ty * kTile, kTile) < kMomentPixels ? 1u : 0u;
     const int2 tp = tile_pixel_of_thread((int)threadIdx.x);
     const int px = tx * kTile + tp.x;
     const int py = ty * kTile + tp.y;
@@ -1067,7 +1073,7 @@ constexpr int kGradRecord = 8;  // per-instance partials: channels 0-7 in one 32
 //    near-plane Gaussians reach ratios of 1e6 and more, where the CPU's gradient is mostly the
 //    rounding of its per-contribution map. A tile with an entry that is not regular forms every term per
 //    contribution with the CPU's operations, the suffix colour and its division included, and sums the
-//    nine values over the wave with lane swaps and DPP moves.
+//    nine values over the wave with lane swaps and DPP moves. So does a tile of few pixels (kMomentPixels).
 //
 // Reduction without atomics: every wave leaves one row of nine sums per entry in LDS, four threads
 // per entry combine the four waves' rows, and the tile writes one 9-float partial per reached
